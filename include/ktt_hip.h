@@ -100,7 +100,11 @@ int ktt_hip_event_elapsed_ms(void* start, void* end, float* milliseconds);
  * the last, partial round of workgroups over atom blocks; 0 does not). Grids of any side whose
  * G^2 rows fit an int: when there are more than 65,535 row groups (G above 1,023 with the
  * compensated defaults, above 1,448 with the plain ones) they fold into the launch's x dimension,
- * and the point index is 64-bit (the reference kernel's int index overflows above G = 1,290). */
+ * and the point index is 64-bit (the reference kernel's int index overflows above G = 1,290).
+ * Without a configuration, sides up to 1,024 that are not a multiple of 256 run the wave engine
+ * (CoulombPacked.hip), whose lanes pack any side and whose waves split the atoms of small grids;
+ * WAVE_SPLIT (1 to 16 waves sharing the atoms of 64 lanes), with POINTS_X (1 to 4, default 2) and
+ * ROWS_PER_THREAD (4 or 8, the default), selects it explicitly. */
 int ktt_coulomb3d(const float* atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
                   int form, const char* config, void* stream, float* kernel_ms);
 
@@ -108,8 +112,9 @@ int ktt_coulomb3d(const float* atoms, int n_atoms, float spacing, int grid_size,
  * (z = atom blocks; with the compensated form's tail split, the blocks the split tiles use), the
  * workgroup shape, the first split tile (tiles are numbered row group * x groups + x group, which
  * is y * grid[0] + x unless the row groups fold into x; equal to the tile
- * count when nothing is split) and the device scratch of the split in bytes. Compiles the kernel
- * (the split depends on its occupancy), so it needs the device. Each output optional. Replaces
+ * count when nothing is split) and the device scratch of the split in bytes. A wave-engine launch
+ * reports its workgroups in grid[0], 64 threads per wave in block[0], nothing split and no scratch.
+ * Compiles the kernel (the split depends on its occupancy), so it needs the device. Each output optional. Replaces
  * nothing in the reference: the occupancy-driven split has no counterpart there. */
 int ktt_coulomb3d_launch_plan(int n_atoms, int grid_size, int form, const char* config, unsigned int grid[3],
                               unsigned int block[3], int* split_from, size_t* scratch_bytes);

@@ -68,6 +68,10 @@ KERNEL_CHECKS = [
      "WORK_GROUP_SIZE_X=128,WORK_GROUP_SIZE_Y=4,POINTS_X=1,ROWS_PER_THREAD=8,ATOM_TILE=128,INNER_UNROLL_FACTOR=16"),
     ("CoulombSum3d.hip", "directCoulombSumCompensated",
      "WORK_GROUP_SIZE_X=128,WORK_GROUP_SIZE_Y=2,POINTS_X=2,ROWS_PER_THREAD=8,ATOM_TILE=256,INNER_UNROLL_FACTOR=16"),
+    ("CoulombPacked.hip", "coulombPacked", "POINTS_X=2,ROWS_PER_THREAD=8,ROW_GROUP_CAP=2"),
+    ("CoulombPacked.hip", "coulombPacked", "POINTS_X=2,ROWS_PER_THREAD=8,ROW_GROUP_CAP=2,COMPENSATED=1"),
+    ("CoulombPacked.hip", "coulombPacked", "POINTS_X=1,ROWS_PER_THREAD=4,ROW_GROUP_CAP=4,COMPENSATED=1"),
+    ("CoulombPacked.hip", "coulombPacked", "POINTS_X=1,ROWS_PER_THREAD=4,ROW_GROUP_CAP=1,ROW_MODE=1"),
     ("CoulombSum3dZ.hip", "directCoulombSum", None),
     ("CoulombSum3dZ.hip", "directCoulombSum", "Z_ITERATIONS=32,INNER_UNROLL_FACTOR=16,USE_SOA=1"),
     ("CoulombSum3dZ.hip", "directCoulombSum", "WORK_GROUP_SIZE_X=16,WORK_GROUP_SIZE_Y=4,Z_ITERATIONS=1,USE_CONSTANT_MEMORY=1"),

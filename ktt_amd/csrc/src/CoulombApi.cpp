@@ -14,6 +14,7 @@
 
 #include "../../../include/ktt_hip.h"
 #include "Common.h"
+#include "CoulombPacked.h"
 #include "CoulombRuntime.h"
 #include "HipEngine.h"
 #include "Kernel.h"
@@ -314,7 +315,7 @@ size_t CoulombRuntime::ResidentWorkgroups(const HipKernel& kernel, const int thr
 }
 
 void CoulombRuntime::Launch(const HipKernel& kernel, const unsigned int grid[3], const unsigned int block[3], void** arguments,
-    hipStream_t stream, float* kernelMs)
+    hipStream_t stream, float* kernelMs, const unsigned int ldsBytes)
 {
     if (grid[0] == 0 || grid[1] == 0 || grid[2] == 0)
     {
@@ -332,8 +333,8 @@ void CoulombRuntime::Launch(const HipKernel& kernel, const unsigned int grid[3],
         CheckHipError(hipEventCreate(&end), "hipEventCreate");
         CheckHipError(hipEventRecord(start, stream), "hipEventRecord");
     }
-    const hipError_t status = hipModuleLaunchKernel(kernel.GetFunction(), grid[0], grid[1], grid[2], block[0], block[1], block[2], 0,
-        stream, arguments, nullptr);
+    const hipError_t status = hipModuleLaunchKernel(kernel.GetFunction(), grid[0], grid[1], grid[2], block[0], block[1], block[2],
+        ldsBytes, stream, arguments, nullptr);
     if (status != hipSuccess)
     {
         if (start != nullptr)
@@ -415,7 +416,7 @@ static CoulombConfig DefaultsSlice(const int atomCount, const long gridX, const 
     return config;
 }
 
-static const std::vector<std::string> kLaunchOnly = {"ATOM_BLOCKS", "TAIL_SPLIT"};
+static const std::vector<std::string> kLaunchOnly = {"ATOM_BLOCKS", "TAIL_SPLIT", "WAVE_SPLIT"};
 
 // Most blocks a tail tile is split over (the tail round then holds at most this many times its tiles).
 constexpr long kMaxTailBlocks = 16;
@@ -837,7 +838,7 @@ struct Coulomb3dPlan
     size_t counterCount = 0;
 };
 
-static Coulomb3dPlan PlanCoulomb3d(const int atomCount, const int gridSize, const int form, const char* config)
+static void CheckForm(const int gridSize, const int form)
 {
     if (gridSize <= 0 || static_cast<long>(gridSize) * gridSize > 0x7fffffffL)
     {
@@ -847,6 +848,38 @@ static Coulomb3dPlan PlanCoulomb3d(const int atomCount, const int gridSize, cons
     {
         throw KttException("unknown form " + std::to_string(form));
     }
+}
+
+// Whether a ktt_coulomb3d call runs the wave engine (CoulombPacked.hip), and with what plan: when its
+// configuration says so (WAVE_SPLIT), or by default on grids that the workgroup shapes of
+// CoulombSum3d.hip do not fill. Those span 128 points of x (256 at multiples of 256) and need some
+// 160^3 points to fill the chip, so on 110 grids of 24^3 to 640^3 points the wave engine was faster at
+// all sides but the multiples of 256 (250^3 x 4,000: 5.36 against 5.86 ms plain, 5.56 against 6.42
+// compensated; 150^3 x 20,011: 5.9 against 11.2, 6.2 against 12.7; 33^3 x 500: 0.007 against 0.108,
+// 0.008 against 0.061). There the workgroup shapes fill every lane and share one set of row brackets
+// among 4 to 8 waves (256^3 x 8,192: 11.67 against 11.66 ms plain, 11.83 against 12.01 compensated). Above 1,024
+// the last span's idle lanes are under an eighth.
+static bool PackedPlanFor(const int atomCount, const int gridSize, const int form, const char* config, PackedPlan& plan)
+{
+    const CoulombConfig given = CoulombConfig::Parse(config, CoulombConfig());
+    const long rows = static_cast<long>(gridSize) * gridSize;
+    const bool compensated = form == KTT_COULOMB_COMPENSATED;
+    if (given.Has("WAVE_SPLIT"))
+    {
+        plan = PackedPlanOf(given, atomCount, gridSize, rows, compensated);
+        return true;
+    }
+    if (!given.values.empty() || gridSize % 256 == 0 || gridSize > 1024)
+    {
+        return false;
+    }
+    plan = ChoosePackedPlan(atomCount, gridSize, rows, compensated);
+    return true;
+}
+
+static Coulomb3dPlan PlanCoulomb3d(const int atomCount, const int gridSize, const int form, const char* config)
+{
+    CheckForm(gridSize, form);
     Coulomb3dPlan plan;
     plan.config = CoulombConfig::Parse(config, Defaults3d(form, gridSize));
     if (!CoulombConfig::Parse(config, CoulombConfig()).Has("ATOM_TILE"))
@@ -908,13 +941,17 @@ int ktt_coulomb3d(const float* atoms, int atomCount, float spacing, int gridSize
     }
     CheckAtoms(atoms, atomCount);
     CheckGrid(energyGrid, static_cast<long>(gridSize) * gridSize * gridSize);
-    if (form != KTT_COULOMB_PLAIN && form != KTT_COULOMB_COMPENSATED)
+    CheckForm(gridSize, form);
+    hipStream_t hipStream = static_cast<hipStream_t>(stream);
+    PackedPlan packed;
+    if (PackedPlanFor(atomCount, gridSize, form, config, packed))
     {
-        return SetLastError("unknown form " + std::to_string(form));
+        LaunchPacked(packed, atoms, atomCount, spacing, gridSize, gridSize * gridSize, energyGrid, form == KTT_COULOMB_COMPENSATED, false,
+            hipStream, kernelMs);
+        return 0;
     }
     Coulomb3dPlan plan = PlanCoulomb3d(atomCount, gridSize, form, config);
     const float* unused = nullptr;
-    hipStream_t hipStream = static_cast<hipStream_t>(stream);
     if (form == KTT_COULOMB_PLAIN)
     {
         void* arguments[] = {&atoms, &unused, &unused, &unused, &unused, &atomCount, &spacing, &gridSize, &energyGrid};
@@ -939,7 +976,22 @@ int ktt_coulomb3d_launch_plan(int atomCount, int gridSize, int form, const char*
     {
         return SetLastError("Number of atoms must not be negative");
     }
-    const Coulomb3dPlan plan = PlanCoulomb3d(atomCount, gridSize, form, config);
+    Coulomb3dPlan plan;
+    PackedPlan packed;
+    CheckForm(gridSize, form);
+    if (PackedPlanFor(atomCount, gridSize, form, config, packed))
+    {
+        CoulombRuntime::Get().EnsureDevice();
+        plan.grid[0] = plan.shape.grid[0] = packed.workgroups;
+        plan.grid[1] = plan.grid[2] = 1;
+        plan.shape.block[0] = static_cast<unsigned int>(packed.waves) * 64;
+        plan.shape.block[1] = plan.shape.block[2] = 1;
+        plan.splitFrom = static_cast<int>(packed.workgroups);
+    }
+    else
+    {
+        plan = PlanCoulomb3d(atomCount, gridSize, form, config);
+    }
     for (int i = 0; i < 3; ++i)
     {
         if (grid != nullptr)

@@ -1,0 +1,167 @@
+#include "CoulombPacked.h"
+
+#include <algorithm>
+#include <cmath>
+#include <limits>
+
+#include <KttException.h>
+
+namespace ktt
+{
+
+namespace
+{
+
+// LDS of a workgroup on gfx950.
+constexpr long kLdsBytes = 160 * 1024;
+
+// Row groups a wave of 64 lanes touches at most (kc::rowGroupsPerWave), of those there are.
+int RowGroupsPerWave(const int lanesX, const int rowGroups)
+{
+    return std::min(rowGroups, lanesX % 64 == 0 ? 1 : (64 % lanesX == 0 ? 64 / lanesX : (64 - 2) / lanesX + 2));
+}
+
+// The plan of a shape, or one with no workgroups when the shape does not fit the LDS or a launch.
+PackedPlan PlanShape(const int px, const int rows, const int waves, const int atomCount, const long rowLength, const long rowsTotal,
+    const bool compensated)
+{
+    PackedPlan plan;
+    plan.px = px;
+    plan.rows = rows;
+    plan.waves = waves;
+    const long lanesX = (rowLength + px - 1) / px;
+    const long rowGroups = (rowsTotal + rows - 1) / rows;
+    const long workgroups = (lanesX * rowGroups + 63) / 64;
+    plan.lanesX = static_cast<int>(lanesX);
+    plan.rowGroups = static_cast<int>(rowGroups);
+    plan.touched = RowGroupsPerWave(plan.lanesX, plan.rowGroups);
+    plan.cap = 1;
+    while (plan.cap < plan.touched)
+    {
+        plan.cap *= 2;
+    }
+    // Whole unrolled steps of 8 atoms per wave.
+    const long perWave = (static_cast<long>(atomCount) + waves - 1) / waves;
+    plan.share = static_cast<int>(std::min<long>((perWave + 7) / 8 * 8, std::numeric_limits<int>::max()));
+    const long ldsBytes = waves * 64L * ((compensated ? 4 : 2) + static_cast<long>(plan.cap) * rows + 4) * 4;
+    // Lane numbers are 32-bit, and a launch holds fewer than 2^32 threads.
+    if (ldsBytes <= kLdsBytes && workgroups * 64 * waves <= 0x7fffffffL)
+    {
+        plan.ldsBytes = static_cast<unsigned int>(ldsBytes);
+        plan.workgroups = static_cast<unsigned int>(workgroups);
+    }
+    return plan;
+}
+
+// The shapes tried, with what the estimate below needs of each.
+struct Shape
+{
+    int px;
+    int rows;
+    double atom;      // us a SIMD takes per wave and atom with enough waves to hide latency
+    double alone;     // share of that rate that one wave per SIMD reaches
+    int wavesPerSimd; // at the kernel's registers, plain and compensated
+    int wavesPerSimdCompensated;
+};
+const Shape kShapes[] = {{2, 8, 0.0932, 0.34, 8, 5}, {1, 8, 0.0505, 0.33, 7, 7}, {1, 4, 0.0268, 0.32, 8, 8}};
+
+// Estimated time of a plan in us. The constants are a fit to 110 grids of 24^3 to 640^3 points with 64 to
+// 30,000 atoms on MI355X, each timed at every shape and 1, 4, 8 and 16 waves; the shape it picks is
+// within 1.2% of the fastest on average (at worst 18%).
+double Estimate(const PackedPlan& plan, const Shape& shape, const bool compensated)
+{
+    const double size = plan.px * plan.rows / 16.0;
+    const double tiles = (plan.share + 63) / 64;
+    // One wave: its atoms, the brackets of its rows per 64 atoms, the start and the store, and, if
+    // the waves of a workgroup split the atoms, their meeting in LDS.
+    double wave = plan.share * shape.atom * (compensated ? 1.12 : 1.0);
+    wave += tiles * plan.touched * plan.rows * (compensated ? 0.010 : 0.0048);
+    wave += 0.13 + size * (compensated ? 0.48 : 0.35);
+    wave += plan.waves > 1 ? size * (compensated ? 0.42 : 0.26) : 0.0;
+    // Waves per SIMD of the 256 CUs: whole workgroups per CU while they all fit at once; more than
+    // that are handed out as others end, with a partial last round.
+    constexpr double kComputeUnits = 256.0;
+    const int slots = compensated ? shape.wavesPerSimdCompensated : shape.wavesPerSimd;
+    const double perGroup = plan.waves / 4.0;
+    const double resident = plan.waves < 4 ? slots : std::max(1, slots * 4 / plan.waves) * perGroup;
+    double load = plan.waves < 4 ? std::ceil(plan.workgroups * perGroup / kComputeUnits)
+                                 : std::ceil(plan.workgroups / kComputeUnits) * perGroup;
+    double busy = load;
+    if (load > resident)
+    {
+        busy = resident;
+        load = plan.workgroups * perGroup / kComputeUnits + 0.67 * std::max(1.0, perGroup);
+    }
+    const double rate = 1.0 - (1.0 - shape.alone) * std::pow(busy, -0.93);
+    return load * wave / rate;
+}
+
+} // namespace
+
+PackedPlan MakePackedPlan(const int px, const int rows, const int waves, const int atomCount, const long rowLength,
+    const long rowsTotal, const bool compensated)
+{
+    if (px < 1 || px > 4 || (rows != 4 && rows != 8) || waves < 1 || waves > 16)
+    {
+        throw KttException("the wave engine takes WAVE_SPLIT 1 to 16, POINTS_X 1 to 4 and ROWS_PER_THREAD 4 or 8");
+    }
+    const PackedPlan plan = PlanShape(px, rows, waves, atomCount, rowLength, rowsTotal, compensated);
+    if (plan.workgroups == 0)
+    {
+        throw KttException("WAVE_SPLIT=" + std::to_string(waves) + " with " + std::to_string(px) + " x " + std::to_string(rows)
+            + " points per thread exceeds the device limits on rows of " + std::to_string(rowLength) + " points",
+            ExceptionReason::DeviceLimitsExceeded);
+    }
+    return plan;
+}
+
+PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, const long rowsTotal, const bool compensated)
+{
+    PackedPlan best;
+    double bestTime = std::numeric_limits<double>::max();
+    for (const Shape& shape : kShapes)
+    {
+        for (const int waves : {1, 4, 8, 16})
+        {
+            const PackedPlan plan = PlanShape(shape.px, shape.rows, waves, atomCount, rowLength, rowsTotal, compensated);
+            // A short row wraps a wave over many row groups, whose brackets then cost more LDS and
+            // instructions than a narrower block saves.
+            if (plan.workgroups == 0 || (shape.px > 1 && plan.touched > 4))
+            {
+                continue;
+            }
+            const double time = Estimate(plan, shape, compensated);
+            if (time < bestTime)
+            {
+                bestTime = time;
+                best = plan;
+            }
+        }
+    }
+    return best;
+}
+
+PackedPlan PackedPlanOf(const CoulombConfig& config, const int atomCount, const long rowLength, const long rowsTotal,
+    const bool compensated)
+{
+    return MakePackedPlan(static_cast<int>(config.Get("POINTS_X", 2)), static_cast<int>(config.Get("ROWS_PER_THREAD", 8)),
+        static_cast<int>(config.Get("WAVE_SPLIT", 1)), atomCount, rowLength, rowsTotal, compensated);
+}
+
+void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, float spacing, int rowLength, int rowsTotal,
+    float* energyGrid, const bool compensated, const bool slice, hipStream_t stream, float* kernelMs)
+{
+    const std::vector<std::string> defines = {"-DPOINTS_X=" + std::to_string(plan.px), "-DROWS_PER_THREAD=" + std::to_string(plan.rows),
+        "-DROW_GROUP_CAP=" + std::to_string(plan.cap), std::string("-DCOMPENSATED=") + (compensated ? "1" : "0"),
+        std::string("-DROW_MODE=") + (slice ? "1" : "0")};
+    const auto kernel = CoulombRuntime::Get().GetKernel("CoulombPacked.hip", "coulombPacked", defines);
+    const unsigned int grid[3] = {plan.workgroups, 1, 1};
+    const unsigned int block[3] = {static_cast<unsigned int>(plan.waves) * 64, 1, 1};
+    int share = plan.share;
+    int lanesX = plan.lanesX;
+    int rowGroups = plan.rowGroups;
+    void* arguments[] = {&atoms, &atomCount, &share, &spacing, &lanesX, &rowGroups, &rowLength, &rowsTotal, &energyGrid};
+    CoulombRuntime::Launch(*kernel, grid, block, arguments, stream, kernelMs, plan.ldsBytes);
+}
+
+} // namespace ktt

@@ -63,7 +63,7 @@ public:
      *  compute units x workgroups per compute unit at the kernel's occupancy. */
     static size_t ResidentWorkgroups(const HipKernel& kernel, const int threads);
     static void Launch(const HipKernel& kernel, const unsigned int grid[3], const unsigned int block[3], void** arguments,
-        hipStream_t stream, float* kernelMs);
+        hipStream_t stream, float* kernelMs, const unsigned int ldsBytes = 0);
 
 private:
     CoulombRuntime();

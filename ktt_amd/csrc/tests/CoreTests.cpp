@@ -28,6 +28,7 @@
 #include "TunerCore.h"
 #include "Exploration.h"
 #include "CoulombBatchPlan.h"
+#include "CoulombPacked.h"
 
 using namespace ktt;
 
@@ -589,6 +590,65 @@ void TestBatchWorkList()
     CHECK(ragged);
 }
 
+/** The wave engine's launch plans over every grid side the default takes them for at small sizes, and
+ *  ragged slices: the plan exists and fits the LDS, the waves' atom shares cover the atoms once in whole
+ *  unrolled steps, every lane's points lie in one row group, and no wave touches more row groups than
+ *  its LDS holds brackets for (the lane numbering of kernels/coulomb_wave.h restated). */
+void TestPackedPlan()
+{
+    bool fits = true;
+    bool covers = true;
+    bool bounded = true;
+    for (int g = 1; g <= 160; ++g)
+    {
+        for (const long rows : {static_cast<long>(g) * g, static_cast<long>(g)})
+        {
+            for (const int atoms : {0, 1, 8, 9, 63, 65, 200, 1001, 65536})
+            {
+                for (const bool compensated : {false, true})
+                {
+                    const ktt::PackedPlan plan = ktt::ChoosePackedPlan(atoms, g, rows, compensated);
+                    fits = fits && plan.workgroups > 0 && plan.waves >= 1 && plan.waves <= 16 && plan.ldsBytes > 0
+                        && plan.ldsBytes <= 160u * 1024u;
+                    covers = covers && plan.share % 8 == 0 && static_cast<long>(plan.share) * plan.waves >= atoms
+                        && static_cast<long>(plan.workgroups) * 64 >= static_cast<long>(plan.lanesX) * plan.rowGroups
+                        && plan.lanesX * plan.px >= g && (plan.lanesX - 1) * plan.px < g
+                        && static_cast<long>(plan.rowGroups) * plan.rows >= rows
+                        && static_cast<long>(plan.rowGroups - 1) * plan.rows < rows;
+                    const long lanes = static_cast<long>(plan.lanesX) * plan.rowGroups;
+                    for (long first = 0; first < lanes; first += 64)
+                    {
+                        const long last = std::min(first + 63, lanes - 1);
+                        const long groups = last / plan.lanesX - first / plan.lanesX + 1;
+                        bounded = bounded && groups <= plan.touched && groups <= plan.cap;
+                    }
+                }
+            }
+        }
+    }
+    CHECK(fits);
+    CHECK(covers);
+    CHECK(bounded);
+    const auto refused = [](const int px, const int rows, const int waves, const long side)
+    {
+        try
+        {
+            ktt::MakePackedPlan(px, rows, waves, 100, side, side * side, true);
+        }
+        catch (const ktt::KttException&)
+        {
+            return true;
+        }
+        return false;
+    };
+    CHECK(!refused(2, 8, 16, 128));
+    CHECK(refused(0, 8, 1, 64));
+    CHECK(refused(2, 6, 1, 64));
+    CHECK(refused(2, 8, 17, 64));
+    CHECK(refused(2, 8, 16, 24));     // 8 row groups of 8 rows per wave: 16 waves' brackets exceed the LDS
+    CHECK(refused(1, 4, 16, 46340));  // more threads than a launch holds
+}
+
 int main(int argc, char** argv)
 {
     if (argc != 2)
@@ -608,6 +668,7 @@ int main(int argc, char** argv)
     TestJsonRoundTrip(results);
     TestProfileSearcherAnalysis();
     TestBatchWorkList();
+    TestPackedPlan();
     std::printf("%d checks, %d failures\n", g_Checks, g_Failures);
     return g_Failures == 0 ? 0 : 1;
 }

@@ -1,0 +1,413 @@
+// Wave engine of the direct Coulomb sum for gfx950: one wave owns a packed run of points and works
+// alone, without workgroup barriers, so that any grid side fills its lanes and the atoms of one run
+// can be split over the waves of a workgroup.
+//
+// Points. A row is the set of x points that share one (y, z) (coulomb_core.h). Rows are taken ROWS at
+// a time (a row group) and a row's points PX at a time, which makes lanesX = ceil(rowLength / PX)
+// lanes per row group. Lanes are numbered row group * lanesX + x lane over the whole grid, and wave b
+// takes lanes [64 b, 64 b + 64): they wrap from one row group into the next, so that only the grid's
+// last wave and a row length that PX does not divide leave lanes idle. (A workgroup of coulomb_core.h
+// spans a fixed number of x points instead: at a side of 150 its 128-point spans leave 41% of the
+// lanes idle, at 64 half of them.) A wave touches at most CAP row groups; the host derives CAP from
+// lanesX (kc::rowGroupsPerWave).
+//
+// Atoms are staged by the wave 64 at a time, one per lane, into LDS that only this wave uses: the
+// atom's x and charge, and the brackets B = (y - Y)^2 + (z - Z)^2 of every row of the wave's groups.
+// A wave's LDS operations complete in order, so the tile needs no barrier. B costs 3 to 4 instructions
+// per (row, atom), formed row after row with the row's y and z in scalars; the atom of the next tile
+// is read from memory while this one is summed. The inner loop is the issue-phased loop of
+// coulomb_core.h, and the last atom's r^-1 stays in flight over the tile's end.
+//
+// Split. The WAVE_SPLIT waves of a workgroup own the same 64 lanes and a contiguous share of the atoms
+// each. They meet in LDS once, in wave order (plain FP32; compensated FP64), so results do not depend on
+// timing. A grid with few points fills the chip this way: 64^3 points are 256 waves of 2 x 8 points, a
+// quarter of the 1,024 SIMDs, and 256 workgroups of 16 waves when the atoms are split.
+//
+// Bound by FP32 VALU issue as the workgroup engine is (per interaction 2 FMAs that pair with another
+// wave's and a v_rsq_f32 of two quad-cycles); small grids by the launch. Measured on MI355X with the
+// fill before it, workgroup shapes -> wave engine: 150^3 x 20,011 compensated 12,990 -> 6,213 us (119
+// TFLOP/s at 11 per interaction), 99^3 x 3,001 plain 636 -> 296, 64^3 x 5,000 compensated 363 -> 140,
+// 32^3 x 200 plain 59 -> 8.6. On 256^3 x 8,192, which the workgroup shapes fill, 11,670 -> 11,660 us
+// plain and 11,830 -> 12,010 compensated: every wave forms its own row brackets, and the compensated
+// dx takes one FMA more per atom.
+#pragma once
+
+#include "coulomb_core.h"
+
+namespace kc
+{
+
+template <bool CONDITION, class A, class B>
+struct Select
+{
+    using Type = A;
+};
+template <class A, class B>
+struct Select<false, A, B>
+{
+    using Type = B;
+};
+
+// Largest number of row groups that 64 consecutive lanes touch when a row group has lanesX lanes.
+constexpr int rowGroupsPerWave(const int lanesX)
+{
+    return lanesX % 64 == 0 ? 1 : (64 % lanesX == 0 ? 64 / lanesX : (64 - 2) / lanesX + 2);
+}
+
+// Orders this wave's LDS accesses for the compiler; the hardware keeps them in order.
+__device__ __forceinline__ void waveFence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int PX, int ROWS, int CAP, int MODE, bool COMP>
+struct WaveEngine
+{
+    static constexpr int Tile = 64;
+    static constexpr int Unroll = 8;
+    static constexpr int FoldTiles = 4;  // tiles per two-sum of the compensated form: 256 atoms
+    static constexpr int Points = PX * ROWS;
+    static constexpr int AtomFloats = COMP ? 4 : 2;
+    // Row brackets of one atom, padded so that the 16-byte stores of 8 lanes hit all 64 banks once.
+    static constexpr int RowStride = CAP * ROWS + 4;
+    static constexpr int WaveFloats = Tile * (AtomFloats + RowStride);
+    // Values per lane that fit a wave's LDS when the waves of a split meet.
+    using Sum = typename Select<COMP, double, float>::Type;
+    static constexpr int MeetWhole = WaveFloats * 4 / (64 * static_cast<int>(sizeof(Sum)));
+    static constexpr int MeetValues = MeetWhole < Points ? MeetWhole : Points;
+
+    static_assert(ROWS % 4 == 0, "row brackets are stored four at a time");
+
+    // Position of this lane's points: x0 = xLane * PX, rows row0 .. row0 + ROWS - 1.
+    int lane;
+    int xLane;
+    int rowGroup;
+    int firstGroup;  // the wave's first row group and the number it touches (uniform)
+    int groups;
+    bool valid;
+
+    float part[ROWS][PX];
+    float sum[ROWS][PX];
+    float comp[ROWS][PX];
+
+    __device__ __forceinline__ void place(const unsigned int waveBlock, const int lanesX, const int rowGroups)
+    {
+        lane = threadIdx.x & 63;
+        const unsigned int total = static_cast<unsigned int>(lanesX) * static_cast<unsigned int>(rowGroups);
+        const unsigned int first = waveBlock * 64u;
+        const unsigned int mine = first + lane;
+        valid = mine < total;
+        const unsigned int index = valid ? mine : total - 1u;
+        rowGroup = static_cast<int>(index / static_cast<unsigned int>(lanesX));
+        xLane = static_cast<int>(index - static_cast<unsigned int>(rowGroup) * lanesX);
+        firstGroup = __builtin_amdgcn_readfirstlane(rowGroup);
+        groups = __builtin_amdgcn_readlane(rowGroup, 63) - firstGroup + 1;
+#pragma unroll
+        for (int k = 0; k < ROWS; ++k)
+        {
+#pragma unroll
+            for (int i = 0; i < PX; ++i)
+            {
+                part[k][i] = 0.0f;
+                sum[k][i] = 0.0f;
+                comp[k][i] = 0.0f;
+            }
+        }
+    }
+
+    static __device__ __forceinline__ float4 loadAtom(const float4* atoms, const unsigned int index, const unsigned int end)
+    {
+        return index < end ? atoms[index] : make_float4(kPadCoord, kPadCoord, kPadCoord, 0.0f);
+    }
+
+    // One atom per lane into the wave's LDS, with the brackets of the wave's rows.
+    // Compensated x: X = h n + d with n a near grid index and d formed in FP64, so that
+    // x - X = h (i - n) - d carries one rounding whatever the coordinate's size. n is clamped to
+    // 2^23, where i - n is still exact in FP32; beyond it (or with h = 0) d holds the rest.
+    __device__ __forceinline__ void stage(float* lds, const float4 at, const float h, const int rowsPerPlane) const
+    {
+        float* sB = lds + Tile * AtomFloats + lane * RowStride;
+        if constexpr (COMP)
+        {
+            const double X = static_cast<double>(at.x);
+            const double n = __builtin_rint(__builtin_fmin(__builtin_fmax(X * (1.0 / static_cast<double>(h)), -8388608.0), 8388608.0));
+            const double d = X - static_cast<double>(h) * n;
+            *reinterpret_cast<float4*>(lds + lane * 4) = make_float4(static_cast<float>(n), static_cast<float>(-d), at.w, 0.0f);
+        }
+        else
+        {
+            *reinterpret_cast<float2*>(lds + lane * 2) = make_float2(at.x, at.w);
+        }
+        using Real = typename Select<COMP, double, float>::Type;
+        const Real Y = static_cast<Real>(at.y);
+        const Real Z = static_cast<Real>(at.z);
+        const Real step = static_cast<Real>(h);
+        int row = firstGroup * ROWS;
+        int y = (MODE == Volume) ? row % rowsPerPlane : row;
+        int z = (MODE == Volume) ? row / rowsPerPlane : 0;
+        Real dz2 = Z;
+        if constexpr (MODE == Volume)
+        {
+            const Real dz = step * static_cast<Real>(z) - Z;
+            dz2 = dz * dz;
+        }
+        Real dy = step * static_cast<Real>(y) - Y;
+        const int quads = groups * (ROWS / 4);
+#pragma unroll 1
+        for (int g = 0; g < quads; ++g)
+        {
+            float b[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+            {
+                b[k] = static_cast<float>(dy * dy + dz2);
+                ++y;
+                if constexpr (COMP)
+                {
+                    dy += step;  // FP64: a step's rounding is far below B's own to FP32
+                }
+                if (MODE == Volume && y == rowsPerPlane)
+                {
+                    y = 0;
+                    ++z;
+                    const Real dz = step * static_cast<Real>(z) - Z;
+                    dz2 = dz * dz;
+                    dy = -Y;
+                }
+                if constexpr (!COMP)
+                {
+                    dy = step * static_cast<Real>(y) - Y;
+                }
+            }
+            *reinterpret_cast<float4*>(sB + g * 4) = make_float4(b[0], b[1], b[2], b[3]);
+        }
+    }
+
+    // Adds atoms [a0, a1) into this lane's points.
+    __device__ __forceinline__ void accumulate(float* lds, const float4* atoms, const unsigned int a0, const unsigned int a1, const float h,
+        const int rowsPerPlane)
+    {
+        const float* sB = lds + Tile * AtomFloats + (rowGroup - firstGroup) * ROWS;
+        float x[PX];
+#pragma unroll
+        for (int i = 0; i < PX; ++i)
+        {
+            x[i] = COMP ? static_cast<float>(xLane * PX + i) : h * static_cast<float>(xLane * PX + i);
+        }
+        float hV = h;  // in a VGPR: an SGPR operand would keep the FMA from pairing
+        asm volatile("" : "+v"(hV));
+        float rr[ROWS][PX];  // r^2 of the atom in flight, then its r^-1
+#pragma unroll
+        for (int k = 0; k < ROWS; ++k)
+        {
+#pragma unroll
+            for (int i = 0; i < PX; ++i)
+            {
+                rr[k][i] = 0.0f;
+            }
+        }
+        float qPrev = 0.0f;
+        int tiles = 0;
+        float4 next;
+        if constexpr (!COMP)
+        {
+            next = loadAtom(atoms, a0 + lane, a1);
+        }
+        for (unsigned int t = a0; t < a1; t += Tile)
+        {
+            waveFence();  // the previous tile has been read
+            if constexpr (COMP)
+            {
+                // Not read ahead: four registers more would cost a wave per SIMD.
+                next = loadAtom(atoms, t + lane, a1);
+            }
+            stage(lds, next, h, rowsPerPlane);
+            if constexpr (!COMP)
+            {
+                next = loadAtom(atoms, t + Tile + lane, a1);
+            }
+            waveFence();
+            const int count = a1 - t < Tile ? static_cast<int>(a1 - t) : Tile;
+            for (int a = 0; a < count; a += Unroll)
+            {
+#pragma unroll
+                for (int u = 0; u < Unroll; ++u)
+                {
+                    __builtin_amdgcn_sched_barrier(0);
+                    __builtin_amdgcn_s_setprio(0);
+                    float dx[PX];
+                    float q;
+                    if constexpr (COMP)
+                    {
+                        const float4 v = *reinterpret_cast<const float4*>(lds + (a + u) * 4);
+                        dx[0] = fmaf(hV, x[0] - v.x, v.y);
+#pragma unroll
+                        for (int i = 1; i < PX; ++i)
+                        {
+                            dx[i] = dx[i - 1] + hV;
+                        }
+                        q = v.z;
+                    }
+                    else
+                    {
+                        const float2 v = *reinterpret_cast<const float2*>(lds + (a + u) * 2);
+#pragma unroll
+                        for (int i = 0; i < PX; ++i)
+                        {
+                            dx[i] = x[i] - v.x;
+                        }
+                        q = v.y;
+                    }
+                    float b[ROWS];
+#pragma unroll
+                    for (int k = 0; k < ROWS; k += 4)
+                    {
+                        const float4 v = *reinterpret_cast<const float4*>(sB + (a + u) * RowStride + k);
+                        b[k] = v.x;
+                        b[k + 1] = v.y;
+                        b[k + 2] = v.z;
+                        b[k + 3] = v.w;
+                    }
+#pragma unroll
+                    for (int k = 0; k < ROWS; ++k)
+                    {
+#pragma unroll
+                        for (int i = 0; i < PX; ++i)
+                        {
+                            part[k][i] = fmaf(qPrev, rr[k][i], part[k][i]);
+                            rr[k][i] = fmaf(dx[i], dx[i], b[k]);
+                        }
+                    }
+                    qPrev = q;
+                    __builtin_amdgcn_sched_barrier(0);
+                    __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+                    for (int k = 0; k < ROWS; ++k)
+                    {
+#pragma unroll
+                        for (int i = 0; i < PX; ++i)
+                        {
+                            rr[k][i] = __builtin_amdgcn_rsqf(rr[k][i]);
+                        }
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(0);
+            if constexpr (COMP)
+            {
+                // Land the atom in flight: its 16 registers are free while the next tile is staged,
+                // which keeps the kernel at 5 waves per SIMD.
+                land(qPrev, rr);
+                qPrev = 0.0f;
+                if (++tiles == FoldTiles)
+                {
+                    tiles = 0;
+                    fold();
+                }
+            }
+        }
+        if constexpr (COMP)
+        {
+            fold();
+        }
+        else
+        {
+            land(qPrev, rr);
+        }
+    }
+
+    // part += q r^-1 of the atom in flight.
+    __device__ __forceinline__ void land(const float q, float (&rr)[ROWS][PX])
+    {
+#pragma unroll
+        for (int k = 0; k < ROWS; ++k)
+        {
+#pragma unroll
+            for (int i = 0; i < PX; ++i)
+            {
+                part[k][i] = fmaf(q, rr[k][i], part[k][i]);
+                rr[k][i] = 0.0f;
+            }
+        }
+    }
+
+    __device__ __forceinline__ void fold()
+    {
+#pragma unroll
+        for (int k = 0; k < ROWS; ++k)
+        {
+#pragma unroll
+            for (int i = 0; i < PX; ++i)
+            {
+                twoSumInto(sum[k][i], comp[k][i], part[k][i]);
+                part[k][i] = 0.0f;
+            }
+            __builtin_amdgcn_sched_barrier(0);  // one row at a time: few registers
+        }
+    }
+
+    // This wave's sum at point v = row * PX + x of the lane (v a constant after unrolling).
+    __device__ __forceinline__ Sum value(const int v) const
+    {
+        if constexpr (COMP)
+        {
+            return addPair(-0.0, sum[v / PX][v % PX], comp[v / PX][v % PX]);
+        }
+        else
+        {
+            return part[v / PX][v % PX];
+        }
+    }
+
+    __device__ __forceinline__ void add(float* grid, const int v, const int rowLength, const int rowsTotal, const Sum total) const
+    {
+        const int x = xLane * PX + v % PX;
+        const int row = rowGroup * ROWS + v / PX;
+        if (valid && x < rowLength && row < rowsTotal)
+        {
+            float* out = grid + static_cast<size_t>(row) * rowLength + x;
+            *out = static_cast<float>(static_cast<Sum>(*out) + total);
+        }
+    }
+
+    // grid += the sum over the workgroup's waves, each of which holds the same points' sums over its
+    // own atoms. shared: waves * WaveFloats floats.
+    __device__ __forceinline__ void store(float* shared, const int waves, const int wave, float* grid, const int rowLength,
+        const int rowsTotal) const
+    {
+        if (waves == 1)
+        {
+#pragma unroll
+            for (int v = 0; v < Points; ++v)
+            {
+                add(grid, v, rowLength, rowsTotal, value(v));
+            }
+            return;
+        }
+        Sum* meet = reinterpret_cast<Sum*>(shared);
+#pragma unroll
+        for (int first = 0; first < Points; first += MeetValues)
+        {
+            __syncthreads();
+#pragma unroll
+            for (int v = first; v < first + MeetValues && v < Points; ++v)
+            {
+                meet[(wave * MeetValues + v - first) * 64 + lane] = value(v);
+            }
+            __syncthreads();
+            for (int v = first + wave; v < first + MeetValues && v < Points; v += waves)
+            {
+                Sum total = meet[(v - first) * 64 + lane];
+                for (int w = 1; w < waves; ++w)
+                {
+                    total += meet[(w * MeetValues + v - first) * 64 + lane];
+                }
+                add(grid, v, rowLength, rowsTotal, total);
+            }
+        }
+    }
+};
+
+} // namespace kc

@@ -1,0 +1,83 @@
+"""The wave engine (ktt_amd/kernels/coulomb_wave.h) against the FP64 oracle at every point, where it
+can go wrong: sides whose rows wrap within a wave, end inside one or are shorter than a lane's run; atom
+counts around a wave's 64-atom tile, the 256 atoms of a two-sum and the unrolled step; one wave, waves
+without atoms, and splits that meet in several passes over the LDS.
+
+Bars as for every form: 1e-5 plain, 1e-6 compensated, normalised by sum_i |q_i| / r_i."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from ktt_amd import workloads
+from oracle import coulomb_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+
+BARS = {0: 1e-5, 1: 1e-6}
+
+
+def run_guarded(capi, atoms, spacing, grid, form, config):
+    """The map added onto zeros, with a guard behind it that must stay as it was."""
+    atoms_buffer = capi.DeviceBuffer.from_array(atoms)
+    start = np.zeros(grid ** 3 + 256, dtype=np.float32)
+    start[grid ** 3:] = 7.0
+    energy = capi.DeviceBuffer.from_array(start)
+    capi.coulomb3d(atoms_buffer, atoms.shape[0], spacing, grid, energy, form=form, config=config)
+    out = energy.download((grid ** 3 + 256,))
+    assert (out[grid ** 3:] == 7.0).all()
+    return out[:grid ** 3]
+
+
+def check(capi, grid, count, form, config, spacing=0.5):
+    atoms = workloads.uniform_atoms(1000 * grid + count, count, box=max(grid, 4) * spacing)
+    z, y, x = np.meshgrid(*(np.arange(grid),) * 3, indexing="ij")
+    points = np.stack([x.ravel(), y.ravel(), z.ravel()], axis=1).astype(np.int32)
+    print(f"grid {grid} atoms {count} form {form} config {config}", flush=True)
+    values, norms = oracle.points_f64(atoms, spacing, points)
+    worst, rms = oracle.normalised_error(run_guarded(capi, atoms, spacing, grid, form, config), values, norms)
+    assert worst <= BARS[form], (worst, rms)
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("grid", [1, 2, 3, 7, 16, 31, 33, 48, 65, 70])
+def test_default_shapes(capi, grid, form):
+    for count in (1, 64, 203):
+        check(capi, grid, count, form, None)
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("shape", ["POINTS_X=2,ROWS_PER_THREAD=8", "POINTS_X=1,ROWS_PER_THREAD=8", "POINTS_X=1,ROWS_PER_THREAD=4",
+                                   "POINTS_X=3,ROWS_PER_THREAD=4"])
+@pytest.mark.parametrize("waves,count", [(1, 7), (1, 65), (3, 257), (4, 521), (16, 9), (16, 1025)])
+def test_splits(capi, shape, waves, count, form):
+    check(capi, 45, count, form, f"WAVE_SPLIT={waves},{shape}")
+
+
+@pytest.mark.parametrize("form", [0, 1])
+def test_odd_spacings_and_far_atoms(capi, form):
+    """A spacing that FP32 rounds, and atoms outside the box on both sides, some so far that their grid
+    index passes 2^23 (where the compensated x offset is clamped)."""
+    grid, spacing = 27, 0.49
+    atoms = workloads.uniform_atoms(77, 90, box=20.0)
+    atoms[:30, :3] -= 15.0
+    atoms[30:33, 0] += np.float32(6.0e6)
+    atoms[33:36, 0] -= np.float32(6.0e6)
+    z, y, x = np.meshgrid(*(np.arange(grid),) * 3, indexing="ij")
+    points = np.stack([x.ravel(), y.ravel(), z.ravel()], axis=1).astype(np.int32)
+    values, norms = oracle.points_f64(atoms, spacing, points)
+    for config in (None, "WAVE_SPLIT=4,POINTS_X=2,ROWS_PER_THREAD=8"):
+        result = run_guarded(capi, atoms, spacing, grid, form, config)
+        assert oracle.normalised_error(result, values, norms)[0] <= BARS[form]
+
+
+def test_repeats_are_bitwise_equal_and_bad_shapes_are_refused(capi):
+    atoms = workloads.uniform_atoms(78, 700, box=20.0)
+    for form in (0, 1):
+        first = run_guarded(capi, atoms, 0.5, 40, form, "WAVE_SPLIT=16,POINTS_X=1,ROWS_PER_THREAD=4")
+        second = run_guarded(capi, atoms, 0.5, 40, form, "WAVE_SPLIT=16,POINTS_X=1,ROWS_PER_THREAD=4")
+        np.testing.assert_array_equal(first, second)
+    for config in ("WAVE_SPLIT=17", "WAVE_SPLIT=0", "WAVE_SPLIT=2,POINTS_X=5", "WAVE_SPLIT=2,ROWS_PER_THREAD=6"):
+        with pytest.raises(capi.KttHipError, match="WAVE_SPLIT"):
+            run_guarded(capi, atoms, 0.5, 40, 0, config)
