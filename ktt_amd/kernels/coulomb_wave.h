@@ -121,6 +121,22 @@ struct WaveEngine
         return index < end ? atoms[index] : make_float4(kPadCoord, kPadCoord, kPadCoord, 0.0f);
     }
 
+    // h * i - X with the grid coordinate rounded first, as the reference kernel and its generator round
+    // it (Examples/CoulombSum3d/CoulombSum3d.cu:13-15): an atom at float(h * i) is then at distance 0.
+    template <class Real>
+    static __device__ __forceinline__ Real offset(const Real h, const int i, const Real X)
+    {
+#pragma clang fp contract(off)
+        const Real coordinate = h * static_cast<Real>(i);
+        return coordinate - X;
+    }
+
+    template <class Real>
+    static __device__ __forceinline__ Real square(const Real v)
+    {
+        return v * v;
+    }
+
     // One atom per lane into the wave's LDS, with the brackets of the wave's rows.
     // Compensated x: X = h n + d with n a near grid index and d formed in FP64, so that
     // x - X = h (i - n) - d carries one rounding whatever the coordinate's size. n is clamped to
@@ -146,13 +162,8 @@ struct WaveEngine
         int row = firstGroup * ROWS;
         int y = (MODE == Volume) ? row % rowsPerPlane : row;
         int z = (MODE == Volume) ? row / rowsPerPlane : 0;
-        Real dz2 = Z;
-        if constexpr (MODE == Volume)
-        {
-            const Real dz = step * static_cast<Real>(z) - Z;
-            dz2 = dz * dz;
-        }
-        Real dy = step * static_cast<Real>(y) - Y;
+        Real dz2 = (MODE == Volume) ? square(offset(step, z, Z)) : Z;
+        Real dy = offset(step, y, Y);
         const int quads = groups * (ROWS / 4);
 #pragma unroll 1
         for (int g = 0; g < quads; ++g)
@@ -171,13 +182,12 @@ struct WaveEngine
                 {
                     y = 0;
                     ++z;
-                    const Real dz = step * static_cast<Real>(z) - Z;
-                    dz2 = dz * dz;
+                    dz2 = square(offset(step, z, Z));
                     dy = -Y;
                 }
                 if constexpr (!COMP)
                 {
-                    dy = step * static_cast<Real>(y) - Y;
+                    dy = offset(step, y, Y);
                 }
             }
             *reinterpret_cast<float4*>(sB + g * 4) = make_float4(b[0], b[1], b[2], b[3]);

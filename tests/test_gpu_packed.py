@@ -72,6 +72,23 @@ def test_odd_spacings_and_far_atoms(capi, form):
         assert oracle.normalised_error(result, values, norms)[0] <= BARS[form]
 
 
+def test_plain_coordinates_round_as_the_reference_does(capi):
+    """A spacing FP32 rounds, atoms at float32(h * i): the reference generator forms the same rounded
+    coordinate and finds distance 0 there (+-inf); so must the plain form's default launch."""
+    grid, spacing = 30, np.float32(0.49)
+    atoms = workloads.uniform_atoms(79, 60, box=14.0)
+    cells = [(3, 17, 28), (29, 5, 11), (7, 7, 23)]
+    for k, (x, y, z) in enumerate(cells):
+        atoms[10 * k] = [spacing * np.float32(x), spacing * np.float32(y), spacing * np.float32(z), -0.5 if k else 0.5]
+    cpu = oracle.coulomb3d_f32(atoms, spacing, grid)
+    result = run_guarded(capi, atoms, float(spacing), grid, 0, None).reshape(grid, grid, grid)
+    for x, y, z in cells:
+        assert np.isinf(cpu[z, y, x]) and result[z, y, x] == cpu[z, y, x]
+    finite = np.isfinite(cpu)
+    assert np.array_equal(finite, np.isfinite(result))
+    assert np.max(np.abs(result[finite] - cpu[finite])) <= 0.01
+
+
 def test_repeats_are_bitwise_equal_and_bad_shapes_are_refused(capi):
     atoms = workloads.uniform_atoms(78, 700, box=20.0)
     for form in (0, 1):
