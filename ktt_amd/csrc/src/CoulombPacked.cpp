@@ -22,13 +22,14 @@ int RowGroupsPerWave(const int lanesX, const int rowGroups)
 }
 
 // The plan of a shape, or one with no workgroups when the shape does not fit the LDS or a launch.
-PackedPlan PlanShape(const int px, const int rows, const int waves, const int atomCount, const long rowLength, const long rowsTotal,
-    const bool compensated)
+PackedPlan PlanShape(const int px, const int rows, const int waves, const int blocks, const int atomCount, const long rowLength,
+    const long rowsTotal, const bool compensated)
 {
     PackedPlan plan;
     plan.px = px;
     plan.rows = rows;
     plan.waves = waves;
+    plan.blocks = blocks;
     const long lanesX = (rowLength + px - 1) / px;
     const long rowGroups = (rowsTotal + rows - 1) / rows;
     const long workgroups = (lanesX * rowGroups + 63) / 64;
@@ -41,11 +42,12 @@ PackedPlan PlanShape(const int px, const int rows, const int waves, const int at
         plan.cap *= 2;
     }
     // Whole unrolled steps of 8 atoms per wave.
-    const long perWave = (static_cast<long>(atomCount) + waves - 1) / waves;
+    const long shares = static_cast<long>(waves) * blocks;
+    const long perWave = (atomCount + shares - 1) / shares;
     plan.share = static_cast<int>(std::min<long>((perWave + 7) / 8 * 8, std::numeric_limits<int>::max()));
     const long ldsBytes = waves * 64L * ((compensated ? 4 : 2) + static_cast<long>(plan.cap) * rows + 4) * 4;
     // Lane numbers are 32-bit, and a launch holds fewer than 2^32 threads.
-    if (ldsBytes <= kLdsBytes && workgroups * 64 * waves <= 0x7fffffffL)
+    if (ldsBytes <= kLdsBytes && workgroups * 64 * shares <= 0x7fffffffL)
     {
         plan.ldsBytes = static_cast<unsigned int>(ldsBytes);
         plan.workgroups = static_cast<unsigned int>(workgroups);
@@ -63,11 +65,12 @@ struct Shape
     int wavesPerSimd; // at the kernel's registers, plain and compensated
     int wavesPerSimdCompensated;
 };
-const Shape kShapes[] = {{2, 8, 0.0932, 0.34, 8, 5}, {1, 8, 0.0505, 0.33, 7, 7}, {1, 4, 0.0268, 0.32, 8, 8}};
+const Shape kShapes[] = {{2, 8, 0.0943, 0.51, 6, 5}, {1, 8, 0.0493, 0.29, 7, 7}, {1, 4, 0.0255, 0.18, 8, 8}};
 
-// Estimated time of a plan in us. The constants are a fit to 110 grids of 24^3 to 640^3 points with 64 to
-// 30,000 atoms on MI355X, each timed at every shape and 1, 4, 8 and 16 waves; the shape it picks is
-// within 1.2% of the fastest on average (at worst 18%).
+// Estimated time of a plan in us. The constants are a fit to 19 grids of 24^3 to 384^3 points with 64 to
+// 30,000 atoms, both forms, each timed on MI355X at every shape and 1, 4, 8 and 16 waves: the shape it
+// picks is within 0.5% of the fastest on average (at worst 4%), while any one shape for all is up to
+// 10 times slower somewhere.
 double Estimate(const PackedPlan& plan, const Shape& shape, const bool compensated)
 {
     const double size = plan.px * plan.rows / 16.0;
@@ -75,9 +78,9 @@ double Estimate(const PackedPlan& plan, const Shape& shape, const bool compensat
     // One wave: its atoms, the brackets of its rows per 64 atoms, the start and the store, and, if
     // the waves of a workgroup split the atoms, their meeting in LDS.
     double wave = plan.share * shape.atom * (compensated ? 1.12 : 1.0);
-    wave += tiles * plan.touched * plan.rows * (compensated ? 0.010 : 0.0048);
-    wave += 0.13 + size * (compensated ? 0.48 : 0.35);
-    wave += plan.waves > 1 ? size * (compensated ? 0.42 : 0.26) : 0.0;
+    wave += tiles * plan.touched * plan.rows * (compensated ? 0.0115 : 0.0032);
+    wave += 0.064 + size * (compensated ? 0.83 : 0.43);
+    wave += plan.waves > 1 ? size * (compensated ? 0.83 : 0.26) : 0.0;
     // Waves per SIMD of the 256 CUs: whole workgroups per CU while they all fit at once; more than
     // that are handed out as others end, with a partial last round.
     constexpr double kComputeUnits = 256.0;
@@ -90,22 +93,26 @@ double Estimate(const PackedPlan& plan, const Shape& shape, const bool compensat
     if (load > resident)
     {
         busy = resident;
-        load = plan.workgroups * perGroup / kComputeUnits + 0.67 * std::max(1.0, perGroup);
+        load = plan.workgroups * perGroup / kComputeUnits + 0.97 * std::max(1.0, perGroup);
     }
-    const double rate = 1.0 - (1.0 - shape.alone) * std::pow(busy, -0.93);
-    return load * wave / rate;
+    const double rate = 1.0 - (1.0 - shape.alone) / busy;
+    return load * wave / rate + 0.0104 * busy;
 }
 
 } // namespace
 
-PackedPlan MakePackedPlan(const int px, const int rows, const int waves, const int atomCount, const long rowLength,
-    const long rowsTotal, const bool compensated)
+PackedPlan MakePackedPlan(const int px, const int rows, const int waves, const int blocks, const int atomCount,
+    const long rowLength, const long rowsTotal, const bool compensated)
 {
     if (px < 1 || px > 4 || (rows != 4 && rows != 8) || waves < 1 || waves > 16)
     {
         throw KttException("the wave engine takes WAVE_SPLIT 1 to 16, POINTS_X 1 to 4 and ROWS_PER_THREAD 4 or 8");
     }
-    const PackedPlan plan = PlanShape(px, rows, waves, atomCount, rowLength, rowsTotal, compensated);
+    if (blocks < 1 || blocks > 65535 || (compensated && blocks > 1))
+    {
+        throw KttException("WAVE_SPLIT takes ATOM_BLOCKS from 1 to 65,535 in the plain form and 1 in the compensated form");
+    }
+    const PackedPlan plan = PlanShape(px, rows, waves, blocks, atomCount, rowLength, rowsTotal, compensated);
     if (plan.workgroups == 0)
     {
         throw KttException("WAVE_SPLIT=" + std::to_string(waves) + " with " + std::to_string(px) + " x " + std::to_string(rows)
@@ -119,11 +126,18 @@ PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, const lon
 {
     PackedPlan best;
     double bestTime = std::numeric_limits<double>::max();
+    int bestSlots = 0;
     for (const Shape& shape : kShapes)
     {
         for (const int waves : {1, 4, 8, 16})
         {
-            const PackedPlan plan = PlanShape(shape.px, shape.rows, waves, atomCount, rowLength, rowsTotal, compensated);
+            const PackedPlan plan = PlanShape(shape.px, shape.rows, waves, 1, atomCount, rowLength, rowsTotal, compensated);
+            // One-wave workgroups win while a wave's atoms are a tile or two (256^3 x 64: 113 us against
+            // 117 with 4 waves) and lose 5 to 10% beyond (180^3 x 500: 303 against 280).
+            if (waves == 1 && atomCount > 128)
+            {
+                continue;
+            }
             // A short row wraps a wave over many row groups, whose brackets then cost more LDS and
             // instructions than a narrower block saves.
             if (plan.workgroups == 0 || (shape.px > 1 && plan.touched > 4))
@@ -135,8 +149,16 @@ PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, const lon
             {
                 bestTime = time;
                 best = plan;
+                bestSlots = compensated ? shape.wavesPerSimdCompensated : shape.wavesPerSimd;
             }
         }
+    }
+    // Four-wave workgroups that all start at once stay where the first round put them, unevenly; eight-wave
+    // ones leave a part for CUs that finish early (100^3 x 30,000: 2,882 us against 3,051).
+    if (best.waves == 4 && atomCount >= 256 && best.workgroups > 256u && best.workgroups <= 256u * static_cast<unsigned int>(bestSlots))
+    {
+        const PackedPlan wider = PlanShape(best.px, best.rows, 8, 1, atomCount, rowLength, rowsTotal, compensated);
+        best = wider.workgroups != 0 ? wider : best;
     }
     return best;
 }
@@ -145,7 +167,7 @@ PackedPlan PackedPlanOf(const CoulombConfig& config, const int atomCount, const 
     const bool compensated)
 {
     return MakePackedPlan(static_cast<int>(config.Get("POINTS_X", 2)), static_cast<int>(config.Get("ROWS_PER_THREAD", 8)),
-        static_cast<int>(config.Get("WAVE_SPLIT", 1)), atomCount, rowLength, rowsTotal, compensated);
+        static_cast<int>(config.Get("WAVE_SPLIT", 1)), static_cast<int>(config.Get("ATOM_BLOCKS", 1)), atomCount, rowLength, rowsTotal, compensated);
 }
 
 void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, float spacing, int rowLength, int rowsTotal,
@@ -155,7 +177,7 @@ void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, flo
         "-DROW_GROUP_CAP=" + std::to_string(plan.cap), std::string("-DCOMPENSATED=") + (compensated ? "1" : "0"),
         std::string("-DROW_MODE=") + (slice ? "1" : "0")};
     const auto kernel = CoulombRuntime::Get().GetKernel("CoulombPacked.hip", "coulombPacked", defines);
-    const unsigned int grid[3] = {plan.workgroups, 1, 1};
+    const unsigned int grid[3] = {plan.workgroups, static_cast<unsigned int>(plan.blocks), 1};
     const unsigned int block[3] = {static_cast<unsigned int>(plan.waves) * 64, 1, 1};
     int share = plan.share;
     int lanesX = plan.lanesX;

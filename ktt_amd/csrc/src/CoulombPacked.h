@@ -17,6 +17,7 @@ struct PackedPlan
     int touched = 0;    // row groups a wave touches at most, and that rounded up to a power of two
     int cap = 0;
     int waves = 0;
+    int blocks = 1;     // atom blocks (plain form; more than one add with FP32 atomics)
     int lanesX = 0;     // lanes per row group
     int rowGroups = 0;
     int share = 0;      // atoms per wave
@@ -26,13 +27,13 @@ struct PackedPlan
 
 /** The plan of one shape; throws KttException for a shape the kernel does not take or that does
  *  not fit the LDS. */
-PackedPlan MakePackedPlan(int px, int rows, int waves, int atomCount, long rowLength, long rowsTotal, bool compensated);
+PackedPlan MakePackedPlan(int px, int rows, int waves, int blocks, int atomCount, long rowLength, long rowsTotal, bool compensated);
 
 /** The shape with the smallest estimated time. */
 PackedPlan ChoosePackedPlan(int atomCount, long rowLength, long rowsTotal, bool compensated);
 
-/** The plan a configuration names: WAVE_SPLIT (waves), POINTS_X and ROWS_PER_THREAD, each optional
- *  but WAVE_SPLIT. */
+/** The plan a configuration names: WAVE_SPLIT (waves), POINTS_X, ROWS_PER_THREAD and ATOM_BLOCKS, each
+ *  optional but WAVE_SPLIT. */
 PackedPlan PackedPlanOf(const CoulombConfig& config, int atomCount, long rowLength, long rowsTotal, bool compensated);
 
 /** energyGrid += V on rows of rowLength points. slice: rows = y and the atoms' z holds dz^2; else

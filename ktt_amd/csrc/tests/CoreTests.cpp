@@ -633,7 +633,7 @@ void TestPackedPlan()
     {
         try
         {
-            ktt::MakePackedPlan(px, rows, waves, 100, side, side * side, true);
+            ktt::MakePackedPlan(px, rows, waves, 1, 100, side, side * side, true);
         }
         catch (const ktt::KttException&)
         {

@@ -5,11 +5,12 @@
 //
 //   POINTS_X, ROWS_PER_THREAD  points per lane (x run, rows)
 //   ROW_GROUP_CAP              row groups a wave may touch (kc::rowGroupsPerWave, rounded up)
-//   COMPENSATED                0: FP32 sums, 1: two-sum per 256 atoms, FP64 merge
+//   COMPENSATED                sums of 64 atoms added in 0: FP32, 1: FP64
 //   ROW_MODE                   0: a volume (rows = z * G + y), 1: one slice (rows = y, .z holds dz^2)
 //
-// Launch: block 64 x waves threads, one workgroup per 64 lanes; dynamic LDS of waves * WaveFloats floats.
-// Wave w sums atoms [w * share, w * share + share).
+// Launch: block 64 x waves threads, grid (64-lane blocks, atom blocks); dynamic LDS of waves * WaveFloats
+// floats. Wave w of atom block b sums atoms [(b * waves + w) * share, + share). Several atom blocks (plain
+// form only) add to the grid with FP32 atomics.
 #include "coulomb_wave.h"
 
 #ifndef ROW_GROUP_CAP
@@ -24,18 +25,18 @@
 
 using W = kc::WaveEngine<POINTS_X, ROWS_PER_THREAD, ROW_GROUP_CAP, ROW_MODE, COMPENSATED != 0>;
 
-// 5 waves per SIMD: the compensated 2 x 8 block takes 98 VGPRs by itself, 2 more than 5 waves allow.
+// 5 waves per SIMD: the compensated 2 x 8 block takes exactly the 96 VGPRs that they allow.
 extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5))) void coulombPacked(const float4* atoms, int numberOfAtoms, int share, float gridSpacing,
     int lanesX, int rowGroups, int rowLength, int rowsTotal, float* energyGrid)
 {
     extern __shared__ __attribute__((aligned(16))) float shared[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int waves = blockDim.x >> 6;
-    const long long first = static_cast<long long>(wave) * share;
+    const long long first = static_cast<long long>(blockIdx.y * waves + wave) * share;
     const int a0 = first < numberOfAtoms ? static_cast<int>(first) : numberOfAtoms;
     const int a1 = share < numberOfAtoms - a0 ? a0 + share : numberOfAtoms;
     W engine;
     engine.place(blockIdx.x, lanesX, rowGroups);
     engine.accumulate(shared + wave * W::WaveFloats, atoms, a0, a1, gridSpacing, rowLength);
-    engine.store(shared, waves, wave, energyGrid, rowLength, rowsTotal);
+    engine.store(shared, waves, wave, energyGrid, rowLength, rowsTotal, gridDim.y > 1);
 }
