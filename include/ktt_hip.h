@@ -138,7 +138,8 @@ int ktt_coulomb3d_reference(const float* atoms, int n_atoms, float spacing, int 
 /* CoulombSum2d, one slice: energy_grid[grid_y][grid_x] += V, where atoms[i].z holds the
  * squared z distance of atom i to the slice (Examples/CoulombSum2d/CoulombSum2d.cl:35-1026).
  * grid_x must be a multiple of WORK_GROUP_SIZE_X*POINTS_X and grid_y of
- * WORK_GROUP_SIZE_Y*ROWS_PER_THREAD. */
+ * WORK_GROUP_SIZE_Y*ROWS_PER_THREAD (of the defaults without a configuration; WAVE_SPLIT, as in
+ * ktt_coulomb3d and with ATOM_BLOCKS that add with FP32 atomics, takes any grid). */
 int ktt_coulomb2d(const float* atoms, int n_atoms, float spacing, int grid_x, int grid_y, float* energy_grid,
                   const char* config, void* stream, float* kernel_ms);
 
@@ -163,8 +164,10 @@ int ktt_coulomb3d_iterative(const float* host_atoms, int n_atoms, float spacing,
 int ktt_coulomb3d_iterative_reference(const float* atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
                                       void* stream, float* kernel_ms);
 
-/* Fused slice loop: the slice kernel forms dz^2 on the device (atoms with their real z on
- * the device), one launch per slice, no host work between launches. */
+/* Fused slice loop: dz^2 is formed on the device (atoms with their real z on the device). Without a
+ * configuration all slices run as the planes of one volume launch (ktt_coulomb3d, plain form); with
+ * one, the slice kernel is launched per slice, no host work between launches. Either way grid_size
+ * must be tiled by the slice kernel's workgroups, as for ktt_coulomb2d. */
 int ktt_coulomb3d_slices(const float* atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
                          const char* config, void* stream, float* kernel_ms);
 

@@ -927,6 +927,33 @@ static Coulomb3dPlan PlanCoulomb3d(const int atomCount, const int gridSize, cons
     return plan;
 }
 
+// The launch of ktt_coulomb3d (its arguments checked).
+static void LaunchVolume(const float* atoms, int atomCount, float spacing, int gridSize, float* energyGrid, const int form,
+    const char* config, hipStream_t stream, float* kernelMs)
+{
+    PackedPlan packed;
+    if (PackedPlanFor(atomCount, gridSize, form, config, packed))
+    {
+        LaunchPacked(packed, atoms, atomCount, spacing, gridSize, gridSize * gridSize, energyGrid, form == KTT_COULOMB_COMPENSATED, false,
+            stream, kernelMs);
+        return;
+    }
+    Coulomb3dPlan plan = PlanCoulomb3d(atomCount, gridSize, form, config);
+    const float* unused = nullptr;
+    if (form == KTT_COULOMB_PLAIN)
+    {
+        void* arguments[] = {&atoms, &unused, &unused, &unused, &unused, &atomCount, &spacing, &gridSize, &energyGrid};
+        CoulombRuntime::Launch(*plan.kernel, plan.grid, plan.shape.block, arguments, stream, kernelMs);
+        return;
+    }
+    auto& runtime = CoulombRuntime::Get();
+    void* partials = plan.partialBytes > 0 ? runtime.GetScratch("coulomb3d.partials", plan.partialBytes) : nullptr;
+    void* counters = runtime.GetScratch("coulomb3d.counters", std::max<size_t>(1, plan.counterCount) * sizeof(unsigned int));
+    void* arguments[] = {&atoms, &unused, &unused, &unused, &unused, &atomCount, &spacing, &gridSize, &energyGrid, &partials, &counters,
+        &plan.splitFrom};
+    CoulombRuntime::Launch(*plan.kernel, plan.grid, plan.shape.block, arguments, stream, kernelMs);
+}
+
 } // namespace ktt
 
 extern "C" {
@@ -942,28 +969,7 @@ int ktt_coulomb3d(const float* atoms, int atomCount, float spacing, int gridSize
     CheckAtoms(atoms, atomCount);
     CheckGrid(energyGrid, static_cast<long>(gridSize) * gridSize * gridSize);
     CheckForm(gridSize, form);
-    hipStream_t hipStream = static_cast<hipStream_t>(stream);
-    PackedPlan packed;
-    if (PackedPlanFor(atomCount, gridSize, form, config, packed))
-    {
-        LaunchPacked(packed, atoms, atomCount, spacing, gridSize, gridSize * gridSize, energyGrid, form == KTT_COULOMB_COMPENSATED, false,
-            hipStream, kernelMs);
-        return 0;
-    }
-    Coulomb3dPlan plan = PlanCoulomb3d(atomCount, gridSize, form, config);
-    const float* unused = nullptr;
-    if (form == KTT_COULOMB_PLAIN)
-    {
-        void* arguments[] = {&atoms, &unused, &unused, &unused, &unused, &atomCount, &spacing, &gridSize, &energyGrid};
-        CoulombRuntime::Launch(*plan.kernel, plan.grid, plan.shape.block, arguments, hipStream, kernelMs);
-        return 0;
-    }
-    auto& runtime = CoulombRuntime::Get();
-    void* partials = plan.partialBytes > 0 ? runtime.GetScratch("coulomb3d.partials", plan.partialBytes) : nullptr;
-    void* counters = runtime.GetScratch("coulomb3d.counters", std::max<size_t>(1, plan.counterCount) * sizeof(unsigned int));
-    void* arguments[] = {&atoms, &unused, &unused, &unused, &unused, &atomCount, &spacing, &gridSize, &energyGrid, &partials, &counters,
-        &plan.splitFrom};
-    CoulombRuntime::Launch(*plan.kernel, plan.grid, plan.shape.block, arguments, hipStream, kernelMs);
+    LaunchVolume(atoms, atomCount, spacing, gridSize, energyGrid, form, config, static_cast<hipStream_t>(stream), kernelMs);
     return 0;
     KTT_C_CATCH
 }
@@ -983,7 +989,8 @@ int ktt_coulomb3d_launch_plan(int atomCount, int gridSize, int form, const char*
     {
         CoulombRuntime::Get().EnsureDevice();
         plan.grid[0] = plan.shape.grid[0] = packed.workgroups;
-        plan.grid[1] = plan.grid[2] = 1;
+        plan.grid[1] = static_cast<unsigned int>(packed.blocks);
+        plan.grid[2] = 1;
         plan.shape.block[0] = static_cast<unsigned int>(packed.waves) * 64;
         plan.shape.block[1] = plan.shape.block[2] = 1;
         plan.splitFrom = static_cast<int>(packed.workgroups);
@@ -1087,6 +1094,13 @@ int ktt_coulomb2d(const float* atoms, int atomCount, float spacing, int gridX, i
         return SetLastError("grid sizes must be positive");
     }
     CheckGrid(energyGrid, static_cast<long>(gridX) * gridY);
+    const CoulombConfig given = CoulombConfig::Parse(config, CoulombConfig());
+    if (given.Has("WAVE_SPLIT"))
+    {
+        LaunchPacked(PackedPlanOf(given, atomCount, gridX, gridY, false), atoms, atomCount, spacing, gridX, gridY, energyGrid, false, true,
+            static_cast<hipStream_t>(stream), kernelMs);
+        return 0;
+    }
     const CoulombConfig parsed = CoulombConfig::Parse(config, DefaultsSlice(atomCount, gridX, gridY));
     const long atomBlocks = EffectiveAtomBlocks(parsed, atomCount);
     const CoulombShape shape = CoulombRuntime::RowShape(parsed, gridX, gridY, atomBlocks);
@@ -1097,6 +1111,17 @@ int ktt_coulomb2d(const float* atoms, int atomCount, float spacing, int gridX, i
     {
         return SetLastError("grid " + std::to_string(gridX) + "x" + std::to_string(gridY) + " is not a multiple of the workgroup span "
             + std::to_string(spanX) + "x" + std::to_string(shape.rowsPerGroup));
+    }
+    // A small slice is over in a few microseconds, most of them one workgroup's start: tile, barriers,
+    // brackets, adds. The wave engine in its smallest block, 32 atoms a wave, starts faster: 256^2 x
+    // 64 in 4.0 us against 5.9, x 500 in 6.2 against 7.5, 64^2 x 4,000 in 4.8 against 7.0. From about
+    // 75 million interactions on its finer split costs more than that saves (512^2 x 500: 16.0 against 15.7 us).
+    if (given.values.empty() && static_cast<long>(gridX) * gridY * atomCount <= 75000000L)
+    {
+        const int blocks = std::max(1, (atomCount + 255) / 256);
+        LaunchPacked(MakePackedPlan(1, 4, 8, blocks, atomCount, gridX, gridY, false), atoms, atomCount, spacing, gridX, gridY, energyGrid,
+            false, true, static_cast<hipStream_t>(stream), kernelMs);
+        return 0;
     }
     auto kernel = CoulombRuntime::Get().GetKernel("CoulombSum2d.hip", "directCoulombSum", parsed.Defines(kLaunchOnly));
     const float* unused = nullptr;
@@ -1293,6 +1318,15 @@ int ktt_coulomb3d_slices(const float* atoms, int atomCount, float spacing, int g
     const long atomBlocks = EffectiveAtomBlocks(parsed, atomCount);
     const CoulombShape shape = CoulombRuntime::RowShape(parsed, gridSize, gridSize, atomBlocks);
     CheckSliceGrid(shape, parsed, gridSize);
+    if (CoulombConfig::Parse(config, CoulombConfig()).values.empty())
+    {
+        // By default the slices are the planes of one volume launch: the same terms, without a launch's
+        // ramp and tail per slice, on a chip that one slice does not fill, and without the FP32 atomics
+        // of the slices' atom blocks.
+        LaunchVolume(atoms, atomCount, spacing, gridSize, energyGrid, KTT_COULOMB_PLAIN, nullptr, static_cast<hipStream_t>(stream),
+            kernelMs);
+        return 0;
+    }
     auto kernel = runtime.GetKernel("CoulombSum3dIterative.hip", "directCoulombSumSlice", parsed.Defines(kLaunchOnly));
     hipStream_t hipStream = static_cast<hipStream_t>(stream);
 

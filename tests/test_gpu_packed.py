@@ -98,3 +98,26 @@ def test_repeats_are_bitwise_equal_and_bad_shapes_are_refused(capi):
     for config in ("WAVE_SPLIT=17", "WAVE_SPLIT=0", "WAVE_SPLIT=2,POINTS_X=5", "WAVE_SPLIT=2,ROWS_PER_THREAD=6"):
         with pytest.raises(capi.KttHipError, match="WAVE_SPLIT"):
             run_guarded(capi, atoms, 0.5, 40, 0, config)
+
+
+@pytest.mark.parametrize("grid_x,grid_y,count,config", [
+    (64, 16, 1, None), (64, 16, 255, None), (128, 48, 257, None), (192, 32, 3000, None),
+    (50, 37, 100, "WAVE_SPLIT=2,POINTS_X=2,ROWS_PER_THREAD=8,ATOM_BLOCKS=3"),
+    (50, 37, 100, "WAVE_SPLIT=16,POINTS_X=1,ROWS_PER_THREAD=4"),
+])
+def test_slices(capi, grid_x, grid_y, count, config):
+    """One slice (dz^2 in .z): the default launch of small slices, one and several atom blocks, and a grid
+    that no workgroup tiles."""
+    spacing = 0.5
+    atoms = workloads.slice_dz2(workloads.uniform_atoms(80 + count, count, box=grid_x * spacing), 7.3)
+    start = np.full(grid_x * grid_y + 64, 7.0, dtype=np.float32)
+    start[:grid_x * grid_y] = 0.0
+    energy = capi.DeviceBuffer.from_array(start)
+    print(f"slice {grid_x} x {grid_y} atoms {count} config {config}", flush=True)
+    capi.coulomb2d(capi.DeviceBuffer.from_array(atoms), count, spacing, grid_x, grid_y, energy, config=config)
+    out = energy.download((grid_x * grid_y + 64,))
+    assert (out[grid_x * grid_y:] == 7.0).all()
+    y, x = np.meshgrid(np.arange(grid_y), np.arange(grid_x), indexing="ij")
+    points = np.stack([x.ravel(), y.ravel()], axis=1).astype(np.int32)
+    values, norms = oracle.points2d_f64(atoms, spacing, points)
+    assert oracle.normalised_error(out[:grid_x * grid_y], values, norms)[0] <= BARS[0]
