@@ -123,8 +123,8 @@ int ktt_coulomb3d_launch_plan(int n_atoms, int grid_size, int form, const char* 
  * No counterpart in the reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, serving loops, harnesses that forbid hipMalloc). The kernels are
  * compiled ahead of time (libktt_hip_noalloc.so, loaded on the first call) and their scratch
- * (the tail split's FP64-merged partials and arrival counters) is a static device array of
- * 64 MiB + 64 KiB per device; a launch needing more is rejected. The first call on a device
+ * (the tail split's FP64-merged partials and arrival counters, at the sides that do not run the wave
+ * engine) is a static device array of 64 MiB + 64 KiB per device; a launch needing more is rejected. The first call on a device
  * sets up (symbol address, occupancy): make it outside graph capture. Calls that overlap on
  * one device race on the shared scratch. grid_size in [1, 46340] (row groups fold as in
  * ktt_coulomb3d); atoms 16-byte aligned. */

@@ -125,7 +125,7 @@ def build_noalloc() -> Path:
     gfx950; libktt_hip.so loads it on first use)."""
     temporary = NOALLOC_LIBRARY.with_suffix(".so.tmp")
     _run([str(ROCM / "bin" / "hipcc"), f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared", *HIP_DEVICE_FLAGS,
-          f"-I{KERNELS}", str(CSRC / "noalloc" / "CoulombNoAlloc.hip"), "-o", str(temporary)])
+          f"-I{KERNELS}", f"-I{CSRC / 'src'}", str(CSRC / "noalloc" / "CoulombNoAlloc.hip"), "-o", str(temporary)])
     os.replace(temporary, NOALLOC_LIBRARY)
     return NOALLOC_LIBRARY
 

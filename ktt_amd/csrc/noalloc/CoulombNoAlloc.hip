@@ -7,7 +7,9 @@
 // KTT_COULOMB_COMPENSATED and the default configuration (same kernel body,
 // kc::volumeCompensated, at the same tile shapes, with the tail split):
 //   grid side a multiple of 256: 128 x 2 threads, 2 x 8 points per thread, tile 256, unroll 16
-//   otherwise:                    64 x 2 threads, same per-thread block.
+//   other sides above 1,024:      64 x 2 threads, same per-thread block
+//   other sides up to 1,024:      the wave engine (kc::packedSum) at the shape of
+//                                 ktt::ChoosePackedPlan, which needs no scratch.
 //
 // Scratch.  The split tiles' (sum, comp) partials and their arrival counters live in the
 // file-scope array `scratch` (kScratchBytes per device, held by every GPU the library runs on
@@ -26,7 +28,9 @@
 #include <cstdio>
 #include <mutex>
 
+#include "CoulombPackedPlan.h"
 #include "coulomb_volume.h"
+#include "coulomb_wave.h"
 
 namespace
 {
@@ -80,6 +84,15 @@ extern "C" __global__ __launch_bounds__(NarrowShape::Threads) void kttNoAllocCom
     kc::volumeCompensated<NarrowShape>(src, numberOfAtoms, gridSpacing, gridSize, energyGrid, partials, tileCounters, splitFrom);
 }
 
+template <int PX, int ROWS, int CAP>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5))) void kttNoAllocPacked(const float4* atoms,
+    int numberOfAtoms, int share, float gridSpacing, int lanesX, int rowGroups, int rowLength, int rowsTotal, float* energyGrid)
+{
+    extern __shared__ __attribute__((aligned(16))) float shared[];
+    kc::packedSum<kc::WaveEngine<PX, ROWS, CAP, kc::Volume, true>>(shared, atoms, numberOfAtoms, share, gridSpacing, lanesX,
+        rowGroups, rowLength, rowsTotal, energyGrid);
+}
+
 extern "C" __global__ __launch_bounds__(256) void kttNoAllocClear(unsigned int* values, unsigned int count)
 {
     for (unsigned int i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x)
@@ -107,6 +120,34 @@ int FailHip(char* message, const size_t length, const char* what, const hipError
         std::snprintf(message, length, "%s: %s", what, hipGetErrorString(status));
     }
     return -1;
+}
+
+using PackedKernel = void (*)(const float4*, int, int, float, int, int, int, int, float*);
+
+// The precompiled kernel of a shape, or null. ChoosePackedPlan gives 2 x 8 points with up to 4 row groups
+// per wave, 1 x 8 with up to 8 and 1 x 4 with up to 16 (a side of 6 or 7).
+PackedKernel PackedKernelOf(const ktt::PackedPlan& plan)
+{
+    struct Entry
+    {
+        int px;
+        int rows;
+        int cap;
+        PackedKernel kernel;
+    };
+    static const Entry entries[] = {{2, 8, 1, kttNoAllocPacked<2, 8, 1>}, {2, 8, 2, kttNoAllocPacked<2, 8, 2>},
+        {2, 8, 4, kttNoAllocPacked<2, 8, 4>}, {1, 8, 1, kttNoAllocPacked<1, 8, 1>}, {1, 8, 2, kttNoAllocPacked<1, 8, 2>},
+        {1, 8, 4, kttNoAllocPacked<1, 8, 4>}, {1, 8, 8, kttNoAllocPacked<1, 8, 8>}, {1, 4, 1, kttNoAllocPacked<1, 4, 1>},
+        {1, 4, 2, kttNoAllocPacked<1, 4, 2>}, {1, 4, 4, kttNoAllocPacked<1, 4, 4>}, {1, 4, 8, kttNoAllocPacked<1, 4, 8>},
+        {1, 4, 16, kttNoAllocPacked<1, 4, 16>}};
+    for (const Entry& entry : entries)
+    {
+        if (entry.px == plan.px && entry.rows == plan.rows && entry.cap == plan.cap)
+        {
+            return entry.kernel;
+        }
+    }
+    return nullptr;
 }
 
 // Set-up of the current device, once: the device address of `scratch`, the CU count and
@@ -195,6 +236,20 @@ extern "C" __attribute__((visibility("default"))) int ktt_noalloc_coulomb3d_comp
     if (EnsureDevice(state, message, messageLength) != 0)
     {
         return -1;
+    }
+
+    if (ktt::WaveEngineByDefault(gridSize))
+    {
+        const ktt::PackedPlan plan = ktt::ChoosePackedPlan(atomCount, gridSize, static_cast<long>(gridSize) * gridSize, true);
+        const PackedKernel kernel = PackedKernelOf(plan);
+        if (kernel != nullptr)
+        {
+            hipLaunchKernelGGL(kernel, dim3(plan.workgroups), dim3(64 * plan.waves), plan.ldsBytes, static_cast<hipStream_t>(stream),
+                reinterpret_cast<const float4*>(atoms), atomCount, plan.share, spacing, plan.lanesX, plan.rowGroups, gridSize,
+                gridSize * gridSize, energyGrid);
+            const hipError_t status = hipGetLastError();
+            return status == hipSuccess ? 0 : FailHip(message, messageLength, "launch of the compensated Coulomb kernel", status);
+        }
     }
 
     // The launch plan of ktt_coulomb3d (compensated, default configuration, TAIL_SPLIT=1).

@@ -869,7 +869,7 @@ static bool PackedPlanFor(const int atomCount, const int gridSize, const int for
         plan = PackedPlanOf(given, atomCount, gridSize, rows, compensated);
         return true;
     }
-    if (!given.values.empty() || gridSize % 256 == 0 || gridSize > 1024)
+    if (!given.values.empty() || !WaveEngineByDefault(gridSize))
     {
         return false;
     }

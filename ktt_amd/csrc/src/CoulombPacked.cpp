@@ -1,105 +1,9 @@
 #include "CoulombPacked.h"
 
-#include <algorithm>
-#include <cmath>
-#include <limits>
-
 #include <KttException.h>
 
 namespace ktt
 {
-
-namespace
-{
-
-// LDS of a workgroup on gfx950.
-constexpr long kLdsBytes = 160 * 1024;
-
-// Row groups a wave of 64 lanes touches at most (kc::rowGroupsPerWave), of those there are.
-int RowGroupsPerWave(const int lanesX, const int rowGroups)
-{
-    return std::min(rowGroups, lanesX % 64 == 0 ? 1 : (64 % lanesX == 0 ? 64 / lanesX : (64 - 2) / lanesX + 2));
-}
-
-// The plan of a shape, or one with no workgroups when the shape does not fit the LDS or a launch.
-PackedPlan PlanShape(const int px, const int rows, const int waves, const int blocks, const int atomCount, const long rowLength,
-    const long rowsTotal, const bool compensated)
-{
-    PackedPlan plan;
-    plan.px = px;
-    plan.rows = rows;
-    plan.waves = waves;
-    plan.blocks = blocks;
-    const long lanesX = (rowLength + px - 1) / px;
-    const long rowGroups = (rowsTotal + rows - 1) / rows;
-    const long workgroups = (lanesX * rowGroups + 63) / 64;
-    plan.lanesX = static_cast<int>(lanesX);
-    plan.rowGroups = static_cast<int>(rowGroups);
-    plan.touched = RowGroupsPerWave(plan.lanesX, plan.rowGroups);
-    plan.cap = 1;
-    while (plan.cap < plan.touched)
-    {
-        plan.cap *= 2;
-    }
-    // Whole unrolled steps of 8 atoms per wave.
-    const long shares = static_cast<long>(waves) * blocks;
-    const long perWave = (atomCount + shares - 1) / shares;
-    plan.share = static_cast<int>(std::min<long>((perWave + 7) / 8 * 8, std::numeric_limits<int>::max()));
-    const long ldsBytes = waves * 64L * ((compensated ? 4 : 2) + static_cast<long>(plan.cap) * rows + 4) * 4;
-    // Lane numbers are 32-bit, and a launch holds fewer than 2^32 threads.
-    if (ldsBytes <= kLdsBytes && workgroups * 64 * shares <= 0x7fffffffL)
-    {
-        plan.ldsBytes = static_cast<unsigned int>(ldsBytes);
-        plan.workgroups = static_cast<unsigned int>(workgroups);
-    }
-    return plan;
-}
-
-// The shapes tried, with what the estimate below needs of each.
-struct Shape
-{
-    int px;
-    int rows;
-    double atom;      // us a SIMD takes per wave and atom with enough waves to hide latency
-    double alone;     // share of that rate that one wave per SIMD reaches
-    int wavesPerSimd; // at the kernel's registers, plain and compensated
-    int wavesPerSimdCompensated;
-};
-const Shape kShapes[] = {{2, 8, 0.0943, 0.51, 6, 5}, {1, 8, 0.0493, 0.29, 7, 7}, {1, 4, 0.0255, 0.18, 8, 8}};
-
-// Estimated time of a plan in us. The constants are a fit to 19 grids of 24^3 to 384^3 points with 64 to
-// 30,000 atoms, both forms, each timed on MI355X at every shape and 1, 4, 8 and 16 waves: the shape it
-// picks is within 0.5% of the fastest on average (at worst 4%), while any one shape for all is up to
-// 10 times slower somewhere.
-double Estimate(const PackedPlan& plan, const Shape& shape, const bool compensated)
-{
-    const double size = plan.px * plan.rows / 16.0;
-    const double tiles = (plan.share + 63) / 64;
-    // One wave: its atoms, the brackets of its rows per 64 atoms, the start and the store, and, if
-    // the waves of a workgroup split the atoms, their meeting in LDS.
-    double wave = plan.share * shape.atom * (compensated ? 1.12 : 1.0);
-    wave += tiles * plan.touched * plan.rows * (compensated ? 0.0115 : 0.0032);
-    wave += 0.064 + size * (compensated ? 0.83 : 0.43);
-    wave += plan.waves > 1 ? size * (compensated ? 0.83 : 0.26) : 0.0;
-    // Waves per SIMD of the 256 CUs: whole workgroups per CU while they all fit at once; more than
-    // that are handed out as others end, with a partial last round.
-    constexpr double kComputeUnits = 256.0;
-    const int slots = compensated ? shape.wavesPerSimdCompensated : shape.wavesPerSimd;
-    const double perGroup = plan.waves / 4.0;
-    const double resident = plan.waves < 4 ? slots : std::max(1, slots * 4 / plan.waves) * perGroup;
-    double load = plan.waves < 4 ? std::ceil(plan.workgroups * perGroup / kComputeUnits)
-                                 : std::ceil(plan.workgroups / kComputeUnits) * perGroup;
-    double busy = load;
-    if (load > resident)
-    {
-        busy = resident;
-        load = plan.workgroups * perGroup / kComputeUnits + 0.97 * std::max(1.0, perGroup);
-    }
-    const double rate = 1.0 - (1.0 - shape.alone) / busy;
-    return load * wave / rate + 0.0104 * busy;
-}
-
-} // namespace
 
 PackedPlan MakePackedPlan(const int px, const int rows, const int waves, const int blocks, const int atomCount,
     const long rowLength, const long rowsTotal, const bool compensated)
@@ -122,52 +26,15 @@ PackedPlan MakePackedPlan(const int px, const int rows, const int waves, const i
     return plan;
 }
 
-PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, const long rowsTotal, const bool compensated)
-{
-    PackedPlan best;
-    double bestTime = std::numeric_limits<double>::max();
-    int bestSlots = 0;
-    for (const Shape& shape : kShapes)
-    {
-        for (const int waves : {1, 4, 8, 16})
-        {
-            const PackedPlan plan = PlanShape(shape.px, shape.rows, waves, 1, atomCount, rowLength, rowsTotal, compensated);
-            // One-wave workgroups win while a wave's atoms are a tile or two (256^3 x 64: 113 us against
-            // 117 with 4 waves) and lose 5 to 10% beyond (180^3 x 500: 303 against 280).
-            if (waves == 1 && atomCount > 128)
-            {
-                continue;
-            }
-            // A short row wraps a wave over many row groups, whose brackets then cost more LDS and
-            // instructions than a narrower block saves.
-            if (plan.workgroups == 0 || (shape.px > 1 && plan.touched > 4))
-            {
-                continue;
-            }
-            const double time = Estimate(plan, shape, compensated);
-            if (time < bestTime)
-            {
-                bestTime = time;
-                best = plan;
-                bestSlots = compensated ? shape.wavesPerSimdCompensated : shape.wavesPerSimd;
-            }
-        }
-    }
-    // Four-wave workgroups that all start at once stay where the first round put them, unevenly; eight-wave
-    // ones leave a part for CUs that finish early (100^3 x 30,000: 2,882 us against 3,051).
-    if (best.waves == 4 && atomCount >= 256 && best.workgroups > 256u && best.workgroups <= 256u * static_cast<unsigned int>(bestSlots))
-    {
-        const PackedPlan wider = PlanShape(best.px, best.rows, 8, 1, atomCount, rowLength, rowsTotal, compensated);
-        best = wider.workgroups != 0 ? wider : best;
-    }
-    return best;
-}
-
 PackedPlan PackedPlanOf(const CoulombConfig& config, const int atomCount, const long rowLength, const long rowsTotal,
     const bool compensated)
 {
-    return MakePackedPlan(static_cast<int>(config.Get("POINTS_X", 2)), static_cast<int>(config.Get("ROWS_PER_THREAD", 8)),
-        static_cast<int>(config.Get("WAVE_SPLIT", 1)), static_cast<int>(config.Get("ATOM_BLOCKS", 1)), atomCount, rowLength, rowsTotal, compensated);
+    const auto value = [&config](const char* name, const long fallback)
+    {
+        return static_cast<int>(std::min<long>(std::max<long>(config.Get(name, fallback), -1), 1 << 20));
+    };
+    return MakePackedPlan(value("POINTS_X", 2), value("ROWS_PER_THREAD", 8), value("WAVE_SPLIT", 1), value("ATOM_BLOCKS", 1), atomCount,
+        rowLength, rowsTotal, compensated);
 }
 
 void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, float spacing, int rowLength, int rowsTotal,

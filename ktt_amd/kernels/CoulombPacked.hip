@@ -8,9 +8,7 @@
 //   COMPENSATED                sums of 64 atoms added in 0: FP32, 1: FP64
 //   ROW_MODE                   0: a volume (rows = z * G + y), 1: one slice (rows = y, .z holds dz^2)
 //
-// Launch: block 64 x waves threads, grid (64-lane blocks, atom blocks); dynamic LDS of waves * WaveFloats
-// floats. Wave w of atom block b sums atoms [(b * waves + w) * share, + share). Several atom blocks (plain
-// form only) add to the grid with FP32 atomics.
+// Launch: kc::packedSum. Several atom blocks (plain form only) add to the grid with FP32 atomics.
 #include "coulomb_wave.h"
 
 #ifndef ROW_GROUP_CAP
@@ -30,13 +28,5 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
     int lanesX, int rowGroups, int rowLength, int rowsTotal, float* energyGrid)
 {
     extern __shared__ __attribute__((aligned(16))) float shared[];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int waves = blockDim.x >> 6;
-    const long long first = static_cast<long long>(blockIdx.y * waves + wave) * share;
-    const int a0 = first < numberOfAtoms ? static_cast<int>(first) : numberOfAtoms;
-    const int a1 = share < numberOfAtoms - a0 ? a0 + share : numberOfAtoms;
-    W engine;
-    engine.place(blockIdx.x, lanesX, rowGroups);
-    engine.accumulate(shared + wave * W::WaveFloats, atoms, a0, a1, gridSpacing, rowLength);
-    engine.store(shared, waves, wave, energyGrid, rowLength, rowsTotal, gridDim.y > 1);
+    kc::packedSum<W>(shared, atoms, numberOfAtoms, share, gridSpacing, lanesX, rowGroups, rowLength, rowsTotal, energyGrid);
 }

@@ -410,4 +410,21 @@ struct WaveEngine
     }
 };
 
+// The body of a wave-engine kernel: block 64 x waves threads, grid (64-lane blocks, atom blocks), dynamic
+// LDS of waves * WaveFloats floats. Wave w of atom block b sums atoms [(b * waves + w) * share, + share).
+template <class W>
+__device__ __forceinline__ void packedSum(float* shared, const float4* atoms, const int numberOfAtoms, const int share,
+    const float gridSpacing, const int lanesX, const int rowGroups, const int rowLength, const int rowsTotal, float* energyGrid)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const long long first = static_cast<long long>(blockIdx.y * waves + wave) * share;
+    const int a0 = first < numberOfAtoms ? static_cast<int>(first) : numberOfAtoms;
+    const int a1 = share < numberOfAtoms - a0 ? a0 + share : numberOfAtoms;
+    W engine;
+    engine.place(blockIdx.x, lanesX, rowGroups);
+    engine.accumulate(shared + wave * W::WaveFloats, atoms, a0, a1, gridSpacing, rowLength);
+    engine.store(shared, waves, wave, energyGrid, rowLength, rowsTotal, gridDim.y > 1);
+}
+
 } // namespace kc

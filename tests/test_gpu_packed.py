@@ -121,3 +121,25 @@ def test_slices(capi, grid_x, grid_y, count, config):
     points = np.stack([x.ravel(), y.ravel()], axis=1).astype(np.int32)
     values, norms = oracle.points2d_f64(atoms, spacing, points)
     assert oracle.normalised_error(out[:grid_x * grid_y], values, norms)[0] <= BARS[0]
+
+
+@pytest.mark.parametrize("grid,count", [(1, 5), (6, 30), (9, 100), (24, 700), (45, 300), (63, 64), (70, 3000), (100, 501)])
+def test_no_alloc_entry_point_takes_the_same_shapes(capi, grid, count):
+    """ktt_coulomb3d_compensated_noalloc at sides that run the wave engine, one for each of its
+    precompiled kernels' row-group caps and blocks, against FP64 and ktt_coulomb3d."""
+    spacing = 0.5
+    atoms = workloads.uniform_atoms(90 + grid, count, box=max(grid, 4) * spacing)
+    start = np.zeros(grid ** 3 + 64, dtype=np.float32)
+    start[grid ** 3:] = 7.0
+    energy = capi.DeviceBuffer.from_array(start)
+    print(f"no-alloc grid {grid} atoms {count}", flush=True)
+    capi.coulomb3d_compensated_noalloc(capi.DeviceBuffer.from_array(atoms), count, spacing, grid, energy)
+    capi.synchronize()
+    out = energy.download((grid ** 3 + 64,))
+    assert (out[grid ** 3:] == 7.0).all()
+    points = workloads.sample_points(91, 2048, grid)
+    values, norms = oracle.points_f64(atoms, spacing, points)
+    index = (points[:, 2].astype(np.int64) * grid + points[:, 1]) * grid + points[:, 0]
+    assert oracle.normalised_error(out[index], values, norms)[0] <= BARS[1]
+    other = run_guarded(capi, atoms, spacing, grid, 1, None)
+    assert (np.abs(out[index].astype(np.float64) - other[index]) / norms).max() <= BARS[1]
