@@ -78,6 +78,8 @@ KERNEL_CHECKS = [
     ("CoulombSum3dZ.hip", "directCoulombSum", "Z_ITERATIONS=4,USE_SOA=1,VECTOR_SIZE=4"),
     ("Nbody.hip", "nbody_kernel", None),
     ("Nbody.hip", "nbody_kernel", "WORK_GROUP_SIZE_X=64,WORK_GROUP_SIZE_Y=4,BODIES_PER_THREAD=8,ATOM_TILE=512,INNER_UNROLL_FACTOR=8,USE_SOA=1"),
+    ("NbodySplit.hip", "nbody_split", None),
+    ("NbodySplit.hip", "nbody_split", "BODY_LANES=8,BODIES_PER_THREAD=1"),
     ("NbodyReference.hip", "nbody_kernel_reference", None),
     ("CoulombBatched.hip", "coulombBatchedPersistent", None),
     ("CoulombBatched.hip", "coulombBatchedSystem", None),

@@ -68,6 +68,44 @@ CoulombConfig NbodyDefaults()
     return defaults;
 }
 
+// A shape of nbody_split (NbodySplit.hip): lanes along the bodies and bodies per thread.
+struct SplitShape
+{
+    long lanes;
+    long bodies;
+};
+
+// The default launch: workgroups of 16 waves own lanes x bodies targets, so few bodies want few lanes. The
+// busiest of the 256 CUs runs ceil(workgroups / 256) of them; a target costs more in the smaller shapes
+// (fewer steps per barrier, fewer targets per source read), and a CU with one workgroup has 4 waves per
+// SIMD where two pair their instructions better. Costs per target from a sweep of 1,024 to 196,608 bodies
+// on MI355X; the shape picked is the fastest of 15 or within 2% of it. Start shape (64 x 16 threads, 4
+// bodies) -> this rule: 4,096 bodies 69 -> 8.4 us, 16,384 263 -> 71, 65,536 1,071 -> 1,016, 98,304
+// 3,006 -> 2,270, 131,072 4,001 -> 3,973.
+SplitShape ChooseSplitShape(const int n)
+{
+    struct Candidate
+    {
+        SplitShape shape;
+        double cost;
+    };
+    const Candidate candidates[] = {{{64, 4}, 1.0}, {{32, 4}, 1.01}, {{16, 4}, 1.02}, {{8, 4}, 1.045}, {{8, 2}, 1.13}, {{8, 1}, 1.3}};
+    SplitShape best = candidates[0].shape;
+    double bestTime = 0.0;
+    for (const Candidate& candidate : candidates)
+    {
+        const long targets = candidate.shape.lanes * candidate.shape.bodies;
+        const long perUnit = ((n + targets - 1) / targets + 255) / 256;
+        const double time = static_cast<double>(perUnit * targets) * candidate.cost * (perUnit == 1 ? 1.07 : 1.0);
+        if (bestTime == 0.0 || time < bestTime)
+        {
+            bestTime = time;
+            best = candidate.shape;
+        }
+    }
+    return best;
+}
+
 void CheckBodies(const void* bodies, const void* velocity, const void* newBodies, const void* newVelocity, const int n)
 {
     if (n <= 0)
@@ -94,6 +132,31 @@ int ktt_nbody_step(const float* bodyInfo, const float* velocity, int n, float ti
     try
     {
         CheckBodies(bodyInfo, velocity, newBodyInfo, newVelocity, n);
+        const CoulombConfig given = CoulombConfig::Parse(config, CoulombConfig());
+        if (given.values.empty() || given.Has("BODY_LANES"))
+        {
+            const SplitShape shape = given.values.empty() ? ChooseSplitShape(n) : SplitShape{given.Get("BODY_LANES", 64),
+                given.Get("BODIES_PER_THREAD", 4)};
+            if (n % 1024 != 0)
+            {
+                return SetLastError("the number of bodies (" + std::to_string(n) + ") must be a multiple of 1024");
+            }
+            if (shape.lanes < 1 || 64 % shape.lanes != 0 || shape.bodies < 1 || 1024 % (shape.lanes * shape.bodies) != 0
+                || shape.lanes * shape.bodies > 256)
+            {
+                return SetLastError("invalid N-body configuration " + given.ToString() + ": BODY_LANES must divide 64 and BODY_LANES * "
+                    "BODIES_PER_THREAD be a power of two up to 256");
+            }
+            CoulombConfig defines = given;
+            defines.Set("BODY_LANES", std::to_string(shape.lanes));
+            defines.Set("BODIES_PER_THREAD", std::to_string(shape.bodies));
+            auto kernel = CoulombRuntime::Get().GetKernel("NbodySplit.hip", "nbody_split", defines.Defines({}));
+            const unsigned int grid[3] = {static_cast<unsigned int>(n / (shape.lanes * shape.bodies)), 1, 1};
+            const unsigned int block[3] = {1024, 1, 1};
+            void* arguments[] = {&timeDelta, &bodyInfo, &newBodyInfo, &velocity, &newVelocity, &damping, &softeningSqr, &n};
+            CoulombRuntime::Launch(*kernel, grid, block, arguments, static_cast<hipStream_t>(stream), kernelMs);
+            return 0;
+        }
         const CoulombConfig parsed = CoulombConfig::Parse(config, NbodyDefaults());
         if (parsed.Get("USE_SOA", 0) != 0)
         {
