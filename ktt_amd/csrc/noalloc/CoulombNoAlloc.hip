@@ -136,8 +136,8 @@ PackedKernel PackedKernelOf(const ktt::PackedPlan& plan)
         PackedKernel kernel;
     };
     static const Entry entries[] = {{2, 8, 1, kttNoAllocPacked<2, 8, 1>}, {2, 8, 2, kttNoAllocPacked<2, 8, 2>},
-        {2, 8, 4, kttNoAllocPacked<2, 8, 4>}, {1, 8, 1, kttNoAllocPacked<1, 8, 1>}, {1, 8, 2, kttNoAllocPacked<1, 8, 2>},
-        {1, 8, 4, kttNoAllocPacked<1, 8, 4>}, {1, 8, 8, kttNoAllocPacked<1, 8, 8>}, {1, 4, 1, kttNoAllocPacked<1, 4, 1>},
+        {2, 8, 3, kttNoAllocPacked<2, 8, 3>}, {2, 8, 4, kttNoAllocPacked<2, 8, 4>}, {1, 8, 1, kttNoAllocPacked<1, 8, 1>}, {1, 8, 2, kttNoAllocPacked<1, 8, 2>},
+        {1, 8, 3, kttNoAllocPacked<1, 8, 3>}, {1, 8, 4, kttNoAllocPacked<1, 8, 4>}, {1, 8, 8, kttNoAllocPacked<1, 8, 8>}, {1, 4, 1, kttNoAllocPacked<1, 4, 1>},
         {1, 4, 2, kttNoAllocPacked<1, 4, 2>}, {1, 4, 4, kttNoAllocPacked<1, 4, 4>}, {1, 4, 8, kttNoAllocPacked<1, 4, 8>},
         {1, 4, 16, kttNoAllocPacked<1, 4, 16>}};
     for (const Entry& entry : entries)

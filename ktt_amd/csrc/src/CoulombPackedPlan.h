@@ -17,7 +17,7 @@ struct PackedPlan
 {
     int px = 0;
     int rows = 0;
-    int touched = 0;    // row groups a wave touches at most, and that rounded up to a power of two
+    int touched = 0;    // row groups a wave touches at most, and what the kernel is compiled for
     int cap = 0;
     int waves = 0;
     int blocks = 1;     // atom blocks (plain form; more than one add with FP32 atomics)
@@ -37,6 +37,23 @@ inline int RowGroupsPerWave(const int lanesX, const int rowGroups)
     return std::min(rowGroups, lanesX % 64 == 0 ? 1 : (64 % lanesX == 0 ? 64 / lanesX : (64 - 2) / lanesX + 2));
 }
 
+// Row groups a kernel is compiled for when its waves touch up to `touched` of them: the next power of two,
+// and 3 for groups of 8 rows, whose brackets then leave room for 19 waves per CU instead of 16 (3
+// groups of 4 rows would put the lanes' 16-byte bracket stores on the same LDS banks).
+inline int RowGroupCap(const int touched, const int rows)
+{
+    if (touched == 3 && rows == 8)
+    {
+        return 3;
+    }
+    int cap = 1;
+    while (cap < touched)
+    {
+        cap *= 2;
+    }
+    return cap;
+}
+
 // The plan of a shape, or one with no workgroups when the shape does not fit the LDS or a launch.
 inline PackedPlan PlanShape(const int px, const int rows, const int waves, const int blocks, const int atomCount, const long rowLength,
     const long rowsTotal, const bool compensated)
@@ -52,11 +69,7 @@ inline PackedPlan PlanShape(const int px, const int rows, const int waves, const
     plan.lanesX = static_cast<int>(lanesX);
     plan.rowGroups = static_cast<int>(rowGroups);
     plan.touched = RowGroupsPerWave(plan.lanesX, plan.rowGroups);
-    plan.cap = 1;
-    while (plan.cap < plan.touched)
-    {
-        plan.cap *= 2;
-    }
+    plan.cap = RowGroupCap(plan.touched, rows);
     // Whole unrolled steps of 8 atoms per wave.
     const long shares = static_cast<long>(waves) * blocks;
     const long perWave = (atomCount + shares - 1) / shares;
@@ -81,38 +94,44 @@ struct PackedShape
     int wavesPerSimd; // at the kernel's registers, plain and compensated
     int wavesPerSimdCompensated;
 };
-constexpr PackedShape kPackedShapes[] = {{2, 8, 0.0943, 0.51, 6, 5}, {1, 8, 0.0493, 0.29, 7, 7}, {1, 4, 0.0255, 0.18, 8, 8}};
+constexpr PackedShape kPackedShapes[] = {{2, 8, 0.0785, 0.58, 6, 5}, {1, 8, 0.0413, 0.41, 7, 7}, {1, 4, 0.0204, 0.24, 8, 8}};
 
-// Estimated time of a plan in us. The constants are a fit to 19 grids of 24^3 to 384^3 points with 64 to
-// 30,000 atoms, both forms, each timed on MI355X at every shape and 1, 4, 8 and 16 waves: the shape it
-// picks is within 0.5% of the fastest on average (at worst 4%), while any one shape for all is up to
-// 10 times slower somewhere.
+// Workgroups a CU holds at once, by registers and LDS.
+inline int PackedGroupsPerUnit(const PackedPlan& plan, const PackedShape& shape, const bool compensated)
+{
+    const int slots = compensated ? shape.wavesPerSimdCompensated : shape.wavesPerSimd;
+    return std::max(1, std::min(slots * 4 / plan.waves, static_cast<int>(kPackedLdsBytes / plan.ldsBytes)));
+}
+
+// Estimated time of a plan in us beyond the launch itself. The constants are a fit to 26 grids of 24^3 to
+// 330^3 points with 64 to 20,000 atoms, both forms, each timed on MI355X at every shape and 1, 4, 8 and
+// 16 waves: the shape it picks is within 1% of the fastest on average (at worst 8%), while any one
+// shape for all is several times slower somewhere.
 inline double EstimatePacked(const PackedPlan& plan, const PackedShape& shape, const bool compensated)
 {
+    constexpr double kComputeUnits = 256.0;
     const double size = plan.px * plan.rows / 16.0;
     const double tiles = (plan.share + 63) / 64;
     // One wave: its atoms, the brackets of its rows per 64 atoms, the start and the store, and, if
     // the waves of a workgroup split the atoms, their meeting in LDS.
-    double wave = plan.share * shape.atom * (compensated ? 1.12 : 1.0);
-    wave += tiles * plan.touched * plan.rows * (compensated ? 0.0115 : 0.0032);
-    wave += 0.064 + size * (compensated ? 0.83 : 0.43);
-    wave += plan.waves > 1 ? size * (compensated ? 0.83 : 0.26) : 0.0;
+    double wave = plan.share * shape.atom * (compensated ? 1.2 : 1.0);
+    wave += tiles * plan.touched * plan.rows * (compensated ? 0.0076 : 0.0086);
+    wave += 0.037 + size * (compensated ? 0.24 : 0.16);
+    wave += plan.waves > 1 ? size * (compensated ? 0.14 : 0.044) : 0.0;
     // Waves per SIMD of the 256 CUs: whole workgroups per CU while they all fit at once; more than
     // that are handed out as others end, with a partial last round.
-    constexpr double kComputeUnits = 256.0;
-    const int slots = compensated ? shape.wavesPerSimdCompensated : shape.wavesPerSimd;
     const double perGroup = plan.waves / 4.0;
-    const double resident = plan.waves < 4 ? slots : std::max(1, slots * 4 / plan.waves) * perGroup;
+    const double resident = PackedGroupsPerUnit(plan, shape, compensated) * perGroup;
     double load = plan.waves < 4 ? std::ceil(plan.workgroups * perGroup / kComputeUnits)
                                  : std::ceil(plan.workgroups / kComputeUnits) * perGroup;
     double busy = load;
     if (load > resident)
     {
         busy = resident;
-        load = plan.workgroups * perGroup / kComputeUnits + 0.97 * std::max(1.0, perGroup);
+        load = plan.workgroups * perGroup / kComputeUnits + 0.66 * std::max(1.0, perGroup);
     }
-    const double rate = 1.0 - (1.0 - shape.alone) / busy;
-    return load * wave / rate + 0.0104 * busy;
+    const double rate = 1.0 - (1.0 - shape.alone) * std::pow(std::max(busy, 1.0), -0.88);
+    return load * wave / rate;
 }
 
 /** Whether a volume of side^3 points runs the wave engine without a configuration: not at multiples of
@@ -128,7 +147,6 @@ inline PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, co
 {
     PackedPlan best;
     double bestTime = std::numeric_limits<double>::max();
-    int bestSlots = 0;
     for (const PackedShape& shape : kPackedShapes)
     {
         for (const int waves : {1, 4, 8, 16})
@@ -146,21 +164,20 @@ inline PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, co
             {
                 continue;
             }
+            // Four-wave workgroups that all start at once stay where the first round put them, unevenly;
+            // eight-wave ones leave a part for CUs that finish early (100^3 x 30,000: 2,882 us against 3,051).
+            if (waves == 4 && atomCount >= 256 && plan.workgroups > 256u
+                && (plan.workgroups + 255u) / 256u <= static_cast<unsigned int>(PackedGroupsPerUnit(plan, shape, compensated)))
+            {
+                continue;
+            }
             const double time = EstimatePacked(plan, shape, compensated);
             if (time < bestTime)
             {
                 bestTime = time;
                 best = plan;
-                bestSlots = compensated ? shape.wavesPerSimdCompensated : shape.wavesPerSimd;
             }
         }
-    }
-    // Four-wave workgroups that all start at once stay where the first round put them, unevenly; eight-wave
-    // ones leave a part for CUs that finish early (100^3 x 30,000: 2,882 us against 3,051).
-    if (best.waves == 4 && atomCount >= 256 && best.workgroups > 256u && best.workgroups <= 256u * static_cast<unsigned int>(bestSlots))
-    {
-        const PackedPlan wider = PlanShape(best.px, best.rows, 8, 1, atomCount, rowLength, rowsTotal, compensated);
-        best = wider.workgroups != 0 ? wider : best;
     }
     return best;
 }
