@@ -186,9 +186,11 @@ int ktt_coulomb_launch_shape(int kind, int grid_size, const char* config, unsign
  * CoulombSum3d kernel's semantics (Examples/CoulombSum3d/CoulombSum3d.cu:1-47) to many systems.
  * host_atoms packs the float4 atoms of system 0, then system 1, ...; atom_counts, grid_sizes
  * and spacings have system_count entries. At most five distinct grid sides per batch; each
- * side is a tile-shape bucket. Config names: BUCKETb_WGX, BUCKETb_PX, BUCKETb_ROWS,
- * BUCKETb_TILE (b = 0..4, buckets in increasing grid side) and GROUPS_PER_CU. The batch owns
- * the device copies of the atoms and one packed output array of all grids. */
+ * side is a tile-shape bucket. Without a configuration the batch runs the wave engine (up to 2 million
+ * 64-lane work items; WAVE_SPLIT sets the waves that split a system's atoms, 1 to 16). Config names of the
+ * persistent bucket kernel: BUCKETb_WGX, BUCKETb_PX, BUCKETb_ROWS, BUCKETb_TILE, BUCKETb_UNROLL (b = 0..4,
+ * buckets in increasing grid side) and GROUPS_PER_CU. The batch owns the device copies of the atoms and one
+ * packed output array of all grids. */
 int ktt_coulomb_batch_create(const float* host_atoms, const int* atom_counts, const int* grid_sizes, const float* spacings,
                              int system_count, const char* config, void** batch);
 int ktt_coulomb_batch_destroy(void* batch);
@@ -202,9 +204,9 @@ int ktt_coulomb_batch_info(void* batch, float** grids, size_t* grid_points, long
 /* Clears all grids of the batch (zero-fill kernel). */
 int ktt_coulomb_batch_zero(void* batch, void* stream);
 
-/* Adds V of every system to its grid: one persistent launch in which workgroups take
- * (system, tile) items from a device-side queue, compensated FP32. use_graph != 0 replays a HIP
- * graph (queue reset + persistent kernel) captured on the first call. */
+/* Adds V of every system to its grid in one launch, compensated: the wave engine's workgroups in the
+ * order of the systems' atoms, or, with buckets set, persistent workgroups that take (system, tile) items
+ * from a device-side queue. use_graph != 0 replays a HIP graph of it captured on the first call. */
 int ktt_coulomb_batch_run(void* batch, int use_graph, void* stream, float* kernel_ms);
 
 /* Baseline: one ktt_coulomb3d launch per system (form KTT_COULOMB_PLAIN or _COMPENSATED), all
@@ -213,7 +215,7 @@ int ktt_coulomb_batch_run_per_system(void* batch, int form, void* stream, float*
 
 /* Tunes the tile shape of every bucket with ktt::Tuner on ComputeApi::HIP (a composite kernel
  * and launcher over the bucket's systems; searcher as in section 4), bucket after bucket, and
- * keeps the winners in the batch. results_file (optional) is a path prefix: the KTT JSON
+ * keeps the winners in the batch, which then runs the bucket kernel. results_file (optional) is a path prefix: the KTT JSON
  * results of bucket b go to <prefix>_bucket<b>.json and the winners to <prefix>_winners.json.
  * best_config (optional) receives the winning shapes as a configuration string. */
 int ktt_coulomb_batch_tune(void* batch, int searcher, int max_configurations_per_bucket, const char* results_file,

@@ -82,6 +82,7 @@ KERNEL_CHECKS = [
     ("NbodySplit.hip", "nbody_split", "BODY_LANES=8,BODIES_PER_THREAD=1"),
     ("NbodyReference.hip", "nbody_kernel_reference", None),
     ("CoulombBatched.hip", "coulombBatchedPersistent", None),
+    ("CoulombBatchPacked.hip", "coulombBatchPacked", None),
     ("CoulombBatched.hip", "coulombBatchedSystem", None),
     ("CoulombBatched.hip", "coulombBatchedReset", None),
 ]

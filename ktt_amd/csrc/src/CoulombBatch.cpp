@@ -16,6 +16,7 @@
 #include "../../../include/ktt_hip.h"
 #include "Common.h"
 #include "CoulombBatchPlan.h"
+#include "CoulombPackedPlan.h"
 #include "CoulombRuntime.h"
 #include "HipEngine.h"
 #include "Json.h"
@@ -89,6 +90,8 @@ public:
     void RunPerSystem(const int form, hipStream_t stream, float* kernelMs);
     void Zero(hipStream_t stream);
     void SetShapes(const std::vector<BucketShape>& shapes);
+    /** Leaves the wave engine for the bucket shapes (before the autotuner works on them). */
+    void UseBuckets();
 
     float* Grids() const { return m_Grids; }
     size_t GridPoints() const { return m_GridPoints; }
@@ -121,6 +124,8 @@ private:
     std::vector<int> m_BucketSides;
     std::vector<BucketShape> m_Shapes;
     std::vector<int> m_Items;   // flattened int4 records
+    bool m_Packed;              // the wave engine (default), or the bucket shapes
+    batch::PackedBatchPlan m_PackedPlan;
     size_t m_ItemCapacity;
     int m_GroupsPerCu;
     int m_PersistentGroups;
@@ -143,6 +148,7 @@ private:
 
 CoulombBatch::CoulombBatch(const float* hostAtoms, const int* atomCounts, const int* gridSizes, const float* spacings,
     const int systemCount, const char* config) :
+    m_Packed(false),
     m_ItemCapacity(0),
     m_GroupsPerCu(4),
     m_PersistentGroups(0),
@@ -225,7 +231,21 @@ CoulombBatch::CoulombBatch(const float* hostAtoms, const int* atomCounts, const 
     m_GridPoints = static_cast<size_t>(gridOffset);
 
     // Item capacity for the configured shapes; the tuner grows it for its own space.
-    m_ItemCapacity = std::max<size_t>(batch::CountWorkItems(m_Systems, m_Shapes), 1);
+    // The wave engine unless the configuration sets the buckets, or its list (one item per 64 lanes)
+    // would be longer than 2 million items (32 MiB).
+    m_Packed = parsed.Has("WAVE_SPLIT")
+        || (parsed.values.empty() && batch::CountPackedItems(m_Systems) <= batch::kMaxPackedItems);
+    if (m_Packed)
+    {
+        const long waves = parsed.Get("WAVE_SPLIT", 0);
+        if (parsed.Has("WAVE_SPLIT") && (waves < 1 || waves > 16))
+        {
+            throw KttException("WAVE_SPLIT must be in [1, 16]");
+        }
+        m_PackedPlan = batch::PlanPackedBatch(m_Systems, static_cast<int>(waves));
+    }
+    const std::vector<int> items = m_Packed ? batch::BuildPackedItems(m_Systems) : BuildItems(m_Shapes);
+    m_ItemCapacity = std::max<size_t>(items.size() / 4, 1);
 
     CheckHipError(hipMalloc(reinterpret_cast<void**>(&m_Atoms), std::max<size_t>(static_cast<size_t>(atomOffset), 1) * 16), "hipMalloc(atoms)");
     CheckHipError(hipMalloc(&m_DeviceSystems, m_Systems.size() * sizeof(HostSystem)), "hipMalloc(systems)");
@@ -247,7 +267,7 @@ CoulombBatch::CoulombBatch(const float* hostAtoms, const int* atomCounts, const 
     CheckHipError(hipGetDeviceProperties(&properties, device), "hipGetDeviceProperties");
     m_PersistentGroups = properties.multiProcessorCount * m_GroupsPerCu;
 
-    UploadItems(BuildItems(m_Shapes));
+    UploadItems(items);
     CompileKernels();
 }
 
@@ -314,6 +334,14 @@ void CoulombBatch::UploadItems(const std::vector<int>& items)
 
 void CoulombBatch::CompileKernels()
 {
+    auto& runtime = CoulombRuntime::Get();
+    if (m_Packed)
+    {
+        m_Persistent = runtime.GetKernel("CoulombBatchPacked.hip", "coulombBatchPacked", {"-DCAP_WIDE=" + std::to_string(m_PackedPlan.caps[0]),
+            "-DCAP_NARROW=" + std::to_string(m_PackedPlan.caps[1]), "-DCAP_SMALL=" + std::to_string(m_PackedPlan.caps[2])});
+        m_Reset = nullptr;
+        return;
+    }
     CoulombConfig defines;
     for (int b = 0; b < kMaxBuckets; ++b)
     {
@@ -325,7 +353,6 @@ void CoulombBatch::CompileKernels()
         defines.Set(prefix + "UNROLL", std::to_string(m_Shapes[b].unroll));
     }
     defines.Set("BATCH_THREADS", std::to_string(kBatchThreads));
-    auto& runtime = CoulombRuntime::Get();
     m_Persistent = runtime.GetKernel("CoulombBatched.hip", "coulombBatchedPersistent", defines.Defines({}));
     m_Reset = runtime.GetKernel("CoulombBatched.hip", "coulombBatchedReset", {});
 }
@@ -338,12 +365,27 @@ void CoulombBatch::SetShapes(const std::vector<BucketShape>& shapes)
     }
     DestroyGraph();
     m_Shapes = shapes;
-    UploadItems(BuildItems(m_Shapes));
+    m_Packed = false;
+    const std::vector<int> items = BuildItems(m_Shapes);
+    EnsureItemCapacity(items.size() / 4);
+    UploadItems(items);
     CompileKernels();
+}
+
+void CoulombBatch::UseBuckets()
+{
+    if (m_Packed)
+    {
+        SetShapes(std::vector<BucketShape>(m_Shapes));
+    }
 }
 
 std::string CoulombBatch::ShapeString() const
 {
+    if (m_Packed)
+    {
+        return "WAVE_SPLIT=" + std::to_string(m_PackedPlan.waves);
+    }
     std::string result;
     for (int b = 0; b < kMaxBuckets; ++b)
     {
@@ -382,6 +424,24 @@ void CoulombBatch::DestroyGraph()
 
 void CoulombBatch::LaunchKernels(hipStream_t stream)
 {
+    const int count = ItemCount();
+    // The kernels read items[0, count): they must all be in the uploaded list.
+    if (count < 0 || static_cast<size_t>(count) * 4 != m_Items.size() || static_cast<size_t>(count) > m_ItemCapacity)
+    {
+        throw KttException("batched work list is inconsistent with its device buffer");
+    }
+    if (m_Packed)
+    {
+        const float* packedAtoms = m_Atoms;
+        const void* packedSystems = m_DeviceSystems;
+        const void* packedItems = m_DeviceItems;
+        float* packedGrids = m_Grids;
+        void* packedArguments[] = {&packedAtoms, &packedSystems, &packedItems, &packedGrids};
+        const unsigned int packedGrid[3] = {static_cast<unsigned int>(count), 1, 1};
+        const unsigned int packedBlock[3] = {static_cast<unsigned int>(m_PackedPlan.waves) * 64, 1, 1};
+        CoulombRuntime::Launch(*m_Persistent, packedGrid, packedBlock, packedArguments, stream, nullptr, m_PackedPlan.ldsBytes);
+        return;
+    }
     unsigned int* counter = m_Counter;
     void* resetArguments[] = {&counter};
     const unsigned int one[3] = {1, 1, 1};
@@ -391,12 +451,7 @@ void CoulombBatch::LaunchKernels(hipStream_t stream)
     const float* atoms = m_Atoms;
     const void* systems = m_DeviceSystems;
     const void* items = m_DeviceItems;
-    int itemCount = ItemCount();
-    // The kernel reads items[0, itemCount): they must all be in the uploaded list.
-    if (itemCount < 0 || static_cast<size_t>(itemCount) * 4 != m_Items.size() || static_cast<size_t>(itemCount) > m_ItemCapacity)
-    {
-        throw KttException("batched work list is inconsistent with its device buffer");
-    }
+    int itemCount = count;
     float* grids = m_Grids;
     void* arguments[] = {&atoms, &systems, &items, &itemCount, &grids, &counter};
     const unsigned int groups = static_cast<unsigned int>(std::max(1, std::min(m_PersistentGroups, std::max(itemCount, 1))));
@@ -735,6 +790,100 @@ std::vector<int> BuildWorkItems(const std::vector<HostSystem>& systems, const st
     return flat;
 }
 
+PackedClass PackedClassOf(const int side)
+{
+    return side >= 64 ? PackedClass{0, 2, 8} : (side >= 32 ? PackedClass{1, 1, 8} : PackedClass{2, 1, 4});
+}
+
+static long PackedBlocks(const HostSystem& system, const PackedClass& shape)
+{
+    const long g = system.gridSize;
+    return ((g + shape.px - 1) / shape.px * ((g * g + shape.rows - 1) / shape.rows) + 63) / 64;
+}
+
+PackedBatchPlan PlanPackedBatch(const std::vector<HostSystem>& systems, const int waves)
+{
+    PackedBatchPlan plan;
+    double work = 0.0;  // wave-atoms
+    double longest = 0.0;
+    long waveFloats = 0;
+    long totalBlocks = 0;
+    for (const auto& system : systems)
+    {
+        const PackedClass shape = PackedClassOf(system.gridSize);
+        const int lanesX = (system.gridSize + shape.px - 1) / shape.px;
+        const int rowGroups = static_cast<int>((static_cast<long>(system.gridSize) * system.gridSize + shape.rows - 1) / shape.rows);
+        int& cap = plan.caps[shape.index];
+        cap = std::max(cap, RowGroupCap(RowGroupsPerWave(lanesX, rowGroups), shape.rows));
+        waveFloats = std::max(waveFloats, 64 * (4 + static_cast<long>(cap) * shape.rows + 4));
+        const long blocks = PackedBlocks(system, shape);
+        totalBlocks += blocks;
+        const double one = system.atomCount * (shape.px * shape.rows / 16.0);
+        work += static_cast<double>(blocks) * one;
+        longest = std::max(longest, one);
+    }
+    if (static_cast<size_t>(totalBlocks) > kMaxPackedItems)
+    {
+        throw KttException("the batch has more than " + std::to_string(kMaxPackedItems) + " work items for the wave engine");
+    }
+    plan.waves = waves;
+    if (waves == 0)
+    {
+        // Four waves per workgroup (128 systems of 32^3 to 128^3: 28.7 ms, 29.4 with eight, whose meeting
+        // and coarser workgroups cost more), unless the longest workgroup, whose waves share their SIMDs with four
+        // others, would outlast twice the batch's share of one SIMD: then more waves split its atoms (40
+        // systems of 24^3: 309 us with 8, 434 with 4).
+        plan.waves = 4;
+        while (plan.waves < 16 && 5.0 * longest / plan.waves > 2.0 * work / 1024.0)
+        {
+            plan.waves *= 2;
+        }
+    }
+    while (waves == 0 && plan.waves > 1 && plan.waves * waveFloats * 4 > kPackedLdsBytes)
+    {
+        plan.waves /= 2;
+    }
+    if (plan.waves * waveFloats * 4 > kPackedLdsBytes)
+    {
+        throw KttException("WAVE_SPLIT=" + std::to_string(plan.waves) + " exceeds the LDS with this batch's grid sides",
+            ExceptionReason::DeviceLimitsExceeded);
+    }
+    plan.ldsBytes = static_cast<unsigned int>(plan.waves * waveFloats * 4);
+    return plan;
+}
+
+size_t CountPackedItems(const std::vector<HostSystem>& systems)
+{
+    size_t total = 0;
+    for (const auto& system : systems)
+    {
+        total += static_cast<size_t>(PackedBlocks(system, PackedClassOf(system.gridSize)));
+    }
+    return total;
+}
+
+std::vector<int> BuildPackedItems(const std::vector<HostSystem>& systems)
+{
+    std::vector<size_t> order(systems.size());
+    std::iota(order.begin(), order.end(), size_t(0));
+    std::stable_sort(order.begin(), order.end(), [&systems](const size_t a, const size_t b)
+    {
+        return systems[a].atomCount > systems[b].atomCount;
+    });
+    std::vector<int> flat;
+    flat.reserve(4 * CountPackedItems(systems));
+    for (const size_t s : order)
+    {
+        const long blocks = PackedBlocks(systems[s], PackedClassOf(systems[s].gridSize));
+        for (long b = 0; b < blocks; ++b)
+        {
+            const int record[4] = {static_cast<int>(s), static_cast<int>(b), 0, 0};
+            flat.insert(flat.end(), record, record + 4);
+        }
+    }
+    return flat;
+}
+
 void CheckItemCapacity(const std::vector<int>& flat, const size_t capacity)
 {
     if (flat.size() % 4 != 0)
@@ -853,6 +1002,7 @@ int ktt_coulomb_batch_tune(void* batch, int searcher, int maxConfigurationsPerBu
         return SetLastError("batch is null");
     }
     auto& value = *static_cast<CoulombBatch*>(batch);
+    value.UseBuckets();
     const std::string prefix = resultsFile != nullptr ? resultsFile : "";
     std::vector<BucketShape> shapes = value.Shapes();
     JsonValue summary = JsonValue::MakeObject();

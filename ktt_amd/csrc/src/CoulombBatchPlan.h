@@ -51,6 +51,37 @@ size_t CountWorkItems(const std::vector<HostSystem>& systems, const std::vector<
  *  system and tile order. Its length is 4 x CountWorkItems. */
 std::vector<int> BuildWorkItems(const std::vector<HostSystem>& systems, const std::vector<BucketShape>& shapes);
 
+/** Points per lane (px x rows) of a system on the wave engine, by its side: the classes of
+ *  kernels/CoulombBatchPacked.hip. */
+struct PackedClass
+{
+    int index;  // 0: side >= 64, 1: 32 to 63, 2: below
+    int px;
+    int rows;
+};
+PackedClass PackedClassOf(int side);
+
+/** Longest work list the wave engine takes: 1,024-thread workgroups of a launch of 2^31 threads. */
+constexpr size_t kMaxPackedItems = 0x7fffffff / 1024;
+
+/** Number of 64-lane blocks of the systems. */
+size_t CountPackedItems(const std::vector<HostSystem>& systems);
+
+/** What a batch on the wave engine compiles and launches. */
+struct PackedBatchPlan
+{
+    int caps[3] = {0, 0, 0};  // row groups a wave touches at most in each class, 0 without such systems
+    int waves = 4;            // waves per workgroup, which split a system's atoms
+    unsigned int ldsBytes = 0;
+};
+
+/** waves 0: by the batch's work. Throws KttException if the waves' brackets exceed the LDS. */
+PackedBatchPlan PlanPackedBatch(const std::vector<HostSystem>& systems, int waves);
+
+/** The wave engine's work list as flattened int4 records (system, 64-lane block, 0, 0), systems with
+ *  the most atoms first. */
+std::vector<int> BuildPackedItems(const std::vector<HostSystem>& systems);
+
 /** Throws KttException unless flat holds whole int4 records and at most capacity of them. */
 void CheckItemCapacity(const std::vector<int>& flat, size_t capacity);
 

@@ -590,6 +590,49 @@ void TestBatchWorkList()
     CHECK(ragged);
 }
 
+/** A batch's work list on the wave engine: every 64-lane block of every system once, systems with the most
+ *  atoms first; the caps hold what the systems of each class touch, and a long system in a small batch gets
+ *  more waves. */
+void TestPackedBatch()
+{
+    using namespace ktt::batch;
+    std::vector<HostSystem> systems;
+    const int sides[] = {5, 24, 31, 32, 47, 63, 64, 99, 128};
+    for (int s = 0; s < 9; ++s)
+    {
+        systems.push_back({0, 50 * (1 + s * 5 % 9), sides[s], 0, 0.5f, 0, 0});
+    }
+    systems.push_back({0, 0, 40, 0, 0.5f, 0, 0});
+    const std::vector<int> flat = BuildPackedItems(systems);
+    CHECK(flat.size() == 4 * CountPackedItems(systems));
+    std::set<std::pair<int, int>> seen;
+    bool ordered = true;
+    int previous = 1 << 30;
+    for (size_t k = 0; k < flat.size(); k += 4)
+    {
+        ordered = ordered && systems[static_cast<size_t>(flat[k])].atomCount <= previous;
+        previous = systems[static_cast<size_t>(flat[k])].atomCount;
+        seen.insert({flat[k], flat[k + 1]});
+    }
+    CHECK(ordered);
+    CHECK(seen.size() == flat.size() / 4);
+    size_t lanesCovered = 0;
+    const PackedBatchPlan plan = PlanPackedBatch(systems, 0);
+    for (const auto& system : systems)
+    {
+        const PackedClass shape = PackedClassOf(system.gridSize);
+        const int lanesX = (system.gridSize + shape.px - 1) / shape.px;
+        const int rowGroups = (system.gridSize * system.gridSize + shape.rows - 1) / shape.rows;
+        lanesCovered += static_cast<size_t>((lanesX * rowGroups + 63) / 64);
+        CHECK(ktt::RowGroupsPerWave(lanesX, rowGroups) <= plan.caps[shape.index]);
+    }
+    CHECK(lanesCovered == seen.size());
+    CHECK(plan.ldsBytes <= 160u * 1024u);
+    CHECK(PlanPackedBatch({{0, 5000, 64, 0, 0.5f, 0, 0}}, 0).waves == 16);
+    CHECK(PlanPackedBatch(std::vector<HostSystem>(200, {0, 2000, 128, 0, 0.5f, 0, 0}), 0).waves == 4);
+    CHECK(PlanPackedBatch({{0, 10, 6, 0, 0.5f, 0, 0}}, 0).ldsBytes <= 160u * 1024u);
+}
+
 /** The wave engine's launch plans over every grid side the default takes them for at small sizes, and
  *  ragged slices: the plan exists and fits the LDS, the waves' atom shares cover the atoms once in whole
  *  unrolled steps, every lane's points lie in one row group, and no wave touches more row groups than
@@ -669,6 +712,7 @@ int main(int argc, char** argv)
     TestProfileSearcherAnalysis();
     TestBatchWorkList();
     TestPackedPlan();
+    TestPackedBatch();
     std::printf("%d checks, %d failures\n", g_Checks, g_Failures);
     return g_Failures == 0 ? 0 : 1;
 }

@@ -143,3 +143,31 @@ def test_no_alloc_entry_point_takes_the_same_shapes(capi, grid, count):
     assert oracle.normalised_error(out[index], values, norms)[0] <= BARS[1]
     other = run_guarded(capi, atoms, spacing, grid, 1, None)
     assert (np.abs(out[index].astype(np.float64) - other[index]) / norms).max() <= BARS[1]
+
+
+@pytest.mark.parametrize("config", [None, "WAVE_SPLIT=1", "WAVE_SPLIT=5"])
+@pytest.mark.parametrize("sides", [(3, 24, 31, 33, 66), (32, 48, 63, 64, 128), (7,)])
+def test_batches(capi, sides, config):
+    """Batches whose sides fall into each class of points per lane, ragged and not, with no atoms in one
+    system, against FP64 at sampled points; eager and graph launches agree bit for bit."""
+    systems = []
+    for k, side in enumerate(sides * 2):
+        count = (0, 1, 65, 300, 701)[k % 5] if k else 513
+        systems.append(workloads.BatchSystem(workloads.uniform_atoms(300 + k, count, box=max(side, 4) * 0.49), side, 0.49))
+    batch = capi.Batch(systems, config=config)
+    print("batch", sides, config, batch.info()["items"], batch.info()["shapes"], flush=True)
+    batch.zero()
+    batch.run(use_graph=False)
+    grids = batch.grids()
+    for k, (system, grid) in enumerate(zip(systems, grids)):
+        if system.atoms.shape[0] == 0:
+            assert (grid == 0.0).all()
+            continue
+        points = workloads.sample_points(400 + k, 500, system.grid)
+        values, norms = oracle.points_f64(system.atoms, system.spacing, points)
+        assert oracle.normalised_error(grid[points[:, 2], points[:, 1], points[:, 0]], values, norms)[0] <= BARS[1]
+    for _ in range(2):
+        batch.zero()
+        batch.run(use_graph=True)
+        for first, again in zip(grids, batch.grids()):
+            np.testing.assert_array_equal(first, again)
