@@ -469,7 +469,9 @@ void CoulombBatch::Run(hipStream_t stream, const bool useGraph, float* kernelMs)
         CheckHipError(hipEventCreate(&start), "hipEventCreate");
         CheckHipError(hipEventCreate(&end), "hipEventCreate");
     }
-    if (useGraph)
+    // The wave engine is a single launch: a graph of it would only cost more (17 us of host time to
+    // replay against 3.3 to launch).
+    if (useGraph && !m_Packed)
     {
         if (m_GraphExec == nullptr || m_GraphStream != stream)
         {
