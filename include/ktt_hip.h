@@ -147,12 +147,14 @@ int ktt_coulomb2d(const float* atoms, int n_atoms, float spacing, int grid_x, in
 int ktt_coulomb2d_reference(const float* atoms, int n_atoms, float spacing, int grid_x, int grid_y,
                             float* energy_grid, void* stream, float* kernel_ms);
 
-/* CoulombSum3dIterative with the reference launcher's semantics
- * (Examples/CoulombSum3dIterative/CoulombSum3dIterative.cpp:146-184): for every slice z the
- * host computes dz^2 = (h*z - Z_i)^2 in FP32 for all atoms, uploads the atom records with .z
- * replaced, and launches the slice kernel (CoulombSum3dIterative.cl:35) with zIndex = z.
- * host_atoms: float4[n_atoms] in host memory with the real z. wall_ms receives the host
- * time of the whole loop, kernel_ms the sum of the slice kernels' event times. */
+/* CoulombSum3dIterative from host atoms, with the reference launcher's arithmetic
+ * (Examples/CoulombSum3dIterative/CoulombSum3dIterative.cpp:146-184): slice z uses dz^2 =
+ * (h*z - Z_i)^2 in FP32. host_atoms: float4[n_atoms] in host memory with the real z. With a
+ * configuration, as the reference launcher does it: for every slice the host computes dz^2 of all atoms,
+ * uploads the atom records with .z replaced, and launches the slice kernel (CoulombSum3dIterative.cl:35)
+ * with zIndex = z. Without one, the atoms are uploaded once and one launch covers all slices, forming
+ * dz^2 on the device. wall_ms receives the host time of the whole call's work, kernel_ms the (sum of the)
+ * kernels' event times; the call returns when they have ended. */
 int ktt_coulomb3d_iterative(const float* host_atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
                             const char* config, void* stream, float* kernel_ms, float* wall_ms);
 
@@ -165,7 +167,7 @@ int ktt_coulomb3d_iterative_reference(const float* atoms, int n_atoms, float spa
                                       void* stream, float* kernel_ms);
 
 /* Fused slice loop: dz^2 is formed on the device (atoms with their real z on the device). Without a
- * configuration all slices run as the planes of one volume launch (ktt_coulomb3d, plain form); with
+ * configuration all slices run as the planes of one volume launch of the wave engine (plain form); with
  * one, the slice kernel is launched per slice, no host work between launches. Either way grid_size
  * must be tiled by the slice kernel's workgroups, as for ktt_coulomb2d. */
 int ktt_coulomb3d_slices(const float* atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
@@ -206,7 +208,8 @@ int ktt_coulomb_batch_zero(void* batch, void* stream);
 
 /* Adds V of every system to its grid in one launch, compensated: the wave engine's workgroups in the
  * order of the systems' atoms, or, with buckets set, persistent workgroups that take (system, tile) items
- * from a device-side queue. use_graph != 0 replays a HIP graph of it captured on the first call. */
+ * from a device-side queue; use_graph != 0 then replays a HIP graph (queue reset + persistent kernel)
+ * captured on the first call. The wave engine is one launch with or without it. */
 int ktt_coulomb_batch_run(void* batch, int use_graph, void* stream, float* kernel_ms);
 
 /* Baseline: one ktt_coulomb3d launch per system (form KTT_COULOMB_PLAIN or _COMPENSATED), all

@@ -1170,6 +1170,22 @@ int ktt_coulomb3d_iterative_reference(const float* atoms, int atomCount, float s
     KTT_C_CATCH
 }
 
+// Whether the slices of a grid run as the planes of one volume launch: without a configuration, as long
+// as a launch holds them. The same terms, without a launch's ramp and tail per slice, on a chip that one
+// slice does not fill, and without the FP32 atomics of the slices' atom blocks (128^3 x 8,192: 2,075 us in 128
+// launches, 1,552 in one). On the wave engine at every side: its 64-atom partial sums keep the slices'
+// precision, which the workgroup shapes' running sums would not (256^3 x 2,480: error against 64 bits
+// 3.5e-7 in slices, 1.2e-6 by CoulombSum3d.hip's plain form).
+static bool SlicesInOneLaunch(const int atomCount, const int gridSize, const char* config, PackedPlan& plan)
+{
+    if (!CoulombConfig::Parse(config, CoulombConfig()).values.empty())
+    {
+        return false;
+    }
+    plan = ChoosePackedPlan(atomCount, gridSize, static_cast<long>(gridSize) * gridSize, false);
+    return plan.workgroups != 0;
+}
+
 static void CheckSliceGrid(const CoulombShape& shape, const CoulombConfig& parsed, const int gridSize)
 {
     const long spanX = static_cast<long>(shape.block[0]) * parsed.Get("POINTS_X", 4);
@@ -1195,8 +1211,48 @@ int ktt_coulomb3d_iterative(const float* hostAtoms, int atomCount, float spacing
     const long atomBlocks = EffectiveAtomBlocks(parsed, atomCount);
     const CoulombShape shape = CoulombRuntime::RowShape(parsed, gridSize, gridSize, atomBlocks);
     CheckSliceGrid(shape, parsed, gridSize);
-    auto kernel = runtime.GetKernel("CoulombSum3dIterative.hip", "directCoulombSum", parsed.Defines(kLaunchOnly));
     hipStream_t hipStream = static_cast<hipStream_t>(stream);
+    // The atoms' device copy is one buffer per process: calls from several threads take turns.
+    static std::mutex atomsMutex;
+    const std::lock_guard<std::mutex> lock(atomsMutex);
+    PackedPlan packed;
+    if (SlicesInOneLaunch(atomCount, gridSize, config, packed))
+    {
+        // By default the atoms go up once and one volume launch forms dz^2 on the device, with the host's
+        // FP32 roundings (coordinate, difference, square). The per-slice scheme below spent most of its time
+        // beside the kernels on small grids: a pinned buffer, streams and events made for each call, and
+        // per slice the host's dz^2, an upload, four event calls and a launch that does not fill the chip
+        // (128^3 x 2,000: 3,737 us, 390 now).
+        const auto begin = std::chrono::steady_clock::now();
+        const size_t atomBytes = static_cast<size_t>(atomCount) * 4 * sizeof(float);
+        float* deviceAtoms = static_cast<float*>(runtime.GetScratch("iterative.atoms", std::max<size_t>(atomBytes, 16)));
+        if (atomBytes > 0)
+        {
+            CheckHipError(hipMemcpyAsync(deviceAtoms, hostAtoms, atomBytes, hipMemcpyHostToDevice, hipStream), "hipMemcpyAsync");
+        }
+        float volumeMs = 0.0f;
+        try
+        {
+            LaunchPacked(packed, deviceAtoms, atomCount, spacing, gridSize, gridSize * gridSize, energyGrid, false, false, hipStream,
+                &volumeMs);
+        }
+        catch (...)
+        {
+            IgnoreHipError(hipStreamSynchronize(hipStream));  // the upload reads the caller's memory
+            throw;
+        }
+        const auto finish = std::chrono::steady_clock::now();
+        if (kernelMs != nullptr)
+        {
+            *kernelMs = volumeMs;
+        }
+        if (wallMs != nullptr)
+        {
+            *wallMs = std::chrono::duration<float, std::milli>(finish - begin).count();
+        }
+        return 0;
+    }
+    auto kernel = runtime.GetKernel("CoulombSum3dIterative.hip", "directCoulombSum", parsed.Defines(kLaunchOnly));
 
     // Per slice, as the reference launcher: dz^2 of every atom in FP32 on the host
     // (CoulombSum3dIterative.cpp:160-168), an upload of the whole atom array and a launch
@@ -1318,13 +1374,11 @@ int ktt_coulomb3d_slices(const float* atoms, int atomCount, float spacing, int g
     const long atomBlocks = EffectiveAtomBlocks(parsed, atomCount);
     const CoulombShape shape = CoulombRuntime::RowShape(parsed, gridSize, gridSize, atomBlocks);
     CheckSliceGrid(shape, parsed, gridSize);
-    if (CoulombConfig::Parse(config, CoulombConfig()).values.empty())
+    PackedPlan packed;
+    if (SlicesInOneLaunch(atomCount, gridSize, config, packed))
     {
-        // By default the slices are the planes of one volume launch: the same terms, without a launch's
-        // ramp and tail per slice, on a chip that one slice does not fill, and without the FP32 atomics
-        // of the slices' atom blocks.
-        LaunchVolume(atoms, atomCount, spacing, gridSize, energyGrid, KTT_COULOMB_PLAIN, nullptr, static_cast<hipStream_t>(stream),
-            kernelMs);
+        LaunchPacked(packed, atoms, atomCount, spacing, gridSize, gridSize * gridSize, energyGrid, false, false,
+            static_cast<hipStream_t>(stream), kernelMs);
         return 0;
     }
     auto kernel = runtime.GetKernel("CoulombSum3dIterative.hip", "directCoulombSumSlice", parsed.Defines(kLaunchOnly));
