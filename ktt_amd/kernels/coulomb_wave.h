@@ -68,14 +68,21 @@ struct WaveEngine
     static constexpr int Tile = 64;
     static constexpr int Unroll = 8;
     static constexpr int Points = PX * ROWS;
+    // Atoms per issue phase. A change of phase costs a few cycles, which the plain 1 x 4 block's four
+    // v_rsq_f32 feel: two atoms at a time take 128^3 x 4,000 from 797 to 779 us and 32^3 x 5,000 from 41.0
+    // to 39.0. The larger blocks, and the compensated ones with their per-tile landing, lose as much
+    // to the registers of the second atom as they gain (1 x 8 758 -> 758, compensated 1 x 4 833 -> 860).
+    static constexpr int Phase = !COMP && Points <= 4 ? 2 : 1;
+    static_assert(Unroll % Phase == 0, "whole phases per unrolled step");
     static constexpr int AtomFloats = COMP ? 4 : 2;
     // Row brackets of one atom, padded so that the 16-byte stores of 8 lanes hit all 64 banks once.
     static constexpr int RowStride = CAP * ROWS + 4;
     static constexpr int WaveFloats = Tile * (AtomFloats + RowStride);
-    // Values per lane that fit a wave's LDS when the waves of a split meet.
-    static constexpr int MeetWhole = WaveFloats * 4 / (64 * static_cast<int>(sizeof(Sum)));
-    static constexpr int MeetValues = MeetWhole < Points ? MeetWhole : Points;
+    // Rows of a lane's points that fit a wave's LDS when the waves of a split meet.
+    static constexpr int MeetWhole = WaveFloats * 4 / (64 * PX * static_cast<int>(sizeof(Sum)));
+    static constexpr int MeetRows = MeetWhole < ROWS ? MeetWhole : ROWS;
 
+    static_assert(MeetRows >= 1, "the waves meet at least one row at a time");
     static_assert(ROWS % 4 == 0, "row brackets are stored four at a time");
 
     // Position of this lane's points: x0 = xLane * PX, rows row0 .. row0 + ROWS - 1.
@@ -85,6 +92,7 @@ struct WaveEngine
     int firstGroup;  // the wave's first row group and the number it touches (uniform)
     int groups;
     bool valid;
+    bool whole;  // every lane of the wave has points (uniform)
 
     float part[ROWS][PX];
     Sum sum[ROWS][PX];
@@ -96,6 +104,7 @@ struct WaveEngine
         const unsigned int first = waveBlock * 64u;
         const unsigned int mine = first + lane;
         valid = mine < total;
+        whole = total >= 64u && first <= total - 64u;
         const unsigned int index = valid ? mine : total - 1u;
         rowGroup = static_cast<int>(index / static_cast<unsigned int>(lanesX));
         xLane = static_cast<int>(index - static_cast<unsigned int>(rowGroup) * lanesX);
@@ -204,17 +213,22 @@ struct WaveEngine
         }
         float hV = h;  // in a VGPR: an SGPR operand would keep the FMA from pairing
         asm volatile("" : "+v"(hV));
-        float rr[ROWS][PX];  // r^2 of the atom in flight, then its r^-1
+        float rr[Phase][ROWS][PX];  // r^2 of the atoms in flight, then their r^-1
+        float qPrev[Phase];
 #pragma unroll
-        for (int k = 0; k < ROWS; ++k)
+        for (int p = 0; p < Phase; ++p)
         {
+            qPrev[p] = 0.0f;
 #pragma unroll
-            for (int i = 0; i < PX; ++i)
+            for (int k = 0; k < ROWS; ++k)
             {
-                rr[k][i] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < PX; ++i)
+                {
+                    rr[p][k][i] = 0.0f;
+                }
             }
         }
-        float qPrev = 0.0f;
         float4 next;
         if constexpr (!COMP)
         {
@@ -238,63 +252,71 @@ struct WaveEngine
             for (int a = 0; a < count; a += Unroll)
             {
 #pragma unroll
-                for (int u = 0; u < Unroll; ++u)
+                for (int u = 0; u < Unroll; u += Phase)
                 {
                     __builtin_amdgcn_sched_barrier(0);
                     __builtin_amdgcn_s_setprio(0);
-                    float dx[PX];
-                    float q;
-                    if constexpr (COMP)
-                    {
-                        const float4 v = *reinterpret_cast<const float4*>(lds + (a + u) * 4);
-                        dx[0] = fmaf(hV, x[0] - v.x, v.y);
 #pragma unroll
-                        for (int i = 1; i < PX; ++i)
+                    for (int p = 0; p < Phase; ++p)
+                    {
+                        float dx[PX];
+                        float q;
+                        if constexpr (COMP)
                         {
-                            dx[i] = dx[i - 1] + hV;
-                        }
-                        q = v.z;
-                    }
-                    else
-                    {
-                        const float2 v = *reinterpret_cast<const float2*>(lds + (a + u) * 2);
+                            const float4 v = *reinterpret_cast<const float4*>(lds + (a + u + p) * 4);
+                            dx[0] = fmaf(hV, x[0] - v.x, v.y);
 #pragma unroll
-                        for (int i = 0; i < PX; ++i)
+                            for (int i = 1; i < PX; ++i)
+                            {
+                                dx[i] = dx[i - 1] + hV;
+                            }
+                            q = v.z;
+                        }
+                        else
                         {
-                            dx[i] = x[i] - v.x;
+                            const float2 v = *reinterpret_cast<const float2*>(lds + (a + u + p) * 2);
+#pragma unroll
+                            for (int i = 0; i < PX; ++i)
+                            {
+                                dx[i] = x[i] - v.x;
+                            }
+                            q = v.y;
                         }
-                        q = v.y;
-                    }
-                    float b[ROWS];
+                        float b[ROWS];
 #pragma unroll
-                    for (int k = 0; k < ROWS; k += 4)
-                    {
-                        const float4 v = *reinterpret_cast<const float4*>(sB + (a + u) * RowStride + k);
-                        b[k] = v.x;
-                        b[k + 1] = v.y;
-                        b[k + 2] = v.z;
-                        b[k + 3] = v.w;
-                    }
-#pragma unroll
-                    for (int k = 0; k < ROWS; ++k)
-                    {
-#pragma unroll
-                        for (int i = 0; i < PX; ++i)
+                        for (int k = 0; k < ROWS; k += 4)
                         {
-                            part[k][i] = fmaf(qPrev, rr[k][i], part[k][i]);
-                            rr[k][i] = fmaf(dx[i], dx[i], b[k]);
+                            const float4 v = *reinterpret_cast<const float4*>(sB + (a + u + p) * RowStride + k);
+                            b[k] = v.x;
+                            b[k + 1] = v.y;
+                            b[k + 2] = v.z;
+                            b[k + 3] = v.w;
                         }
+#pragma unroll
+                        for (int k = 0; k < ROWS; ++k)
+                        {
+#pragma unroll
+                            for (int i = 0; i < PX; ++i)
+                            {
+                                part[k][i] = fmaf(qPrev[p], rr[p][k][i], part[k][i]);
+                                rr[p][k][i] = fmaf(dx[i], dx[i], b[k]);
+                            }
+                        }
+                        qPrev[p] = q;
                     }
-                    qPrev = q;
                     __builtin_amdgcn_sched_barrier(0);
                     __builtin_amdgcn_s_setprio(3);
 #pragma unroll
-                    for (int k = 0; k < ROWS; ++k)
+                    for (int p = 0; p < Phase; ++p)
                     {
 #pragma unroll
-                        for (int i = 0; i < PX; ++i)
+                        for (int k = 0; k < ROWS; ++k)
                         {
-                            rr[k][i] = __builtin_amdgcn_rsqf(rr[k][i]);
+#pragma unroll
+                            for (int i = 0; i < PX; ++i)
+                            {
+                                rr[p][k][i] = __builtin_amdgcn_rsqf(rr[p][k][i]);
+                            }
                         }
                     }
                 }
@@ -306,7 +328,6 @@ struct WaveEngine
                 // Land the atom in flight: its 16 registers are free while the next tile is staged,
                 // which keeps the kernel at 5 waves per SIMD.
                 land(qPrev, rr);
-                qPrev = 0.0f;
             }
             fold();
         }
@@ -317,18 +338,23 @@ struct WaveEngine
         fold();
     }
 
-    // part += q r^-1 of the atom in flight.
-    __device__ __forceinline__ void land(const float q, float (&rr)[ROWS][PX])
+    // part += q r^-1 of the atoms in flight, which are then none.
+    __device__ __forceinline__ void land(float (&q)[Phase], float (&rr)[Phase][ROWS][PX])
     {
 #pragma unroll
-        for (int k = 0; k < ROWS; ++k)
+        for (int p = 0; p < Phase; ++p)
         {
 #pragma unroll
-            for (int i = 0; i < PX; ++i)
+            for (int k = 0; k < ROWS; ++k)
             {
-                part[k][i] = fmaf(q, rr[k][i], part[k][i]);
-                rr[k][i] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < PX; ++i)
+                {
+                    part[k][i] = fmaf(q[p], rr[p][k][i], part[k][i]);
+                    rr[p][k][i] = 0.0f;
+                }
             }
+            q[p] = 0.0f;
         }
     }
 
@@ -352,59 +378,116 @@ struct WaveEngine
         }
     }
 
-    // grid += total at point v. atomic: workgroups of other atom blocks add to the same point.
-    __device__ __forceinline__ void add(float* grid, const int v, const int rowLength, const int rowsTotal, const Sum total,
-        const bool atomic) const
+    // grid += v over row k of this lane's points. inside: the wave's points are all in the grid (uniform),
+    // pairs: and two x points may be read and written at once. atomic: other workgroups add to the same points.
+    __device__ __forceinline__ void addRow(float* out, const int k, const Sum (&v)[PX], const int rowLength, const int rowsTotal,
+        const bool inside, const bool pairs, const bool atomic) const
     {
-        const int x = xLane * PX + v % PX;
-        const int row = rowGroup * ROWS + v / PX;
-        if (valid && x < rowLength && row < rowsTotal)
+        float* row = out + static_cast<size_t>(k) * rowLength;
+        if (!COMP && atomic)
         {
-            float* out = grid + static_cast<size_t>(row) * rowLength + x;
-            if (!COMP && atomic)
+#pragma unroll
+            for (int i = 0; i < PX; ++i)
             {
-                unsafeAtomicAdd(out, static_cast<float>(total));
+                if (inside || (valid && xLane * PX + i < rowLength && rowGroup * ROWS + k < rowsTotal))
+                {
+                    unsafeAtomicAdd(row + i, static_cast<float>(v[i]));
+                }
             }
-            else
+            return;
+        }
+        if constexpr (PX == 2)
+        {
+            if (pairs)
             {
-                *out = static_cast<float>(static_cast<Sum>(*out) + total);
+                float2 o = *reinterpret_cast<float2*>(row);
+                o.x = static_cast<float>(static_cast<Sum>(o.x) + v[0]);
+                o.y = static_cast<float>(static_cast<Sum>(o.y) + v[1]);
+                *reinterpret_cast<float2*>(row) = o;
+                return;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < PX; ++i)
+        {
+            if (inside || (valid && xLane * PX + i < rowLength && rowGroup * ROWS + k < rowsTotal))
+            {
+                row[i] = static_cast<float>(static_cast<Sum>(row[i]) + v[i]);
             }
         }
     }
 
     // grid += the sum over the workgroup's waves, each of which holds the same points' sums over its
-    // own atoms. shared: waves * WaveFloats floats.
+    // own atoms. shared: waves * WaveFloats floats. A wave whose points are all inside the grid stores
+    // without a check per point, which a launch of few atoms feels (256^3 x 64: 16 read-modify-writes of
+    // some 20 instructions each beside 64 atoms of 67).
     __device__ __forceinline__ void store(float* shared, const int waves, const int wave, float* grid, const int rowLength,
         const int rowsTotal, const bool atomic) const
     {
+        float* out = grid + static_cast<size_t>(rowGroup) * ROWS * rowLength + xLane * PX;
+        const bool inside = whole && rowLength % PX == 0 && (firstGroup + groups) * ROWS <= rowsTotal;
+        const bool pairs = inside && rowLength % 2 == 0 && (reinterpret_cast<size_t>(grid) & 7u) == 0;
         if (waves == 1)
         {
-#pragma unroll
-            for (int v = 0; v < Points; ++v)
+            if constexpr (PX == 2)
             {
-                add(grid, v, rowLength, rowsTotal, sum[v / PX][v % PX], atomic);
+                if (pairs && !atomic)
+                {
+                    float2 o[ROWS];
+#pragma unroll
+                    for (int k = 0; k < ROWS; ++k)
+                    {
+                        o[k] = *reinterpret_cast<float2*>(out + static_cast<size_t>(k) * rowLength);
+                    }
+#pragma unroll
+                    for (int k = 0; k < ROWS; ++k)
+                    {
+                        o[k].x = static_cast<float>(static_cast<Sum>(o[k].x) + sum[k][0]);
+                        o[k].y = static_cast<float>(static_cast<Sum>(o[k].y) + sum[k][1]);
+                        *reinterpret_cast<float2*>(out + static_cast<size_t>(k) * rowLength) = o[k];
+                    }
+                    return;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < ROWS; ++k)
+            {
+                addRow(out, k, sum[k], rowLength, rowsTotal, inside, pairs, atomic);
             }
             return;
         }
         Sum* meet = reinterpret_cast<Sum*>(shared);
 #pragma unroll
-        for (int first = 0; first < Points; first += MeetValues)
+        for (int first = 0; first < ROWS; first += MeetRows)
         {
             __syncthreads();
 #pragma unroll
-            for (int v = first; v < first + MeetValues && v < Points; ++v)
+            for (int k = first; k < first + MeetRows && k < ROWS; ++k)
             {
-                meet[(wave * MeetValues + v - first) * 64 + lane] = sum[v / PX][v % PX];
+#pragma unroll
+                for (int i = 0; i < PX; ++i)
+                {
+                    meet[((wave * MeetRows + k - first) * PX + i) * 64 + lane] = sum[k][i];
+                }
             }
             __syncthreads();
-            for (int v = first + wave; v < first + MeetValues && v < Points; v += waves)
+            for (int k = first + wave; k < first + MeetRows && k < ROWS; k += waves)
             {
-                Sum total = meet[(v - first) * 64 + lane];
+                Sum total[PX];
+#pragma unroll
+                for (int i = 0; i < PX; ++i)
+                {
+                    total[i] = meet[((k - first) * PX + i) * 64 + lane];
+                }
                 for (int w = 1; w < waves; ++w)
                 {
-                    total += meet[(w * MeetValues + v - first) * 64 + lane];
+#pragma unroll
+                    for (int i = 0; i < PX; ++i)
+                    {
+                        total[i] += meet[((w * MeetRows + k - first) * PX + i) * 64 + lane];
+                    }
                 }
-                add(grid, v, rowLength, rowsTotal, total, atomic);
+                addRow(out, k, total, rowLength, rowsTotal, inside, pairs, atomic);
             }
         }
     }
