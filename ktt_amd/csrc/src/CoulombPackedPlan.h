@@ -90,11 +90,13 @@ struct PackedShape
     int px;
     int rows;
     double atom;      // us a SIMD takes per wave and atom with enough waves to hide latency
+    double compensated; // what the compensated form's offsets and sums multiply it by
     double alone;     // share of that rate that one wave per SIMD reaches
     int wavesPerSimd; // at the kernel's registers, plain and compensated
     int wavesPerSimdCompensated;
 };
-constexpr PackedShape kPackedShapes[] = {{2, 8, 0.0785, 0.58, 6, 5}, {1, 8, 0.0413, 0.41, 7, 7}, {1, 4, 0.0204, 0.24, 8, 8}};
+constexpr PackedShape kPackedShapes[] = {{2, 8, 0.071, 1.035, 0.49, 6, 5}, {1, 8, 0.0376, 1.0, 0.36, 7, 7},
+    {1, 4, 0.0192, 1.124, 0.41, 8, 8}};
 
 // Workgroups a CU holds at once, by registers and LDS.
 inline int PackedGroupsPerUnit(const PackedPlan& plan, const PackedShape& shape, const bool compensated)
@@ -103,10 +105,10 @@ inline int PackedGroupsPerUnit(const PackedPlan& plan, const PackedShape& shape,
     return std::max(1, std::min(slots * 4 / plan.waves, static_cast<int>(kPackedLdsBytes / plan.ldsBytes)));
 }
 
-// Estimated time of a plan in us beyond the launch itself. The constants are a fit to 26 grids of 24^3 to
-// 330^3 points with 64 to 20,000 atoms, both forms, each timed on MI355X at every shape and 1, 4, 8 and
-// 16 waves: the shape it picks is within 1% of the fastest on average (at worst 8%), while any one
-// shape for all is several times slower somewhere.
+// Estimated time of a plan in us beyond the launch itself. The constants are a fit to 27 grids of 24^3 to
+// 320^3 points with 64 to 20,000 atoms, both forms, each timed on MI355X at every shape and 4, 8 and 16
+// waves (1 too for 64 atoms): the shape it picks is within 1.0% of the fastest on average (at worst
+// 7%), while any one shape for all is several times slower somewhere.
 inline double EstimatePacked(const PackedPlan& plan, const PackedShape& shape, const bool compensated)
 {
     constexpr double kComputeUnits = 256.0;
@@ -114,10 +116,10 @@ inline double EstimatePacked(const PackedPlan& plan, const PackedShape& shape, c
     const double tiles = (plan.share + 63) / 64;
     // One wave: its atoms, the brackets of its rows per 64 atoms, the start and the store, and, if
     // the waves of a workgroup split the atoms, their meeting in LDS.
-    double wave = plan.share * shape.atom * (compensated ? 1.2 : 1.0);
-    wave += tiles * plan.touched * plan.rows * (compensated ? 0.0076 : 0.0086);
-    wave += 0.037 + size * (compensated ? 0.24 : 0.16);
-    wave += plan.waves > 1 ? size * (compensated ? 0.14 : 0.044) : 0.0;
+    double wave = plan.share * shape.atom * (compensated ? shape.compensated : 1.0);
+    wave += tiles * plan.touched * plan.rows * (compensated ? 0.0054 : 0.0085);
+    wave += 0.07 + size * (compensated ? 0.51 : 0.24);
+    wave += plan.waves > 1 ? size * (compensated ? 0.044 : 0.012) : 0.0;
     // Waves per SIMD of the 256 CUs: whole workgroups per CU while they all fit at once; more than
     // that are handed out as others end, with a partial last round.
     const double perGroup = plan.waves / 4.0;
@@ -128,9 +130,9 @@ inline double EstimatePacked(const PackedPlan& plan, const PackedShape& shape, c
     if (load > resident)
     {
         busy = resident;
-        load = plan.workgroups * perGroup / kComputeUnits + 0.66 * std::max(1.0, perGroup);
+        load = plan.workgroups * perGroup / kComputeUnits + 0.62 * std::max(1.0, perGroup);
     }
-    const double rate = 1.0 - (1.0 - shape.alone) * std::pow(std::max(busy, 1.0), -0.88);
+    const double rate = 1.0 - (1.0 - shape.alone) * std::pow(std::max(busy, 1.0), -0.735);
     return load * wave / rate;
 }
 
