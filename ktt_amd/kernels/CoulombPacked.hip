@@ -4,7 +4,7 @@
 // (Examples/CoulombSum3d/CoulombSum3d.cu:10-15, :46; Examples/CoulombSum2d/CoulombSum2d.cl:126, :945).
 //
 //   POINTS_X, ROWS_PER_THREAD  points per lane (x run, rows)
-//   ROW_GROUP_CAP              row groups a wave may touch (kc::rowGroupsPerWave, rounded up)
+//   ROW_GROUP_CAP              row groups a wave may touch (RowGroupCap in CoulombPackedPlan.h)
 //   COMPENSATED                sums of 64 atoms added in 0: FP32, 1: FP64
 //   ROW_MODE                   0: a volume (rows = z * G + y), 1: one slice (rows = y, .z holds dz^2)
 //

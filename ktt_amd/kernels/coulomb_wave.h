@@ -9,14 +9,15 @@
 // last wave and a row length that PX does not divide leave lanes idle. (A workgroup of coulomb_core.h
 // spans a fixed number of x points instead: at a side of 150 its 128-point spans leave 41% of the
 // lanes idle, at 64 half of them.) A wave touches at most CAP row groups; the host derives CAP from
-// lanesX (kc::rowGroupsPerWave).
+// lanesX (RowGroupsPerWave in CoulombPackedPlan.h).
 //
 // Atoms are staged by the wave 64 at a time, one per lane, into LDS that only this wave uses: the
 // atom's x and charge, and the brackets B = (y - Y)^2 + (z - Z)^2 of every row of the wave's groups.
 // A wave's LDS operations complete in order, so the tile needs no barrier. B costs 3 to 4 instructions
 // per (row, atom), formed row after row with the row's y and z in scalars; the atom of the next tile
 // is read from memory while this one is summed. The inner loop is the issue-phased loop of
-// coulomb_core.h, and the last atom's r^-1 stays in flight over the tile's end.
+// coulomb_core.h. The plain form keeps the last atom's r^-1 in flight over the tile's end; the compensated
+// form, whose brackets in FP64 need its registers, lands it there.
 //
 // Split. The WAVE_SPLIT waves of a workgroup own the same 64 lanes and a contiguous share of the atoms
 // each. They meet in LDS once, in wave order (plain FP32; compensated FP64), so results do not depend on
@@ -25,10 +26,10 @@
 //
 // Bound by FP32 VALU issue as the workgroup engine is (per interaction 2 FMAs that pair with another
 // wave's and a v_rsq_f32 of two quad-cycles); small grids by the launch. Measured on MI355X with the
-// fill before it, workgroup shapes -> wave engine: 150^3 x 20,011 compensated 12,990 -> 6,213 us (119
-// TFLOP/s at 11 per interaction), 99^3 x 3,001 plain 636 -> 296, 64^3 x 5,000 compensated 363 -> 140,
-// 32^3 x 200 plain 59 -> 8.6. On 256^3 x 8,192, which the workgroup shapes fill, 11,670 -> 11,660 us
-// plain and 11,830 -> 12,010 compensated: every wave forms its own row brackets, and the compensated
+// fill before it, workgroup shapes -> wave engine: 150^3 x 20,011 compensated 12,990 -> 6,194 us (120
+// TFLOP/s at 11 per interaction), 99^3 x 3,001 plain 636 -> 292, 64^3 x 5,000 compensated 363 -> 138,
+// 32^3 x 200 plain 59 -> 7.0. On 256^3 x 8,192, which the workgroup shapes fill, 11,650 -> 11,750 us
+// plain and 11,750 -> 12,200 compensated: every wave forms its own row brackets, and the compensated
 // dx takes one FMA more per atom.
 #pragma once
 
@@ -47,12 +48,6 @@ struct Select<false, A, B>
 {
     using Type = B;
 };
-
-// Largest number of row groups that 64 consecutive lanes touch when a row group has lanesX lanes.
-constexpr int rowGroupsPerWave(const int lanesX)
-{
-    return lanesX % 64 == 0 ? 1 : (64 % lanesX == 0 ? 64 / lanesX : (64 - 2) / lanesX + 2);
-}
 
 // Orders this wave's LDS accesses for the compiler; the hardware keeps them in order.
 __device__ __forceinline__ void waveFence()
@@ -249,77 +244,15 @@ struct WaveEngine
             }
             waveFence();
             const int count = a1 - t < Tile ? static_cast<int>(a1 - t) : Tile;
-            for (int a = 0; a < count; a += Unroll)
+            int a = 0;
+            if constexpr (COMP)
             {
-#pragma unroll
-                for (int u = 0; u < Unroll; u += Phase)
-                {
-                    __builtin_amdgcn_sched_barrier(0);
-                    __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-                    for (int p = 0; p < Phase; ++p)
-                    {
-                        float dx[PX];
-                        float q;
-                        if constexpr (COMP)
-                        {
-                            const float4 v = *reinterpret_cast<const float4*>(lds + (a + u + p) * 4);
-                            dx[0] = fmaf(hV, x[0] - v.x, v.y);
-#pragma unroll
-                            for (int i = 1; i < PX; ++i)
-                            {
-                                dx[i] = dx[i - 1] + hV;
-                            }
-                            q = v.z;
-                        }
-                        else
-                        {
-                            const float2 v = *reinterpret_cast<const float2*>(lds + (a + u + p) * 2);
-#pragma unroll
-                            for (int i = 0; i < PX; ++i)
-                            {
-                                dx[i] = x[i] - v.x;
-                            }
-                            q = v.y;
-                        }
-                        float b[ROWS];
-#pragma unroll
-                        for (int k = 0; k < ROWS; k += 4)
-                        {
-                            const float4 v = *reinterpret_cast<const float4*>(sB + (a + u + p) * RowStride + k);
-                            b[k] = v.x;
-                            b[k + 1] = v.y;
-                            b[k + 2] = v.z;
-                            b[k + 3] = v.w;
-                        }
-#pragma unroll
-                        for (int k = 0; k < ROWS; ++k)
-                        {
-#pragma unroll
-                            for (int i = 0; i < PX; ++i)
-                            {
-                                part[k][i] = fmaf(qPrev[p], rr[p][k][i], part[k][i]);
-                                rr[p][k][i] = fmaf(dx[i], dx[i], b[k]);
-                            }
-                        }
-                        qPrev[p] = q;
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                    __builtin_amdgcn_s_setprio(3);
-#pragma unroll
-                    for (int p = 0; p < Phase; ++p)
-                    {
-#pragma unroll
-                        for (int k = 0; k < ROWS; ++k)
-                        {
-#pragma unroll
-                            for (int i = 0; i < PX; ++i)
-                            {
-                                rr[p][k][i] = __builtin_amdgcn_rsqf(rr[p][k][i]);
-                            }
-                        }
-                    }
-                }
+                addAtoms<true>(lds, sB, 0, x, hV, qPrev, rr);
+                a = Unroll;
+            }
+            for (; a < count; a += Unroll)
+            {
+                addAtoms<false>(lds, sB, a, x, hV, qPrev, rr);
             }
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_setprio(0);
@@ -334,12 +267,107 @@ struct WaveEngine
         if constexpr (!COMP)
         {
             land(qPrev, rr);
+            fold();
         }
-        fold();
     }
 
-    // part += q r^-1 of the atoms in flight, which are then none.
-    __device__ __forceinline__ void land(float (&q)[Phase], float (&rr)[Phase][ROWS][PX])
+    // Adds Unroll atoms of the staged tile from atom a on, in issue phases. FIRST (one atom per phase): the
+    // tile's first atoms, before which no atom is in flight and no sum begun. Clearing both per tile and
+    // adding a charge of zero takes three instructions per point and tile, 1.5% of the compensated loop: without
+    // them 150^3 x 20,011 takes 6,194 us instead of 6,303, 64^3 x 5,000 138.5 instead of 141.3. The plain form
+    // carries its atom over the tiles and has only the sums to clear.
+    template <bool FIRST>
+    __device__ __forceinline__ void addAtoms(const float* lds, const float* sB, const int a, const float (&x)[PX], const float hV,
+        float (&qPrev)[Phase], float (&rr)[Phase][ROWS][PX])
+    {
+#pragma unroll
+        for (int u = 0; u < Unroll; u += Phase)
+        {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+            for (int p = 0; p < Phase; ++p)
+            {
+                float dx[PX];
+                float q;
+                if constexpr (COMP)
+                {
+                    const float4 v = *reinterpret_cast<const float4*>(lds + (a + u + p) * 4);
+                    dx[0] = fmaf(hV, x[0] - v.x, v.y);
+#pragma unroll
+                    for (int i = 1; i < PX; ++i)
+                    {
+                        dx[i] = dx[i - 1] + hV;
+                    }
+                    q = v.z;
+                }
+                else
+                {
+                    const float2 v = *reinterpret_cast<const float2*>(lds + (a + u + p) * 2);
+#pragma unroll
+                    for (int i = 0; i < PX; ++i)
+                    {
+                        dx[i] = x[i] - v.x;
+                    }
+                    q = v.y;
+                }
+                float b[ROWS];
+#pragma unroll
+                for (int k = 0; k < ROWS; k += 4)
+                {
+                    const float4 v = *reinterpret_cast<const float4*>(sB + (a + u + p) * RowStride + k);
+                    b[k] = v.x;
+                    b[k + 1] = v.y;
+                    b[k + 2] = v.z;
+                    b[k + 3] = v.w;
+                }
+#pragma unroll
+                for (int k = 0; k < ROWS; ++k)
+                {
+#pragma unroll
+                    for (int i = 0; i < PX; ++i)
+                    {
+                        if constexpr (FIRST)
+                        {
+                            // The tile's first atom finds none in flight, and its second starts the sums.
+                            if (u == 1)
+                            {
+                                part[k][i] = qPrev[p] * rr[p][k][i];
+                            }
+                            else if (u > 1)
+                            {
+                                part[k][i] = fmaf(qPrev[p], rr[p][k][i], part[k][i]);
+                            }
+                        }
+                        else
+                        {
+                            part[k][i] = fmaf(qPrev[p], rr[p][k][i], part[k][i]);
+                        }
+                        rr[p][k][i] = fmaf(dx[i], dx[i], b[k]);
+                    }
+                }
+                qPrev[p] = q;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+            for (int p = 0; p < Phase; ++p)
+            {
+#pragma unroll
+                for (int k = 0; k < ROWS; ++k)
+                {
+#pragma unroll
+                    for (int i = 0; i < PX; ++i)
+                    {
+                        rr[p][k][i] = __builtin_amdgcn_rsqf(rr[p][k][i]);
+                    }
+                }
+            }
+        }
+    }
+
+    // part += q r^-1 of the atoms in flight.
+    __device__ __forceinline__ void land(const float (&q)[Phase], const float (&rr)[Phase][ROWS][PX])
     {
 #pragma unroll
         for (int p = 0; p < Phase; ++p)
@@ -351,10 +379,8 @@ struct WaveEngine
                 for (int i = 0; i < PX; ++i)
                 {
                     part[k][i] = fmaf(q[p], rr[p][k][i], part[k][i]);
-                    rr[p][k][i] = 0.0f;
                 }
             }
-            q[p] = 0.0f;
         }
     }
 
@@ -372,7 +398,10 @@ struct WaveEngine
             for (int i = 0; i < PX; ++i)
             {
                 sum[k][i] += static_cast<Sum>(part[k][i]);
-                part[k][i] = 0.0f;
+                if constexpr (!COMP)
+                {
+                    part[k][i] = 0.0f;
+                }
             }
             __builtin_amdgcn_sched_barrier(0);  // one row at a time: few registers
         }
