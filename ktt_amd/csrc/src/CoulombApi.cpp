@@ -857,8 +857,10 @@ static void CheckForm(const int gridSize, const int form)
 // all sides but the multiples of 256 (250^3 x 4,000: 5.36 against 5.86 ms plain, 5.56 against 6.42
 // compensated; 150^3 x 20,011: 5.9 against 11.2, 6.2 against 12.7; 33^3 x 500: 0.007 against 0.108,
 // 0.008 against 0.061). There the workgroup shapes fill every lane and share one set of row brackets
-// among 4 to 8 waves (256^3 x 8,192: 11.67 against 11.66 ms plain, 11.83 against 12.01 compensated). Above 1,024
-// the last span's idle lanes are under an eighth.
+// among 4 to 8 waves: 256^3 and 512^3 with 64 to 8,192 atoms ran between 4% faster and 3% slower than the wave
+// engine (256^3 x 8,192: 11.65 against 11.75 ms plain, 11.75 against 12.20 compensated; x 500
+// compensated 0.804 against 0.778, where the last round of workgroups is nearly empty), with no line between
+// the two. Above 1,024 the last span's idle lanes are under an eighth.
 static bool PackedPlanFor(const int atomCount, const int gridSize, const int form, const char* config, PackedPlan& plan)
 {
     const CoulombConfig given = CoulombConfig::Parse(config, CoulombConfig());

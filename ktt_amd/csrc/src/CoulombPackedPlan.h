@@ -31,7 +31,7 @@ struct PackedPlan
 // LDS of a workgroup on gfx950.
 constexpr long kPackedLdsBytes = 160 * 1024;
 
-// Row groups a wave of 64 lanes touches at most (kc::rowGroupsPerWave), of those there are.
+// Row groups a wave of 64 lanes touches at most when a row group has lanesX lanes, of those there are.
 inline int RowGroupsPerWave(const int lanesX, const int rowGroups)
 {
     return std::min(rowGroups, lanesX % 64 == 0 ? 1 : (64 % lanesX == 0 ? 64 / lanesX : (64 - 2) / lanesX + 2));
@@ -154,8 +154,8 @@ inline PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, co
         for (const int waves : {1, 4, 8, 16})
         {
             const PackedPlan plan = PlanShape(shape.px, shape.rows, waves, 1, atomCount, rowLength, rowsTotal, compensated);
-            // One-wave workgroups win while a wave's atoms are a tile or two (256^3 x 64: 113 us against
-            // 117 with 4 waves) and lose 5 to 10% beyond (180^3 x 500: 303 against 280).
+            // One-wave workgroups win while a wave's atoms are a tile or two (256^3 x 64: 102 us against
+            // 118 with 4 waves) and lose 5 to 10% beyond (180^3 x 500: 303 against 280).
             if (waves == 1 && atomCount > 128)
             {
                 continue;
