@@ -857,9 +857,9 @@ static void CheckForm(const int gridSize, const int form)
 // all sides but the multiples of 256 (250^3 x 4,000: 5.36 against 5.86 ms plain, 5.56 against 6.42
 // compensated; 150^3 x 20,011: 5.9 against 11.2, 6.2 against 12.7; 33^3 x 500: 0.007 against 0.108,
 // 0.008 against 0.061). There the workgroup shapes fill every lane and share one set of row brackets
-// among 4 to 8 waves: 256^3 and 512^3 with 64 to 8,192 atoms ran between 4% faster and 3% slower than the wave
-// engine (256^3 x 8,192: 11.65 against 11.75 ms plain, 11.75 against 12.20 compensated; x 500
-// compensated 0.804 against 0.778, where the last round of workgroups is nearly empty), with no line between
+// among 4 to 8 waves: 256^3 and 512^3 with 64 to 8,192 atoms ran between 3% faster and 5% slower than the wave
+// engine (256^3 x 8,192: 11.66 against 11.74 ms plain, 11.77 against 12.01 compensated; x 500
+// compensated 0.803 against 0.765, where the last round of workgroups is nearly empty), with no line between
 // the two. Above 1,024 the last span's idle lanes are under an eighth.
 static bool PackedPlanFor(const int atomCount, const int gridSize, const int form, const char* config, PackedPlan& plan)
 {
@@ -1174,8 +1174,8 @@ int ktt_coulomb3d_iterative_reference(const float* atoms, int atomCount, float s
 
 // Whether the slices of a grid run as the planes of one volume launch: without a configuration, as long
 // as a launch holds them. The same terms, without a launch's ramp and tail per slice, on a chip that one
-// slice does not fill, and without the FP32 atomics of the slices' atom blocks (128^3 x 8,192: 2,075 us in 128
-// launches, 1,552 in one). On the wave engine at every side: its 64-atom partial sums keep the slices'
+// slice does not fill, and without the FP32 atomics of the slices' atom blocks (128^3 x 8,192: 2,072 us in 128
+// launches, 1,543 in one). On the wave engine at every side: its 64-atom partial sums keep the slices'
 // precision, which the workgroup shapes' running sums would not (256^3 x 2,480: error against 64 bits
 // 3.5e-7 in slices, 1.2e-6 by CoulombSum3d.hip's plain form).
 static bool SlicesInOneLaunch(const int atomCount, const int gridSize, const char* config, PackedPlan& plan)

@@ -28,8 +28,8 @@
 // wave's and a v_rsq_f32 of two quad-cycles); small grids by the launch. Measured on MI355X with the
 // fill before it, workgroup shapes -> wave engine: 150^3 x 20,011 compensated 12,990 -> 6,194 us (120
 // TFLOP/s at 11 per interaction), 99^3 x 3,001 plain 636 -> 292, 64^3 x 5,000 compensated 363 -> 138,
-// 32^3 x 200 plain 59 -> 7.0. On 256^3 x 8,192, which the workgroup shapes fill, 11,650 -> 11,750 us
-// plain and 11,750 -> 12,200 compensated: every wave forms its own row brackets, and the compensated
+// 32^3 x 200 plain 59 -> 7 to 8. On 256^3 x 8,192, which the workgroup shapes fill, 11,660 -> 11,740 us
+// plain and 11,770 -> 12,010 compensated: every wave forms its own row brackets, and the compensated
 // dx takes one FMA more per atom.
 #pragma once
 
