@@ -84,12 +84,12 @@ extern "C" __global__ __launch_bounds__(NarrowShape::Threads) void kttNoAllocCom
     kc::volumeCompensated<NarrowShape>(src, numberOfAtoms, gridSpacing, gridSize, energyGrid, partials, tileCounters, splitFrom);
 }
 
-template <int PX, int ROWS, int CAP>
+template <int PX, int ROWS, int CAP, int LANES = 64>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5))) void kttNoAllocPacked(const float4* atoms,
     int numberOfAtoms, int share, float gridSpacing, int lanesX, int rowGroups, int rowLength, int rowsTotal, float* energyGrid)
 {
     extern __shared__ __attribute__((aligned(16))) float shared[];
-    kc::packedSum<kc::WaveEngine<PX, ROWS, CAP, kc::Volume, true>>(shared, atoms, numberOfAtoms, share, gridSpacing, lanesX,
+    kc::packedSum<kc::WaveEngine<PX, ROWS, CAP, kc::Volume, true>, LANES>(shared, atoms, numberOfAtoms, share, gridSpacing, lanesX,
         rowGroups, rowLength, rowsTotal, energyGrid);
 }
 
@@ -125,7 +125,7 @@ int FailHip(char* message, const size_t length, const char* what, const hipError
 using PackedKernel = void (*)(const float4*, int, int, float, int, int, int, int, float*);
 
 // The precompiled kernel of a shape, or null. ChoosePackedPlan gives 2 x 8 points with up to 4 row groups
-// per wave, 1 x 8 with up to 8 and 1 x 4 with up to 16 (a side of 6 or 7).
+// per wave, 1 x 8 and 1 x 4 with up to 8, the latter also on 32 lanes (a side of 6 or 7).
 PackedKernel PackedKernelOf(const ktt::PackedPlan& plan)
 {
     struct Entry
@@ -133,16 +133,19 @@ PackedKernel PackedKernelOf(const ktt::PackedPlan& plan)
         int px;
         int rows;
         int cap;
+        int lanes;
         PackedKernel kernel;
     };
-    static const Entry entries[] = {{2, 8, 1, kttNoAllocPacked<2, 8, 1>}, {2, 8, 2, kttNoAllocPacked<2, 8, 2>},
-        {2, 8, 3, kttNoAllocPacked<2, 8, 3>}, {2, 8, 4, kttNoAllocPacked<2, 8, 4>}, {1, 8, 1, kttNoAllocPacked<1, 8, 1>}, {1, 8, 2, kttNoAllocPacked<1, 8, 2>},
-        {1, 8, 3, kttNoAllocPacked<1, 8, 3>}, {1, 8, 4, kttNoAllocPacked<1, 8, 4>}, {1, 8, 8, kttNoAllocPacked<1, 8, 8>}, {1, 4, 1, kttNoAllocPacked<1, 4, 1>},
-        {1, 4, 2, kttNoAllocPacked<1, 4, 2>}, {1, 4, 4, kttNoAllocPacked<1, 4, 4>}, {1, 4, 8, kttNoAllocPacked<1, 4, 8>},
-        {1, 4, 16, kttNoAllocPacked<1, 4, 16>}};
+    static const Entry entries[] = {{2, 8, 1, 64, kttNoAllocPacked<2, 8, 1>}, {2, 8, 2, 64, kttNoAllocPacked<2, 8, 2>},
+        {2, 8, 3, 64, kttNoAllocPacked<2, 8, 3>}, {2, 8, 4, 64, kttNoAllocPacked<2, 8, 4>},
+        {1, 8, 1, 64, kttNoAllocPacked<1, 8, 1>}, {1, 8, 2, 64, kttNoAllocPacked<1, 8, 2>},
+        {1, 8, 3, 64, kttNoAllocPacked<1, 8, 3>}, {1, 8, 4, 64, kttNoAllocPacked<1, 8, 4>},
+        {1, 8, 8, 64, kttNoAllocPacked<1, 8, 8>}, {1, 4, 1, 64, kttNoAllocPacked<1, 4, 1>},
+        {1, 4, 2, 64, kttNoAllocPacked<1, 4, 2>}, {1, 4, 4, 64, kttNoAllocPacked<1, 4, 4>},
+        {1, 4, 8, 64, kttNoAllocPacked<1, 4, 8>}, {1, 4, 8, 32, kttNoAllocPacked<1, 4, 8, 32>}};
     for (const Entry& entry : entries)
     {
-        if (entry.px == plan.px && entry.rows == plan.rows && entry.cap == plan.cap)
+        if (entry.px == plan.px && entry.rows == plan.rows && entry.cap == plan.cap && entry.lanes == plan.lanes)
         {
             return entry.kernel;
         }

@@ -797,10 +797,23 @@ PackedClass PackedClassOf(const int side)
     return side >= 64 ? PackedClass{0, 2, 8} : (side >= 32 ? PackedClass{1, 1, 8} : PackedClass{2, 1, 4});
 }
 
-static long PackedBlocks(const HostSystem& system, const PackedClass& shape)
+// Lanes of a system: per row group, the row groups there are, and those a wave takes.
+struct PackedLanes
 {
-    const long g = system.gridSize;
-    return ((g + shape.px - 1) / shape.px * ((g * g + shape.rows - 1) / shape.rows) + 63) / 64;
+    int lanesX;
+    int rowGroups;
+    int lanes;
+
+    long Blocks() const { return (static_cast<long>(lanesX) * rowGroups + lanes - 1) / lanes; }
+};
+
+static PackedLanes PackedLanesOf(const HostSystem& system, const PackedClass& shape)
+{
+    PackedLanes result;
+    result.lanesX = (system.gridSize + shape.px - 1) / shape.px;
+    result.rowGroups = static_cast<int>((static_cast<long>(system.gridSize) * system.gridSize + shape.rows - 1) / shape.rows);
+    result.lanes = LanesPerWave(result.lanesX, result.rowGroups);
+    return result;
 }
 
 PackedBatchPlan PlanPackedBatch(const std::vector<HostSystem>& systems, const int waves)
@@ -813,12 +826,11 @@ PackedBatchPlan PlanPackedBatch(const std::vector<HostSystem>& systems, const in
     for (const auto& system : systems)
     {
         const PackedClass shape = PackedClassOf(system.gridSize);
-        const int lanesX = (system.gridSize + shape.px - 1) / shape.px;
-        const int rowGroups = static_cast<int>((static_cast<long>(system.gridSize) * system.gridSize + shape.rows - 1) / shape.rows);
+        const PackedLanes packed = PackedLanesOf(system, shape);
         int& cap = plan.caps[shape.index];
-        cap = std::max(cap, RowGroupCap(RowGroupsPerWave(lanesX, rowGroups), shape.rows));
+        cap = std::max(cap, RowGroupCap(RowGroupsPerWave(packed.lanesX, packed.rowGroups, packed.lanes), shape.rows));
         waveFloats = std::max(waveFloats, 64 * (4 + static_cast<long>(cap) * shape.rows + 4));
-        const long blocks = PackedBlocks(system, shape);
+        const long blocks = packed.Blocks();
         totalBlocks += blocks;
         const double one = system.atomCount * (shape.px * shape.rows / 16.0);
         work += static_cast<double>(blocks) * one;
@@ -859,7 +871,7 @@ size_t CountPackedItems(const std::vector<HostSystem>& systems)
     size_t total = 0;
     for (const auto& system : systems)
     {
-        total += static_cast<size_t>(PackedBlocks(system, PackedClassOf(system.gridSize)));
+        total += static_cast<size_t>(PackedLanesOf(system, PackedClassOf(system.gridSize)).Blocks());
     }
     return total;
 }
@@ -876,10 +888,10 @@ std::vector<int> BuildPackedItems(const std::vector<HostSystem>& systems)
     flat.reserve(4 * CountPackedItems(systems));
     for (const size_t s : order)
     {
-        const long blocks = PackedBlocks(systems[s], PackedClassOf(systems[s].gridSize));
-        for (long b = 0; b < blocks; ++b)
+        const PackedLanes packed = PackedLanesOf(systems[s], PackedClassOf(systems[s].gridSize));
+        for (long b = 0; b < packed.Blocks(); ++b)
         {
-            const int record[4] = {static_cast<int>(s), static_cast<int>(b), 0, 0};
+            const int record[4] = {static_cast<int>(s), static_cast<int>(b), packed.lanes, 0};
             flat.insert(flat.end(), record, record + 4);
         }
     }

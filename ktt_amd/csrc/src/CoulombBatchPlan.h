@@ -64,7 +64,7 @@ PackedClass PackedClassOf(int side);
 /** Longest work list the wave engine takes: 1,024-thread workgroups of a launch of 2^31 threads. */
 constexpr size_t kMaxPackedItems = 0x7fffffff / 1024;
 
-/** Number of 64-lane blocks of the systems. */
+/** Number of lane blocks (64 lanes, or fewer by LanesPerWave) of the systems. */
 size_t CountPackedItems(const std::vector<HostSystem>& systems);
 
 /** What a batch on the wave engine compiles and launches. */
@@ -78,7 +78,7 @@ struct PackedBatchPlan
 /** waves 0: by the batch's work. Throws KttException if the waves' brackets exceed the LDS. */
 PackedBatchPlan PlanPackedBatch(const std::vector<HostSystem>& systems, int waves);
 
-/** The wave engine's work list as flattened int4 records (system, 64-lane block, 0, 0), systems with
+/** The wave engine's work list as flattened int4 records (system, block, lanes per block, 0), systems with
  *  the most atoms first. */
 std::vector<int> BuildPackedItems(const std::vector<HostSystem>& systems);
 

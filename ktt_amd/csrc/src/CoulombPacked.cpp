@@ -40,9 +40,13 @@ PackedPlan PackedPlanOf(const CoulombConfig& config, const int atomCount, const 
 void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, float spacing, int rowLength, int rowsTotal,
     float* energyGrid, const bool compensated, const bool slice, hipStream_t stream, float* kernelMs)
 {
-    const std::vector<std::string> defines = {"-DPOINTS_X=" + std::to_string(plan.px), "-DROWS_PER_THREAD=" + std::to_string(plan.rows),
+    std::vector<std::string> defines = {"-DPOINTS_X=" + std::to_string(plan.px), "-DROWS_PER_THREAD=" + std::to_string(plan.rows),
         "-DROW_GROUP_CAP=" + std::to_string(plan.cap), std::string("-DCOMPENSATED=") + (compensated ? "1" : "0"),
         std::string("-DROW_MODE=") + (slice ? "1" : "0")};
+    if (plan.lanes != 64)
+    {
+        defines.push_back("-DWAVE_LANES=" + std::to_string(plan.lanes));
+    }
     const auto kernel = CoulombRuntime::Get().GetKernel("CoulombPacked.hip", "coulombPacked", defines);
     const unsigned int grid[3] = {plan.workgroups, static_cast<unsigned int>(plan.blocks), 1};
     const unsigned int block[3] = {static_cast<unsigned int>(plan.waves) * 64, 1, 1};

@@ -17,6 +17,7 @@ struct PackedPlan
 {
     int px = 0;
     int rows = 0;
+    int lanes = 64;     // lanes a wave takes
     int touched = 0;    // row groups a wave touches at most, and what the kernel is compiled for
     int cap = 0;
     int waves = 0;
@@ -31,10 +32,24 @@ struct PackedPlan
 // LDS of a workgroup on gfx950.
 constexpr long kPackedLdsBytes = 160 * 1024;
 
-// Row groups a wave of 64 lanes touches at most when a row group has lanesX lanes, of those there are.
-inline int RowGroupsPerWave(const int lanesX, const int rowGroups)
+// Row groups a wave of `lanes` lanes touches at most when a row group has lanesX lanes, of those there are.
+inline int RowGroupsPerWave(const int lanesX, const int rowGroups, const int lanes = 64)
 {
-    return std::min(rowGroups, lanesX % 64 == 0 ? 1 : (64 % lanesX == 0 ? 64 / lanesX : (64 - 2) / lanesX + 2));
+    return std::min(rowGroups, lanesX % lanes == 0 ? 1 : (lanes % lanesX == 0 ? lanes / lanesX : (lanes - 2) / lanesX + 2));
+}
+
+// Lanes a wave takes by default: 64, fewer while they touch more than 8 row groups (of volumes, 32 at sides 6 and
+// 7 in groups of 4 rows). 9 or 10 groups need brackets for 16 (RowGroupCap), 18 KiB of LDS per wave, and
+// leave 8 waves per CU where 8 groups leave 16: 7^3 x 200,000 compensated takes 2,342 us on 64 lanes and
+// 1,656 on 32, a batch of 128 systems up to 128^3 with some of side 7 33.1 and 28.0 ms.
+inline int LanesPerWave(const int lanesX, const int rowGroups)
+{
+    int lanes = 64;
+    while (lanes > 1 && RowGroupsPerWave(lanesX, rowGroups, lanes) > 8)
+    {
+        lanes /= 2;
+    }
+    return lanes;
 }
 
 // Row groups a kernel is compiled for when its waves touch up to `touched` of them: the next power of two,
@@ -56,7 +71,7 @@ inline int RowGroupCap(const int touched, const int rows)
 
 // The plan of a shape, or one with no workgroups when the shape does not fit the LDS or a launch.
 inline PackedPlan PlanShape(const int px, const int rows, const int waves, const int blocks, const int atomCount, const long rowLength,
-    const long rowsTotal, const bool compensated)
+    const long rowsTotal, const bool compensated, const int lanes = 64)
 {
     PackedPlan plan;
     plan.px = px;
@@ -65,10 +80,11 @@ inline PackedPlan PlanShape(const int px, const int rows, const int waves, const
     plan.blocks = blocks;
     const long lanesX = (rowLength + px - 1) / px;
     const long rowGroups = (rowsTotal + rows - 1) / rows;
-    const long workgroups = (lanesX * rowGroups + 63) / 64;
+    const long workgroups = (lanesX * rowGroups + lanes - 1) / lanes;
+    plan.lanes = lanes;
     plan.lanesX = static_cast<int>(lanesX);
     plan.rowGroups = static_cast<int>(rowGroups);
-    plan.touched = RowGroupsPerWave(plan.lanesX, plan.rowGroups);
+    plan.touched = RowGroupsPerWave(plan.lanesX, plan.rowGroups, lanes);
     plan.cap = RowGroupCap(plan.touched, rows);
     // Whole unrolled steps of 8 atoms per wave.
     const long shares = static_cast<long>(waves) * blocks;
@@ -153,7 +169,9 @@ inline PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, co
     {
         for (const int waves : {1, 4, 8, 16})
         {
-            const PackedPlan plan = PlanShape(shape.px, shape.rows, waves, 1, atomCount, rowLength, rowsTotal, compensated);
+            const int lanes = LanesPerWave(static_cast<int>((rowLength + shape.px - 1) / shape.px),
+                static_cast<int>((rowsTotal + shape.rows - 1) / shape.rows));
+            const PackedPlan plan = PlanShape(shape.px, shape.rows, waves, 1, atomCount, rowLength, rowsTotal, compensated, lanes);
             // One-wave workgroups win while a wave's atoms are a tile or two (256^3 x 64: 102 us against
             // 118 with 4 waves) and lose 5 to 10% beyond (180^3 x 500: 303 against 280).
             if (waves == 1 && atomCount > 128)

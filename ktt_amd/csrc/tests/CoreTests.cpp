@@ -631,6 +631,17 @@ void TestPackedBatch()
     CHECK(PlanPackedBatch({{0, 5000, 64, 0, 0.5f, 0, 0}}, 0).waves == 16);
     CHECK(PlanPackedBatch(std::vector<HostSystem>(200, {0, 2000, 128, 0, 0.5f, 0, 0}), 0).waves == 4);
     CHECK(PlanPackedBatch({{0, 10, 6, 0, 0.5f, 0, 0}}, 0).ldsBytes <= 160u * 1024u);
+    // One small system must not take the LDS of the others' waves: at most 10 KiB per wave at any side.
+    for (int side = 1; side <= 24; ++side)
+    {
+        const std::vector<HostSystem> mixed = {{0, 5000, 128, 0, 0.5f, 0, 0}, {0, 300, side, 0, 0.5f, 0, 0}};
+        const PackedBatchPlan mixedPlan = PlanPackedBatch(mixed, 0);
+        CHECK(mixedPlan.ldsBytes / static_cast<unsigned int>(mixedPlan.waves) <= 10240u);
+        const std::vector<int> items = BuildPackedItems({{0, 300, side, 0, 0.5f, 0, 0}});
+        const long lanes = static_cast<long>(side) * ((static_cast<long>(side) * side + 3) / 4);
+        CHECK(items.size() == 4 * static_cast<size_t>((lanes + items[2] - 1) / items[2]));
+        CHECK(ktt::RowGroupsPerWave(side, (side * side + 3) / 4, items[2]) <= mixedPlan.caps[2]);
+    }
 }
 
 /** The wave engine's launch plans over every grid side the default takes them for at small sizes, and
@@ -654,14 +665,15 @@ void TestPackedPlan()
                     fits = fits && plan.workgroups > 0 && plan.waves >= 1 && plan.waves <= 16 && plan.ldsBytes > 0
                         && plan.ldsBytes <= 160u * 1024u;
                     covers = covers && plan.share % 8 == 0 && static_cast<long>(plan.share) * plan.waves >= atoms
-                        && static_cast<long>(plan.workgroups) * 64 >= static_cast<long>(plan.lanesX) * plan.rowGroups
+                        && static_cast<long>(plan.workgroups) * plan.lanes >= static_cast<long>(plan.lanesX) * plan.rowGroups
+                        && static_cast<long>(plan.workgroups - 1) * plan.lanes < static_cast<long>(plan.lanesX) * plan.rowGroups
                         && plan.lanesX * plan.px >= g && (plan.lanesX - 1) * plan.px < g
                         && static_cast<long>(plan.rowGroups) * plan.rows >= rows
                         && static_cast<long>(plan.rowGroups - 1) * plan.rows < rows;
                     const long lanes = static_cast<long>(plan.lanesX) * plan.rowGroups;
-                    for (long first = 0; first < lanes; first += 64)
+                    for (long first = 0; first < lanes; first += plan.lanes)
                     {
-                        const long last = std::min(first + 63, lanes - 1);
+                        const long last = std::min(first + plan.lanes - 1, lanes - 1);
                         const long groups = last / plan.lanesX - first / plan.lanesX + 1;
                         bounded = bounded && groups <= plan.touched && groups <= plan.cap;
                     }
@@ -672,6 +684,14 @@ void TestPackedPlan()
     CHECK(fits);
     CHECK(covers);
     CHECK(bounded);
+    // Sides 6 and 7 take 32 lanes a wave, and their brackets no more LDS than the sides around them (10 KiB).
+    for (const int g : {5, 6, 7, 8})
+    {
+        const ktt::PackedPlan plan = ktt::ChoosePackedPlan(200000, g, static_cast<long>(g) * g, true);
+        CHECK(plan.lanes == (g == 6 || g == 7 ? 32 : 64));
+        CHECK(plan.waves == 16);
+        CHECK(plan.ldsBytes / static_cast<unsigned int>(plan.waves) <= 10240u);
+    }
     const auto refused = [](const int px, const int rows, const int waves, const long side)
     {
         try

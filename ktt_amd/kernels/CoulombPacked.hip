@@ -6,6 +6,7 @@
 //   POINTS_X, ROWS_PER_THREAD  points per lane (x run, rows)
 //   ROW_GROUP_CAP              row groups a wave may touch (RowGroupCap in CoulombPackedPlan.h)
 //   COMPENSATED                sums of 64 atoms added in 0: FP32, 1: FP64
+//   WAVE_LANES                 lanes a wave takes (LanesPerWave in CoulombPackedPlan.h)
 //   ROW_MODE                   0: a volume (rows = z * G + y), 1: one slice (rows = y, .z holds dz^2)
 //
 // Launch: kc::packedSum. Several atom blocks (plain form only) add to the grid with FP32 atomics.
@@ -16,6 +17,9 @@
 #endif
 #ifndef COMPENSATED
 #define COMPENSATED 0
+#endif
+#ifndef WAVE_LANES
+#define WAVE_LANES 64
 #endif
 #ifndef ROW_MODE
 #define ROW_MODE 0
@@ -28,5 +32,5 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
     int lanesX, int rowGroups, int rowLength, int rowsTotal, float* energyGrid)
 {
     extern __shared__ __attribute__((aligned(16))) float shared[];
-    kc::packedSum<W>(shared, atoms, numberOfAtoms, share, gridSpacing, lanesX, rowGroups, rowLength, rowsTotal, energyGrid);
+    kc::packedSum<W, WAVE_LANES>(shared, atoms, numberOfAtoms, share, gridSpacing, lanesX, rowGroups, rowLength, rowsTotal, energyGrid);
 }

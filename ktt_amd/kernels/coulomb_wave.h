@@ -9,7 +9,8 @@
 // last wave and a row length that PX does not divide leave lanes idle. (A workgroup of coulomb_core.h
 // spans a fixed number of x points instead: at a side of 150 its 128-point spans leave 41% of the
 // lanes idle, at 64 half of them.) A wave touches at most CAP row groups; the host derives CAP from
-// lanesX (RowGroupsPerWave in CoulombPackedPlan.h).
+// lanesX (RowGroupsPerWave in CoulombPackedPlan.h). Rows of 6 and 7 points would make 64 lanes touch 9
+// and 10 groups, whose brackets leave room for 8 waves per CU: such waves take 32 lanes (LanesPerWave).
 //
 // Atoms are staged by the wave 64 at a time, one per lane, into LDS that only this wave uses: the
 // atom's x and charge, and the brackets B = (y - Y)^2 + (z - Z)^2 of every row of the wave's groups.
@@ -92,15 +93,17 @@ struct WaveEngine
     float part[ROWS][PX];
     Sum sum[ROWS][PX];
 
-    __device__ __forceinline__ void place(const unsigned int waveBlock, const int lanesX, const int rowGroups)
+    // lanes: lanes that a wave takes, 64 or a power of two below it (the others idle).
+    __device__ __forceinline__ void place(const unsigned int waveBlock, const int lanesX, const int rowGroups, const int lanes)
     {
         lane = threadIdx.x & 63;
         const unsigned int total = static_cast<unsigned int>(lanesX) * static_cast<unsigned int>(rowGroups);
-        const unsigned int first = waveBlock * 64u;
+        const unsigned int first = waveBlock * static_cast<unsigned int>(lanes);
+        const unsigned int end = total - first < static_cast<unsigned int>(lanes) ? total : first + static_cast<unsigned int>(lanes);
         const unsigned int mine = first + lane;
-        valid = mine < total;
-        whole = total >= 64u && first <= total - 64u;
-        const unsigned int index = valid ? mine : total - 1u;
+        valid = mine < end;
+        whole = end - first == 64u;
+        const unsigned int index = valid ? mine : end - 1u;
         rowGroup = static_cast<int>(index / static_cast<unsigned int>(lanesX));
         xLane = static_cast<int>(index - static_cast<unsigned int>(rowGroup) * lanesX);
         firstGroup = __builtin_amdgcn_readfirstlane(rowGroup);
@@ -522,9 +525,9 @@ struct WaveEngine
     }
 };
 
-// The body of a wave-engine kernel: block 64 x waves threads, grid (64-lane blocks, atom blocks), dynamic
+// The body of a wave-engine kernel: block 64 x waves threads, grid (blocks of LANES lanes, atom blocks), dynamic
 // LDS of waves * WaveFloats floats. Wave w of atom block b sums atoms [(b * waves + w) * share, + share).
-template <class W>
+template <class W, int LANES>
 __device__ __forceinline__ void packedSum(float* shared, const float4* atoms, const int numberOfAtoms, const int share,
     const float gridSpacing, const int lanesX, const int rowGroups, const int rowLength, const int rowsTotal, float* energyGrid)
 {
@@ -534,7 +537,7 @@ __device__ __forceinline__ void packedSum(float* shared, const float4* atoms, co
     const int a0 = first < numberOfAtoms ? static_cast<int>(first) : numberOfAtoms;
     const int a1 = share < numberOfAtoms - a0 ? a0 + share : numberOfAtoms;
     W engine;
-    engine.place(blockIdx.x, lanesX, rowGroups);
+    engine.place(blockIdx.x, lanesX, rowGroups, LANES);
     engine.accumulate(shared + wave * W::WaveFloats, atoms, a0, a1, gridSpacing, rowLength);
     engine.store(shared, waves, wave, energyGrid, rowLength, rowsTotal, gridDim.y > 1);
 }

@@ -41,7 +41,7 @@ def check(capi, grid, count, form, config, spacing=0.5):
 
 
 @pytest.mark.parametrize("form", [0, 1])
-@pytest.mark.parametrize("grid", [1, 2, 3, 7, 16, 31, 33, 48, 65, 70])
+@pytest.mark.parametrize("grid", [1, 2, 3, 6, 7, 16, 31, 33, 48, 65, 70])
 def test_default_shapes(capi, grid, form):
     for count in (1, 64, 203):
         check(capi, grid, count, form, None)
@@ -146,7 +146,7 @@ def test_no_alloc_entry_point_takes_the_same_shapes(capi, grid, count):
 
 
 @pytest.mark.parametrize("config", [None, "WAVE_SPLIT=1", "WAVE_SPLIT=5"])
-@pytest.mark.parametrize("sides", [(3, 24, 31, 33, 66), (32, 48, 63, 64, 128), (7,)])
+@pytest.mark.parametrize("sides", [(3, 24, 31, 33, 66), (32, 48, 63, 64, 128), (7,), (6, 7, 48)])
 def test_batches(capi, sides, config):
     """Batches whose sides fall into each class of points per lane, ragged and not, with no atoms in one
     system, against FP64 at sampled points; eager and graph launches agree bit for bit."""
