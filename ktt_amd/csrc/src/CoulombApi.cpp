@@ -1114,15 +1114,10 @@ int ktt_coulomb2d(const float* atoms, int atomCount, float spacing, int gridX, i
         return SetLastError("grid " + std::to_string(gridX) + "x" + std::to_string(gridY) + " is not a multiple of the workgroup span "
             + std::to_string(spanX) + "x" + std::to_string(shape.rowsPerGroup));
     }
-    // A small slice is over in a few microseconds, most of them one workgroup's start: tile, barriers,
-    // brackets, adds. The wave engine in its smallest block, 32 atoms a wave, starts faster: 256^2 x
-    // 64 in 4.0 us against 5.9, x 500 in 6.2 against 7.5, 64^2 x 4,000 in 4.8 against 7.0. From about
-    // 75 million interactions on its finer split costs more than that saves (512^2 x 500: 16.0 against 15.7 us).
-    if (given.values.empty() && static_cast<long>(gridX) * gridY * atomCount <= 75000000L)
+    if (given.values.empty() && SliceOnWaveEngine(gridX, gridY, atomCount))
     {
-        const int blocks = std::max(1, (atomCount + 255) / 256);
-        LaunchPacked(MakePackedPlan(1, 4, 8, blocks, atomCount, gridX, gridY, false), atoms, atomCount, spacing, gridX, gridY, energyGrid,
-            false, true, static_cast<hipStream_t>(stream), kernelMs);
+        LaunchPacked(MakePackedPlan(kSlicePx, kSliceRows, kSliceWaves, SliceAtomBlocks(atomCount), atomCount, gridX, gridY, false), atoms,
+            atomCount, spacing, gridX, gridY, energyGrid, false, true, static_cast<hipStream_t>(stream), kernelMs);
         return 0;
     }
     auto kernel = CoulombRuntime::Get().GetKernel("CoulombSum2d.hip", "directCoulombSum", parsed.Defines(kLaunchOnly));

@@ -160,6 +160,52 @@ inline bool WaveEngineByDefault(const int side)
     return side % 256 != 0 && side <= 1024;
 }
 
+// The wave engine's launch for a slice: 1 x 4 points per lane, 8 waves per workgroup, at most 32 atoms a wave.
+constexpr int kSlicePx = 1;
+constexpr int kSliceRows = 4;
+constexpr int kSliceWaves = 8;
+inline int SliceAtomBlocks(const int atomCount)
+{
+    return atomCount > 256 ? (atomCount - 1) / 256 + 1 : 1;
+}
+
+/** Whether a slice runs the wave engine without a configuration. A small slice is over in a few microseconds,
+ *  most of them one workgroup's start: tile, barriers, brackets, adds, which the wave engine does faster. It
+ *  then costs more per atom and per workgroup than the workgroup shapes of CoulombSum2d.hip. Over 19 grids of
+ *  64^2 to 2,048^2 points and 1 to 30,000 atoms (MI355X, workgroup shapes / wave engine) it is the faster one
+ *   - while all its workgroups start at once (4 per CU) and the busiest CU's work through at most 64 atoms per
+ *     wave one after the other: 256^2 x 64 5.97 / 4.14 us, 64 x 1,024 x 512 7.20 / 6.17, 192^2 x 768 6.80 / 6.13,
+ *     512^2 x 128 7.04 / 6.77; beyond, 256^2 x 1,024 9.64 / 9.70, 192^2 x 1,024 7.49 / 7.96, 512^2 x 256 9.53 / 9.80;
+ *   - on up to 4,096 points, where the atom blocks of the workgroup shapes end at 128: 64^2 x 16,384 12.77 / 9.91,
+ *     to 75 million interactions (64^2 x 30,000 16.81 / 16.83);
+ *   - with at most 16 atoms, whose brackets and adds are little beside the grid: 768^2 x 16 8.07 / 6.50, 1,024^2 x
+ *     16 10.06 / 9.72; beyond, 1,024^2 x 32 10.03 / 10.83 and x 64 10.0 / 14.3, 2,048^2 x 16 31.0 / 32.4, 4,096^2 x 1
+ *     105 / 116. */
+inline bool SliceOnWaveEngine(const long gridX, const long gridY, const int atomCount)
+{
+    const long points = gridX * gridY;
+    const int blocks = SliceAtomBlocks(atomCount);
+    if (blocks > 65535)
+    {
+        return false;
+    }
+    const PackedPlan plan = PlanShape(kSlicePx, kSliceRows, kSliceWaves, blocks, atomCount, gridX, gridY, false);
+    if (plan.workgroups == 0)
+    {
+        return false;
+    }
+    const long workgroups = static_cast<long>(plan.workgroups) * blocks;
+    if (workgroups <= 4 * 256 && (workgroups + 255) / 256 * plan.share <= 64)
+    {
+        return true;
+    }
+    if (points <= 4096 && points * atomCount <= 75000000L)
+    {
+        return true;
+    }
+    return atomCount <= 16 && points <= 1L << 22 && points * atomCount <= 1L << 24;
+}
+
 /** The shape with the smallest estimated time. */
 inline PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, const long rowsTotal, const bool compensated)
 {

@@ -712,6 +712,44 @@ void TestPackedPlan()
     CHECK(refused(1, 4, 16, 46340));  // more threads than a launch holds
 }
 
+/** Which slices run the wave engine by default: the faster kernel of the measured ones, and a launch that exists
+ *  for all it takes. */
+void TestSliceRule()
+{
+    struct Measured
+    {
+        long x;
+        long y;
+        int atoms;
+        bool wave;
+    };
+    const Measured measured[] = {{64, 16, 1, true}, {64, 64, 8000, true}, {64, 64, 16384, true}, {64, 1024, 512, true},
+        {128, 128, 2048, true}, {192, 192, 768, true}, {256, 256, 64, true}, {256, 256, 500, true}, {320, 320, 256, true},
+        {384, 384, 128, true}, {512, 256, 256, true}, {512, 512, 64, true}, {512, 512, 128, true}, {64, 8192, 16, true},
+        {768, 768, 16, true}, {1024, 1024, 8, true}, {2048, 2048, 4, true}, {256, 256, 4000, false}, {192, 192, 1024, false},
+        {320, 320, 512, false}, {384, 384, 256, false}, {512, 512, 256, false}, {64, 8192, 64, false}, {8192, 64, 64, false},
+        {768, 768, 64, false}, {1024, 512, 64, false}, {1024, 1024, 32, false}, {1024, 1024, 64, false}, {2048, 1024, 32, false},
+        {2048, 2048, 16, false}, {4096, 4096, 1, false}, {64, 1024, 3000, false}, {256, 256, 1 << 30, false}};
+    for (const Measured& m : measured)
+    {
+        CHECK(ktt::SliceOnWaveEngine(m.x, m.y, m.atoms) == m.wave);
+    }
+    bool exists = true;
+    for (const long x : {64L, 192L, 1024L, 8192L})
+    {
+        for (const long y : {16L, 48L, 1024L, 8192L})
+        {
+            for (const int atoms : {0, 1, 17, 256, 257, 5000, 70000})
+            {
+                exists = exists && (!ktt::SliceOnWaveEngine(x, y, atoms)
+                    || ktt::MakePackedPlan(ktt::kSlicePx, ktt::kSliceRows, ktt::kSliceWaves, ktt::SliceAtomBlocks(atoms), atoms, x, y, false)
+                            .workgroups > 0);
+            }
+        }
+    }
+    CHECK(exists);
+}
+
 int main(int argc, char** argv)
 {
     if (argc != 2)
@@ -732,6 +770,7 @@ int main(int argc, char** argv)
     TestProfileSearcherAnalysis();
     TestBatchWorkList();
     TestPackedPlan();
+    TestSliceRule();
     TestPackedBatch();
     std::printf("%d checks, %d failures\n", g_Checks, g_Failures);
     return g_Failures == 0 ? 0 : 1;
