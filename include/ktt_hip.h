@@ -102,9 +102,11 @@ int ktt_hip_event_elapsed_ms(void* start, void* end, float* milliseconds);
  * compensated defaults, above 1,448 with the plain ones) they fold into the launch's x dimension,
  * and the point index is 64-bit (the reference kernel's int index overflows above G = 1,290).
  * Without a configuration, sides up to 1,024 that are not a multiple of 256 run the wave engine
- * (CoulombPacked.hip), whose lanes pack any side and whose waves split the atoms of small grids;
+ * (CoulombPacked.hip), whose lanes pack any side and whose waves split the atoms of small grids (up to
+ * 64 atoms on sides that suit the workgroup shapes excepted);
  * WAVE_SPLIT (1 to 16 waves sharing the atoms of 64 lanes), with POINTS_X (1 to 4, default 2) and
- * ROWS_PER_THREAD (4 or 8, the default), selects it explicitly. */
+ * ROWS_PER_THREAD (4 or 8, the default), selects it explicitly. The kernel that a call without a
+ * configuration compiles at its first use depends on the side, the form and the number of atoms. */
 int ktt_coulomb3d(const float* atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
                   int form, const char* config, void* stream, float* kernel_ms);
 

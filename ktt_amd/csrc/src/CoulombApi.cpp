@@ -871,7 +871,7 @@ static bool PackedPlanFor(const int atomCount, const int gridSize, const int for
         plan = PackedPlanOf(given, atomCount, gridSize, rows, compensated);
         return true;
     }
-    if (!given.values.empty() || !WaveEngineByDefault(gridSize))
+    if (!given.values.empty() || !WaveEngineByDefault(gridSize) || FewAtomsOnWorkgroupShapes(gridSize, atomCount, compensated))
     {
         return false;
     }
@@ -950,7 +950,8 @@ static void LaunchVolume(const float* atoms, int atomCount, float spacing, int g
     }
     auto& runtime = CoulombRuntime::Get();
     void* partials = plan.partialBytes > 0 ? runtime.GetScratch("coulomb3d.partials", plan.partialBytes) : nullptr;
-    void* counters = runtime.GetScratch("coulomb3d.counters", std::max<size_t>(1, plan.counterCount) * sizeof(unsigned int));
+    // The kernel reads neither when no tile is split; such a launch then allocates nothing, also under capture.
+    void* counters = plan.counterCount > 0 ? runtime.GetScratch("coulomb3d.counters", plan.counterCount * sizeof(unsigned int)) : nullptr;
     void* arguments[] = {&atoms, &unused, &unused, &unused, &unused, &atomCount, &spacing, &gridSize, &energyGrid, &partials, &counters,
         &plan.splitFrom};
     CoulombRuntime::Launch(*plan.kernel, plan.grid, plan.shape.block, arguments, stream, kernelMs);

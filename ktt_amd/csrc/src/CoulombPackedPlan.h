@@ -206,6 +206,33 @@ inline bool SliceOnWaveEngine(const long gridX, const long gridY, const int atom
     return atomCount <= 16 && points <= 1L << 22 && points * atomCount <= 1L << 24;
 }
 
+/** Whether a volume of few atoms runs faster on the workgroup shapes although its side takes the wave engine by default.
+ *  Up to 64 atoms are one tile of either kernel, and clearing, reading and writing the grid count as much as the sum.
+ *  The workgroup shapes win where they compute no padding to speak of: atoms that fill their 16-, 32- or 64-atom
+ *  tile to the wave engine's step of 8, and rows that nearly fill the 128-point spans. (MI355X, workgroup shapes / wave
+ *  engine, plain and compensated:)
+ *   - below a side of 128, where 2 x 8 blocks are two waves per SIMD and the chooser's narrower ones pay for their
+ *     start: 117^3 x 16 0.86 and 0.91, 125^3 x 32 0.83 and 0.83, 127^3 x 64 0.90 and 0.87, but 113^3 x 64 1.07 and 1.07;
+ *   - in the plain form at odd sides, whose rows the wave engine stores point by point: 9 to 16 atoms at 251^3 0.90,
+ *     at 511^3 0.85, at 1,023^3 0.87 (32 atoms 0.96, 0.94, 0.98; even sides and the compensated form 1.0 to 1.5), and
+ *     1 to 8 atoms above a side of 448: 511^3 0.93, 1,023^3 0.94 (383^3 1.10).
+ *  The sums are as exact either way: one tile, added in order. */
+inline bool FewAtomsOnWorkgroupShapes(const int side, const int atomCount, const bool compensated)
+{
+    const int spans = (side + 127) / 128;
+    const int tile = atomCount <= 16 ? 16 : (atomCount <= 32 ? 32 : 64);
+    if (atomCount < 1 || atomCount > tile)
+    {
+        return false;
+    }
+    const bool full = (atomCount + 7) / 8 * 8 == tile;
+    if (side < 128)
+    {
+        return full && side * 10 >= 128 * 9;
+    }
+    return !compensated && side % 2 != 0 && side * 20 >= spans * 128 * 17 && atomCount <= 16 && (full || side > 448);
+}
+
 /** The shape with the smallest estimated time. */
 inline PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, const long rowsTotal, const bool compensated)
 {

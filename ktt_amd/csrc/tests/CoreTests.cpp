@@ -750,6 +750,26 @@ void TestSliceRule()
     CHECK(exists);
 }
 
+/** Which volumes of few atoms leave the wave engine: those measured slower on it. */
+void TestFewAtomsRule()
+{
+    const auto plain = [](const int side, const int atoms) { return ktt::FewAtomsOnWorkgroupShapes(side, atoms, false); };
+    const auto compensated = [](const int side, const int atoms) { return ktt::FewAtomsOnWorkgroupShapes(side, atoms, true); };
+    for (const auto& [side, atoms] : {std::pair<int, int>{117, 16}, {120, 12}, {121, 32}, {125, 16}, {125, 32}, {127, 64}})
+    {
+        CHECK(plain(side, atoms) && compensated(side, atoms));
+    }
+    for (const auto& [side, atoms] : {std::pair<int, int>{251, 16}, {383, 12}, {511, 16}, {511, 1}, {1023, 16}, {1023, 8}})
+    {
+        CHECK(plain(side, atoms) && !compensated(side, atoms));
+    }
+    for (const auto& [side, atoms] : {std::pair<int, int>{24, 16}, {101, 16}, {113, 64}, {125, 48}, {127, 65}, {127, 200}, {127, 0},
+        {191, 16}, {250, 16}, {251, 32}, {383, 8}, {510, 16}, {511, 20}, {511, 64}, {640, 16}, {1000, 1}})
+    {
+        CHECK(!plain(side, atoms) && !compensated(side, atoms));
+    }
+}
+
 int main(int argc, char** argv)
 {
     if (argc != 2)
@@ -771,6 +791,7 @@ int main(int argc, char** argv)
     TestBatchWorkList();
     TestPackedPlan();
     TestSliceRule();
+    TestFewAtomsRule();
     TestPackedBatch();
     std::printf("%d checks, %d failures\n", g_Checks, g_Failures);
     return g_Failures == 0 ? 0 : 1;

@@ -171,3 +171,20 @@ def test_batches(capi, sides, config):
         batch.run(use_graph=True)
         for first, again in zip(grids, batch.grids()):
             np.testing.assert_array_equal(first, again)
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("grid,count", [(117, 16), (127, 64), (251, 12), (255, 16)])
+def test_few_atoms(capi, grid, count, form):
+    """Sides of the wave engine whose few atoms run on the workgroup shapes (plain; compensated below 128):
+    the plan says so, and the map meets the bar at sampled points."""
+    plan = capi.coulomb3d_launch_plan(count, grid, form=form)
+    workgroup_shapes = grid < 128 or form == 0
+    assert (plan["block"][1] > 1) == workgroup_shapes, plan
+    assert plan["scratch_bytes"] == 0
+    atoms = workloads.uniform_atoms(500 + grid, count, box=grid * 0.5)
+    print(f"few atoms: grid {grid} atoms {count} form {form}", flush=True)
+    out = run_guarded(capi, atoms, 0.5, grid, form, None).reshape(grid, grid, grid)
+    points = workloads.sample_points(501, 2048, grid)
+    values, norms = oracle.points_f64(atoms, 0.5, points)
+    assert oracle.normalised_error(out[points[:, 2], points[:, 1], points[:, 0]], values, norms)[0] <= BARS[form]
