@@ -37,8 +37,7 @@ PackedPlan PackedPlanOf(const CoulombConfig& config, const int atomCount, const 
         rowLength, rowsTotal, compensated);
 }
 
-void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, float spacing, int rowLength, int rowsTotal,
-    float* energyGrid, const bool compensated, const bool slice, hipStream_t stream, float* kernelMs)
+std::shared_ptr<HipKernel> GetPackedKernel(const PackedPlan& plan, const bool compensated, const bool slice)
 {
     std::vector<std::string> defines = {"-DPOINTS_X=" + std::to_string(plan.px), "-DROWS_PER_THREAD=" + std::to_string(plan.rows),
         "-DROW_GROUP_CAP=" + std::to_string(plan.cap), std::string("-DCOMPENSATED=") + (compensated ? "1" : "0"),
@@ -47,7 +46,13 @@ void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, flo
     {
         defines.push_back("-DWAVE_LANES=" + std::to_string(plan.lanes));
     }
-    const auto kernel = CoulombRuntime::Get().GetKernel("CoulombPacked.hip", "coulombPacked", defines);
+    return CoulombRuntime::Get().GetKernel("CoulombPacked.hip", "coulombPacked", defines);
+}
+
+void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, float spacing, int rowLength, int rowsTotal,
+    float* energyGrid, const bool compensated, const bool slice, hipStream_t stream, float* kernelMs)
+{
+    const auto kernel = GetPackedKernel(plan, compensated, slice);
     const unsigned int grid[3] = {plan.workgroups, static_cast<unsigned int>(plan.blocks), 1};
     const unsigned int block[3] = {static_cast<unsigned int>(plan.waves) * 64, 1, 1};
     int share = plan.share;

@@ -17,6 +17,9 @@ PackedPlan MakePackedPlan(int px, int rows, int waves, int blocks, int atomCount
  *  optional but WAVE_SPLIT. */
 PackedPlan PackedPlanOf(const CoulombConfig& config, int atomCount, long rowLength, long rowsTotal, bool compensated);
 
+/** The compiled kernel of a plan (compiles at its first use). slice as for LaunchPacked. */
+std::shared_ptr<HipKernel> GetPackedKernel(const PackedPlan& plan, bool compensated, bool slice);
+
 /** energyGrid += V on rows of rowLength points. slice: rows = y and the atoms' z holds dz^2; else
  *  rows = z * rowLength + y of a cube. */
 void LaunchPacked(const PackedPlan& plan, const float* atoms, int atomCount, float spacing, int rowLength, int rowsTotal,
