@@ -154,8 +154,8 @@ int ktt_coulomb2d_reference(const float* atoms, int n_atoms, float spacing, int 
  * (h*z - Z_i)^2 in FP32. host_atoms: float4[n_atoms] in host memory with the real z. With a
  * configuration, as the reference launcher does it: for every slice the host computes dz^2 of all atoms,
  * uploads the atom records with .z replaced, and launches the slice kernel (CoulombSum3dIterative.cl:35)
- * with zIndex = z. Without one, the atoms are uploaded once and one launch covers all slices, forming
- * dz^2 on the device. wall_ms receives the host time of the whole call's work, kernel_ms the (sum of the)
+ * with zIndex = z. Without one, or with WAVE_SPLIT as in ktt_coulomb3d, the atoms are uploaded once and one
+ * launch covers all slices, forming dz^2 on the device. wall_ms receives the host time of the whole call's work, kernel_ms the (sum of the)
  * kernels' event times; the call returns when they have ended. */
 int ktt_coulomb3d_iterative(const float* host_atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
                             const char* config, void* stream, float* kernel_ms, float* wall_ms);
@@ -169,9 +169,10 @@ int ktt_coulomb3d_iterative_reference(const float* atoms, int n_atoms, float spa
                                       void* stream, float* kernel_ms);
 
 /* Fused slice loop: dz^2 is formed on the device (atoms with their real z on the device). Without a
- * configuration all slices run as the planes of one volume launch of the wave engine (plain form); with
- * one, the slice kernel is launched per slice, no host work between launches. Either way grid_size
- * must be tiled by the slice kernel's workgroups, as for ktt_coulomb2d. */
+ * configuration, or with WAVE_SPLIT as in ktt_coulomb3d, all slices run as the planes of one volume launch
+ * of the wave engine (plain form); with another, the slice kernel is launched per slice, no host work
+ * between launches. In every case grid_size must be tiled by the slice kernel's workgroups (its defaults
+ * with the POINTS_X and ROWS_PER_THREAD given), as for ktt_coulomb2d without WAVE_SPLIT. */
 int ktt_coulomb3d_slices(const float* atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
                          const char* config, void* stream, float* kernel_ms);
 

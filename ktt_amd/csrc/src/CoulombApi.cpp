@@ -1168,19 +1168,26 @@ int ktt_coulomb3d_iterative_reference(const float* atoms, int atomCount, float s
     KTT_C_CATCH
 }
 
-// Whether the slices of a grid run as the planes of one volume launch: without a configuration, as long
-// as a launch holds them. The same terms, without a launch's ramp and tail per slice, on a chip that one
+// Whether the slices of a grid run as the planes of one volume launch: with WAVE_SPLIT in the configuration, and
+// without a configuration as long as a launch holds them. The same terms, without a launch's ramp and tail per slice, on a chip that one
 // slice does not fill, and without the FP32 atomics of the slices' atom blocks (128^3 x 8,192: 2,072 us in 128
 // launches, 1,543 in one). On the wave engine at every side: its 64-atom partial sums keep the slices'
 // precision, which the workgroup shapes' running sums would not (256^3 x 2,480: error against 64 bits
 // 3.5e-7 in slices, 1.2e-6 by CoulombSum3d.hip's plain form).
 static bool SlicesInOneLaunch(const int atomCount, const int gridSize, const char* config, PackedPlan& plan)
 {
-    if (!CoulombConfig::Parse(config, CoulombConfig()).values.empty())
+    const CoulombConfig given = CoulombConfig::Parse(config, CoulombConfig());
+    const long rows = static_cast<long>(gridSize) * gridSize;
+    if (given.Has("WAVE_SPLIT"))
+    {
+        plan = PackedPlanOf(given, atomCount, gridSize, rows, false);
+        return true;
+    }
+    if (!given.values.empty())
     {
         return false;
     }
-    plan = ChoosePackedPlan(atomCount, gridSize, static_cast<long>(gridSize) * gridSize, false);
+    plan = ChoosePackedPlan(atomCount, gridSize, rows, false);
     return plan.workgroups != 0;
 }
 

@@ -123,6 +123,31 @@ def test_slices(capi, grid_x, grid_y, count, config):
     assert oracle.normalised_error(out[:grid_x * grid_y], values, norms)[0] <= BARS[0]
 
 
+def test_slice_calls_take_wave_split(capi):
+    """WAVE_SPLIT in the two iterative entry points: the planes of the volume launch that ktt_coulomb3d makes of the
+    same configuration, bit for bit, and its refusals; sides the slice kernels do not tile stay refused."""
+    grid, spacing = 128, 0.5
+    atoms = workloads.uniform_atoms(81, 700, box=grid * spacing)
+    atoms_buffer = capi.DeviceBuffer.from_array(atoms)
+    energy = capi.DeviceBuffer(4 * grid ** 3)
+    for config in ("WAVE_SPLIT=4,POINTS_X=1,ROWS_PER_THREAD=8", "WAVE_SPLIT=2"):
+        volume = run_guarded(capi, atoms, spacing, grid, 0, config).reshape(grid, grid, grid)
+        energy.zero()
+        capi.coulomb3d_slices(atoms_buffer, atoms.shape[0], spacing, grid, energy, config=config)
+        np.testing.assert_array_equal(energy.download((grid,) * 3), volume)
+        energy.zero()
+        capi.coulomb3d_iterative(atoms, spacing, grid, energy, config=config)
+        np.testing.assert_array_equal(energy.download((grid,) * 3), volume)
+    for config in ("WAVE_SPLIT=17", "WAVE_SPLIT=2,ROWS_PER_THREAD=6"):
+        for call in (lambda: capi.coulomb3d_slices(atoms_buffer, atoms.shape[0], spacing, grid, energy, config=config),
+                     lambda: capi.coulomb3d_iterative(atoms, spacing, grid, energy, config=config)):
+            with pytest.raises(capi.KttHipError):
+                call()
+    for config in (None, "WAVE_SPLIT=4"):
+        with pytest.raises(capi.KttHipError, match="multiple of the workgroup span"):
+            capi.coulomb3d_slices(atoms_buffer, atoms.shape[0], spacing, 100, energy, config=config)
+
+
 @pytest.mark.parametrize("grid,count", [(1, 5), (6, 30), (9, 100), (24, 700), (45, 300), (63, 64), (70, 3000), (100, 501)])
 def test_no_alloc_entry_point_takes_the_same_shapes(capi, grid, count):
     """ktt_coulomb3d_compensated_noalloc at sides that run the wave engine, one for each of its
