@@ -181,7 +181,10 @@ int ktt_coulomb3d_slices(const float* atoms, int n_atoms, float spacing, int gri
  * 2 = CoulombSum2d / slice kernels (rows = grid_size), with the defaults of a slice of more
  * than 16,384 atoms; z is the configuration's ATOM_BLOCKS, before it is capped at the atom
  * tiles of a call. For kind 3, more than 65,535 row groups fold into x: grid[0] is then
- * fold * x groups and grid[1] the row groups / fold, rounded up. */
+ * fold * x groups and grid[1] the row groups / fold, rounded up. With WAVE_SPLIT the wave engine's
+ * launch (plain form): its workgroups in grid[0], the atom blocks in grid[1], 64 threads per wave.
+ * Without it the workgroup kernels' launch, also where a call without a configuration runs the wave
+ * engine: that choice depends on the atoms and the form, and ktt_coulomb3d_launch_plan reports it. */
 int ktt_coulomb_launch_shape(int kind, int grid_size, const char* config, unsigned int grid[3], unsigned int block[3]);
 
 /* ---- 5. Batches of independent systems --------------------------------------------------- */

@@ -808,8 +808,18 @@ int ktt_coulomb_launch_shape(int kind, int gridSize, const char* config, unsigne
     {
         return SetLastError("invalid arguments");
     }
-    const CoulombConfig parsed = CoulombConfig::Parse(config, kind == 3 ? Defaults3d(KTT_COULOMB_PLAIN, gridSize) : DefaultsSlice(1 << 30, gridSize, gridSize));
     const long rows = kind == 3 ? static_cast<long>(gridSize) * gridSize : gridSize;
+    const CoulombConfig given = CoulombConfig::Parse(config, CoulombConfig());
+    if (given.Has("WAVE_SPLIT"))
+    {
+        const PackedPlan packed = PackedPlanOf(given, 1 << 30, gridSize, rows, false);
+        grid[0] = packed.workgroups;
+        grid[1] = static_cast<unsigned int>(packed.blocks);
+        block[0] = static_cast<unsigned int>(packed.waves) * 64;
+        grid[2] = block[1] = block[2] = 1;
+        return 0;
+    }
+    const CoulombConfig parsed = CoulombConfig::Parse(config, kind == 3 ? Defaults3d(KTT_COULOMB_PLAIN, gridSize) : DefaultsSlice(1 << 30, gridSize, gridSize));
     const CoulombShape shape = CoulombRuntime::RowShape(parsed, gridSize, rows, parsed.Get("ATOM_BLOCKS", 1), kind == 3);
     for (int i = 0; i < 3; ++i)
     {

@@ -66,6 +66,14 @@ def test_launch_shape_follows_configuration():
         capi.launch_shape(3, 256, "WORK_GROUP_SIZE_X=64,WORK_GROUP_SIZE_Y=32")
 
 
+def test_launch_shape_of_the_wave_engine():
+    # 2 x 8 points per lane: 50 lanes per row group, 1,250 row groups, 64 lanes a workgroup.
+    assert capi.launch_shape(3, 100, "WAVE_SPLIT=4") == ((-(-50 * 1250 // 64), 1, 1), (256, 1, 1))
+    assert capi.launch_shape(2, 96, "WAVE_SPLIT=16,POINTS_X=1,ROWS_PER_THREAD=4,ATOM_BLOCKS=3") == ((96 * 24 // 64, 3, 1), (1024, 1, 1))
+    with pytest.raises(capi.KttHipError, match="WAVE_SPLIT"):
+        capi.launch_shape(3, 100, "WAVE_SPLIT=17")
+
+
 def fold_cover(grid_side, grid, block, span, rows_per_group):
     """The tiles (row group * x groups + x group) of the workgroups of a volume launch that do
     not exit, as the kernels derive them (kc::volumeGroup in ktt_amd/kernels/coulomb_core.h),
