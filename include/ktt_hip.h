@@ -197,7 +197,8 @@ int ktt_coulomb_launch_shape(int kind, int grid_size, const char* config, unsign
  * side is a tile-shape bucket. Without a configuration the batch runs the wave engine (up to 2 million
  * 64-lane work items; WAVE_SPLIT sets the waves that split a system's atoms, 1 to 16). Config names of the
  * persistent bucket kernel: BUCKETb_WGX, BUCKETb_PX, BUCKETb_ROWS, BUCKETb_TILE, BUCKETb_UNROLL (b = 0..4,
- * buckets in increasing grid side) and GROUPS_PER_CU. The batch owns the device copies of the atoms and one
+ * buckets in increasing grid side) and GROUPS_PER_CU; beside WAVE_SPLIT they are the shapes that
+ * ktt_coulomb_batch_tune starts from. The batch owns the device copies of the atoms and one
  * packed output array of all grids. */
 int ktt_coulomb_batch_create(const float* host_atoms, const int* atom_counts, const int* grid_sizes, const float* spacings,
                              int system_count, const char* config, void** batch);
@@ -224,9 +225,11 @@ int ktt_coulomb_batch_run_per_system(void* batch, int form, void* stream, float*
 
 /* Tunes the tile shape of every bucket with ktt::Tuner on ComputeApi::HIP (a composite kernel
  * and launcher over the bucket's systems; searcher as in section 4), bucket after bucket, and
- * keeps the winners in the batch, which then runs the bucket kernel. results_file (optional) is a path prefix: the KTT JSON
+ * keeps the winners in the batch. A batch that ran the wave engine, which the buckets' space does not hold,
+ * is then timed on both and keeps the faster one. results_file (optional) is a path prefix: the KTT JSON
  * results of bucket b go to <prefix>_bucket<b>.json and the winners to <prefix>_winners.json.
- * best_config (optional) receives the winning shapes as a configuration string. */
+ * best_config (optional) receives the winning shapes as a configuration string, with WAVE_SPLIT in front
+ * if the batch stays on the wave engine. */
 int ktt_coulomb_batch_tune(void* batch, int searcher, int max_configurations_per_bucket, const char* results_file,
                            char* best_config, size_t best_config_length);
 

@@ -100,6 +100,23 @@ def test_bucket_tuning_keeps_results_correct(capi, tmp_path):
     check_against_oracle(systems, batch.grids(), COMPENSATED_BAR)
 
 
+def test_bucket_tuning_does_not_leave_a_batch_slower(capi):
+    """A batch that runs the wave engine by default keeps it when the tuned buckets are not faster. At a side of 113 every
+    span of the buckets' space leaves at least 11% of its lanes idle. The configuration it returns creates the same batch."""
+    systems = [workloads.BatchSystem(workloads.uniform_atoms(5600 + k, 1500 + 100 * k, box=56.5, stream=3), 113, 0.5) for k in range(8)]
+    batch = capi.Batch(systems)
+    before = batch.info()["shapes"]
+    assert before.startswith("WAVE_SPLIT=")
+    best = batch.tune(searcher=capi.SEARCHER_RANDOM, max_configurations=2)
+    print("tuned 113^3 batch:", best, flush=True)
+    assert batch.info()["shapes"] == before
+    assert best.startswith(before + ",BUCKET0_WGX=")
+    assert capi.Batch(systems, config=best).info()["shapes"] == before
+    batch.zero()
+    batch.run(use_graph=True)
+    check_against_oracle(systems, batch.grids(), COMPENSATED_BAR)
+
+
 def test_full_batch_every_system_against_oracle(capi):
     """The 1,024-system batch of the benchmark (atom counts log-uniform in [200, 20000], sides
     32/48/64/96/128, so every bucket's tile shape runs) through the graph-launched persistent
