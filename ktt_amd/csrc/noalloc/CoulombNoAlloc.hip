@@ -9,7 +9,8 @@
 //   grid side a multiple of 256: 128 x 2 threads, 2 x 8 points per thread, tile 256, unroll 16
 //   other sides above 1,024:      64 x 2 threads, same per-thread block
 //   other sides up to 1,024:      the wave engine (kc::packedSum) at the shape of
-//                                 ktt::ChoosePackedPlan, which needs no scratch.
+//                                 ktt::ChoosePackedPlan, one of ktt::kPackedVariants,
+//                                 which needs no scratch.
 //
 // Scratch.  The split tiles' (sum, comp) partials and their arrival counters live in the
 // file-scope array `scratch` (kScratchBytes per device, held by every GPU the library runs on
@@ -27,6 +28,7 @@
 #include <cstddef>
 #include <cstdio>
 #include <mutex>
+#include <utility>
 
 #include "CoulombPackedPlan.h"
 #include "coulomb_volume.h"
@@ -84,7 +86,7 @@ extern "C" __global__ __launch_bounds__(NarrowShape::Threads) void kttNoAllocCom
     kc::volumeCompensated<NarrowShape>(src, numberOfAtoms, gridSpacing, gridSize, energyGrid, partials, tileCounters, splitFrom);
 }
 
-template <int PX, int ROWS, int CAP, int LANES = 64>
+template <int PX, int ROWS, int CAP, int LANES>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5))) void kttNoAllocPacked(const float4* atoms,
     int numberOfAtoms, int share, float gridSpacing, int lanesX, int rowGroups, int rowLength, int rowsTotal, float* energyGrid)
 {
@@ -124,33 +126,12 @@ int FailHip(char* message, const size_t length, const char* what, const hipError
 
 using PackedKernel = void (*)(const float4*, int, int, float, int, int, int, int, float*);
 
-// The precompiled kernel of a shape, or null. ChoosePackedPlan gives 2 x 8 points with up to 4 row groups
-// per wave, 1 x 8 and 1 x 4 with up to 8, the latter also on 32 lanes (a side of 6 or 7).
-PackedKernel PackedKernelOf(const ktt::PackedPlan& plan)
+template <size_t... V>
+PackedKernel PackedKernelAt(const int variant, std::index_sequence<V...>)
 {
-    struct Entry
-    {
-        int px;
-        int rows;
-        int cap;
-        int lanes;
-        PackedKernel kernel;
-    };
-    static const Entry entries[] = {{2, 8, 1, 64, kttNoAllocPacked<2, 8, 1>}, {2, 8, 2, 64, kttNoAllocPacked<2, 8, 2>},
-        {2, 8, 3, 64, kttNoAllocPacked<2, 8, 3>}, {2, 8, 4, 64, kttNoAllocPacked<2, 8, 4>},
-        {1, 8, 1, 64, kttNoAllocPacked<1, 8, 1>}, {1, 8, 2, 64, kttNoAllocPacked<1, 8, 2>},
-        {1, 8, 3, 64, kttNoAllocPacked<1, 8, 3>}, {1, 8, 4, 64, kttNoAllocPacked<1, 8, 4>},
-        {1, 8, 8, 64, kttNoAllocPacked<1, 8, 8>}, {1, 4, 1, 64, kttNoAllocPacked<1, 4, 1>},
-        {1, 4, 2, 64, kttNoAllocPacked<1, 4, 2>}, {1, 4, 4, 64, kttNoAllocPacked<1, 4, 4>},
-        {1, 4, 8, 64, kttNoAllocPacked<1, 4, 8>}, {1, 4, 8, 32, kttNoAllocPacked<1, 4, 8, 32>}};
-    for (const Entry& entry : entries)
-    {
-        if (entry.px == plan.px && entry.rows == plan.rows && entry.cap == plan.cap && entry.lanes == plan.lanes)
-        {
-            return entry.kernel;
-        }
-    }
-    return nullptr;
+    static const PackedKernel kernels[] = {kttNoAllocPacked<ktt::kPackedVariants[V].px, ktt::kPackedVariants[V].rows,
+        ktt::kPackedVariants[V].cap, ktt::kPackedVariants[V].lanes>...};
+    return kernels[variant];
 }
 
 // Set-up of the current device, once: the device address of `scratch`, the CU count and
@@ -244,15 +225,17 @@ extern "C" __attribute__((visibility("default"))) int ktt_noalloc_coulomb3d_comp
     if (ktt::WaveEngineByDefault(gridSize))
     {
         const ktt::PackedPlan plan = ktt::ChoosePackedPlan(atomCount, gridSize, static_cast<long>(gridSize) * gridSize, true);
-        const PackedKernel kernel = PackedKernelOf(plan);
-        if (kernel != nullptr)
+        const int variant = ktt::PackedVariantOf(plan);
+        if (variant < 0)
         {
-            hipLaunchKernelGGL(kernel, dim3(plan.workgroups), dim3(64 * plan.waves), plan.ldsBytes, static_cast<hipStream_t>(stream),
-                reinterpret_cast<const float4*>(atoms), atomCount, plan.share, spacing, plan.lanesX, plan.rowGroups, gridSize,
-                gridSize * gridSize, energyGrid);
-            const hipError_t status = hipGetLastError();
-            return status == hipSuccess ? 0 : FailHip(message, messageLength, "launch of the compensated Coulomb kernel", status);
+            return Fail(message, messageLength, "no precompiled kernel for the wave engine's launch of this grid");
         }
+        const PackedKernel kernel = PackedKernelAt(variant, std::make_index_sequence<ktt::kPackedVariantCount>());
+        hipLaunchKernelGGL(kernel, dim3(plan.workgroups), dim3(64 * plan.waves), plan.ldsBytes, static_cast<hipStream_t>(stream),
+            reinterpret_cast<const float4*>(atoms), atomCount, plan.share, spacing, plan.lanesX, plan.rowGroups, gridSize,
+            gridSize * gridSize, energyGrid);
+        const hipError_t status = hipGetLastError();
+        return status == hipSuccess ? 0 : FailHip(message, messageLength, "launch of the compensated Coulomb kernel", status);
     }
 
     // The launch plan of ktt_coulomb3d (compensated, default configuration, TAIL_SPLIT=1).

@@ -275,4 +275,31 @@ inline PackedPlan ChoosePackedPlan(const int atomCount, const long rowLength, co
     return best;
 }
 
+// The compensated kernels that ChoosePackedPlan picks among for the volumes WaveEngineByDefault takes: all of them, each
+// for some volume. The no-allocation library holds these.
+struct PackedVariant
+{
+    int px;
+    int rows;
+    int cap;
+    int lanes;
+};
+constexpr PackedVariant kPackedVariants[] = {{2, 8, 1, 64}, {2, 8, 2, 64}, {2, 8, 3, 64}, {2, 8, 4, 64}, {1, 8, 1, 64}, {1, 8, 2, 64},
+    {1, 8, 3, 64}, {1, 4, 1, 64}, {1, 4, 2, 64}, {1, 4, 4, 64}, {1, 4, 8, 64}, {1, 4, 8, 32}};
+constexpr int kPackedVariantCount = static_cast<int>(sizeof(kPackedVariants) / sizeof(kPackedVariants[0]));
+
+// Index of a plan's kernel in kPackedVariants, or -1.
+inline int PackedVariantOf(const PackedPlan& plan)
+{
+    for (int v = 0; v < kPackedVariantCount; ++v)
+    {
+        const PackedVariant& variant = kPackedVariants[v];
+        if (variant.px == plan.px && variant.rows == plan.rows && variant.cap == plan.cap && variant.lanes == plan.lanes)
+        {
+            return v;
+        }
+    }
+    return -1;
+}
+
 } // namespace ktt

@@ -712,6 +712,37 @@ void TestPackedPlan()
     CHECK(refused(1, 4, 16, 46340));  // more threads than a launch holds
 }
 
+/** The no-allocation library's kernels: every default plan of a volume has one, and every one has a volume. */
+void TestPackedVariants()
+{
+    bool found = true;
+    std::set<int> used;
+    for (int g = 1; g <= 1024; ++g)
+    {
+        if (!ktt::WaveEngineByDefault(g))
+        {
+            continue;
+        }
+        for (long atoms = 0; atoms <= 0x7fffffffL; atoms += 1 + atoms / 3)
+        {
+            const int variant = ktt::PackedVariantOf(ktt::ChoosePackedPlan(static_cast<int>(atoms), g, static_cast<long>(g) * g, true));
+            found = found && variant >= 0;
+            used.insert(variant);
+        }
+    }
+    CHECK(found);
+    CHECK(used.size() == static_cast<size_t>(ktt::kPackedVariantCount));
+    // The volumes that the GPU test of the entry point runs, one for each kernel.
+    const std::pair<int, int> tested[] = {{1, 5}, {6, 30}, {9, 100}, {24, 700}, {43, 600}, {59, 600}, {63, 64}, {63, 600}, {64, 300},
+        {76, 300}, {100, 501}, {127, 5}};
+    std::set<int> covered;
+    for (const auto& [g, atoms] : tested)
+    {
+        covered.insert(ktt::PackedVariantOf(ktt::ChoosePackedPlan(atoms, g, static_cast<long>(g) * g, true)));
+    }
+    CHECK(covered.size() == static_cast<size_t>(ktt::kPackedVariantCount));
+}
+
 /** Which slices run the wave engine by default: the faster kernel of the measured ones, and a launch that exists
  *  for all it takes. */
 void TestSliceRule()
@@ -790,6 +821,7 @@ int main(int argc, char** argv)
     TestProfileSearcherAnalysis();
     TestBatchWorkList();
     TestPackedPlan();
+    TestPackedVariants();
     TestSliceRule();
     TestFewAtomsRule();
     TestPackedBatch();

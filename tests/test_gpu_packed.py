@@ -148,10 +148,11 @@ def test_slice_calls_take_wave_split(capi):
             capi.coulomb3d_slices(atoms_buffer, atoms.shape[0], spacing, 100, energy, config=config)
 
 
-@pytest.mark.parametrize("grid,count", [(1, 5), (6, 30), (9, 100), (24, 700), (45, 300), (63, 64), (70, 3000), (100, 501)])
+@pytest.mark.parametrize("grid,count", [(1, 5), (6, 30), (9, 100), (24, 700), (43, 600), (45, 300), (59, 600), (63, 64), (63, 600), (64, 300),
+                                        (70, 3000), (76, 300), (100, 501), (127, 5)])
 def test_no_alloc_entry_point_takes_the_same_shapes(capi, grid, count):
-    """ktt_coulomb3d_compensated_noalloc at sides that run the wave engine, one for each of its
-    precompiled kernels' row-group caps and blocks, against FP64 and ktt_coulomb3d."""
+    """ktt_coulomb3d_compensated_noalloc at sides that run the wave engine, at least one for each of its
+    precompiled kernels (ktt_core_tests checks that these sizes reach every one), against FP64 and ktt_coulomb3d."""
     spacing = 0.5
     atoms = workloads.uniform_atoms(90 + grid, count, box=max(grid, 4) * spacing)
     start = np.zeros(grid ** 3 + 64, dtype=np.float32)
