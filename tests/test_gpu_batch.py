@@ -1,4 +1,5 @@
-"""Batched form: many independent systems in one persistent, graph-captured launch."""
+"""Batched form: many independent systems in one launch, on the wave engine (the default) and on the persistent bucket
+kernel, which use_graph replays from a captured graph."""
 
 from __future__ import annotations
 
@@ -41,7 +42,7 @@ UNROLLED = ("BUCKET0_UNROLL=8,BUCKET1_UNROLL=8,BUCKET2_UNROLL=8,BUCKET1_TILE=32,
             "BUCKET2_TILE=128")
 
 
-@pytest.mark.parametrize("config", [None, UNROLLED])
+@pytest.mark.parametrize("config", [None, "GROUPS_PER_CU=4", UNROLLED])
 def test_batch_matches_oracle_and_graph_replays_match_eager(capi, config):
     systems = small_batch()
     print("batch config", config, flush=True)
@@ -117,15 +118,17 @@ def test_bucket_tuning_does_not_leave_a_batch_slower(capi):
     check_against_oracle(systems, batch.grids(), COMPENSATED_BAR)
 
 
-def test_full_batch_every_system_against_oracle(capi):
+@pytest.mark.parametrize("config", [None, "GROUPS_PER_CU=4"])
+def test_full_batch_every_system_against_oracle(capi, config):
     """The 1,024-system batch of the benchmark (atom counts log-uniform in [200, 20000], sides
-    32/48/64/96/128, so every bucket's tile shape runs) through the graph-launched persistent
-    kernel: every system at 64 sampled points against FP64, compensated bar; a graph replay
-    equals the first run bit for bit."""
+    32/48/64/96/128) on the wave engine and through the graph-launched persistent kernel, where every
+    bucket's default tile shape runs: every system at 64 sampled points against FP64, compensated bar;
+    a second run (with buckets a graph replay) equals the first bit for bit."""
     systems = workloads.batch()
     assert sorted({s.grid for s in systems}) == list(workloads.BATCH_SIDES)
-    batch = capi.Batch(systems)
+    batch = capi.Batch(systems, config=config)
     info = batch.info()
+    assert info["shapes"].startswith("BUCKET0_WGX" if config else "WAVE_SPLIT")
     print("full batch:", len(systems), "systems,", info["items"], "items,", info["shapes"], flush=True)
     assert info["interactions"] == sum(s.interactions for s in systems)
     batch.zero()

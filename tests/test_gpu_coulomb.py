@@ -343,12 +343,14 @@ def test_iterative_wall_time_excludes_set_up():
     assert 0.0 < kernel_ms <= wall_ms < 0.5 * compile_ms
 
 
-def test_full_size_iterative_forms(capi):
-    """CoulombSum3dIterative at 256^3 x 65,536 atoms, both launchers with their default slice
-    shape (256 atom blocks per slice adding with FP32 atomics): the reference's host dz^2
-    scheme (Examples/CoulombSum3dIterative/CoulombSum3dIterative.cpp:146-184) and the fused
-    device dz^2, each against FP64 at 4,096 sampled points and against the volume kernel
-    (SideBySide 0.01) everywhere."""
+@pytest.mark.parametrize("config", [None, "ATOM_BLOCKS=256"])
+def test_full_size_iterative_forms(capi, config):
+    """CoulombSum3dIterative at 256^3 x 65,536 atoms, both launchers: by default one volume launch from host
+    and from device atoms; with the slice kernel's default shape named (256 atom blocks per slice adding
+    with FP32 atomics) the reference's host dz^2 scheme
+    (Examples/CoulombSum3dIterative/CoulombSum3dIterative.cpp:146-184) and the fused device dz^2, a launch
+    per slice. Each against FP64 at 4,096 sampled points and against the volume kernel (SideBySide 0.01)
+    everywhere."""
     work = workloads.volume3d()
     points = workloads.sample_points(36, 4096, work.grid)
     values, norms = oracle.points_f64(work.atoms, work.spacing, points)
@@ -358,10 +360,10 @@ def test_full_size_iterative_forms(capi):
     capi.coulomb3d(atoms_buffer, work.atoms.shape[0], work.spacing, work.grid, energy)
     volume = energy.download((work.grid, work.grid, work.grid))
     energy.zero()
-    kernel_ms, wall_ms = capi.coulomb3d_iterative(work.atoms, work.spacing, work.grid, energy)
+    kernel_ms, wall_ms = capi.coulomb3d_iterative(work.atoms, work.spacing, work.grid, energy, config=config)
     host = energy.download((work.grid, work.grid, work.grid))
     energy.zero()
-    slices_ms = capi.coulomb3d_slices(atoms_buffer, work.atoms.shape[0], work.spacing, work.grid, energy)
+    slices_ms = capi.coulomb3d_slices(atoms_buffer, work.atoms.shape[0], work.spacing, work.grid, energy, config=config)
     fused = energy.download((work.grid, work.grid, work.grid))
     for name, result, ms in (("host dz2", host, kernel_ms), ("device dz2", fused, slices_ms)):
         worst, rms = oracle.normalised_error(result[points[:, 2], points[:, 1], points[:, 0]], values, norms)
@@ -477,25 +479,28 @@ def test_translation_and_axis_swap(capi):
         assert difference.max() <= 2 * bar, (form, difference.max())
 
 
-def test_compensated_tail_split(capi):
-    """The compensated default splits only the tiles of the last, partial round of workgroups over
-    atom blocks; those meet in FP64 partials, the others store directly. The grid side is the first
-    of 160..256 whose tile count leaves this device (at the kernel's occupancy) a partial round to
-    split, as the launch plan reports. Points of the split tiles and sampled points everywhere meet
+@pytest.mark.parametrize("config", ["TAIL_SPLIT=1", "TAIL_SPLIT=1,WORK_GROUP_SIZE_X=64"])
+def test_compensated_tail_split(capi, config):
+    """The compensated workgroup shapes, 128 and 64 threads wide, split only the tiles of the last, partial
+    round of workgroups over atom blocks; those meet in FP64 partials, the others store directly. The grid
+    side is the first of 256, 160..240 whose tile count leaves this device (at the kernel's occupancy) a
+    partial round to split, as the launch plan reports (256 is the only one that splits without a
+    configuration; the others run the wave engine then). Points of the split tiles and sampled points everywhere meet
     the bar, a second launch is bitwise equal (the merge order is fixed), and TAIL_SPLIT=0 (no
     split) agrees on the split tiles to twice the bar."""
     atoms = workloads.uniform_atoms(30, 600, box=80.0)
     spacing = 0.5
-    for grid in (160, 176, 192, 208, 224, 240, 256):
-        plan = capi.coulomb3d_launch_plan(atoms.shape[0], grid, form=capi.COMPENSATED)
+    whole_config = config.replace("TAIL_SPLIT=1", "TAIL_SPLIT=0")
+    for grid in (256, 160, 176, 192, 208, 224, 240):
+        plan = capi.coulomb3d_launch_plan(atoms.shape[0], grid, form=capi.COMPENSATED, config=config)
         if plan["grid"][2] > 1:
             break
     print(f"tail split plan at {grid}^3:", plan, flush=True)
     # The split path must run: more than one atom block, and some (not all) tiles split.
     assert plan["grid"][2] > 1 and 0 < plan["split_from"] < plan["groups"] and plan["scratch_bytes"] > 0
-    assert capi.coulomb3d_launch_plan(atoms.shape[0], grid, form=capi.COMPENSATED, config="TAIL_SPLIT=0")["grid"][2] == 1
-    first = run_volume(capi, atoms, spacing, grid, form=capi.COMPENSATED)
-    second = run_volume(capi, atoms, spacing, grid, form=capi.COMPENSATED)
+    assert capi.coulomb3d_launch_plan(atoms.shape[0], grid, form=capi.COMPENSATED, config=whole_config)["grid"][2] == 1
+    first = run_volume(capi, atoms, spacing, grid, form=capi.COMPENSATED, config=config)
+    second = run_volume(capi, atoms, spacing, grid, form=capi.COMPENSATED, config=config)
     np.testing.assert_array_equal(first, second)
     # Rows (z * G + y) of the split tiles: from the first split tile's row group to the end.
     rows_per_group = (grid * grid) // plan["grid"][1]
@@ -506,7 +511,7 @@ def test_compensated_tail_split(capi):
     for points in (split_points, workloads.sample_points(31, 4096, grid)):
         worst, _ = normalised(first, atoms, spacing, points)
         assert worst <= COMPENSATED_BAR, worst
-    whole = run_volume(capi, atoms, spacing, grid, form=capi.COMPENSATED, config="TAIL_SPLIT=0")
+    whole = run_volume(capi, atoms, spacing, grid, form=capi.COMPENSATED, config=whole_config)
     _, norms = oracle.points_f64(atoms, spacing, split_points)
     index = (split_points[:, 2], split_points[:, 1], split_points[:, 0])
     assert (np.abs(first[index].astype(np.float64) - whole[index]) / norms).max() <= 2 * COMPENSATED_BAR

@@ -1,7 +1,7 @@
 """The wave engine (ktt_amd/kernels/coulomb_wave.h) against the FP64 oracle at every point, where it
 can go wrong: sides whose rows wrap within a wave, end inside one or are shorter than a lane's run; atom
-counts around a wave's 64-atom tile, the 256 atoms of a two-sum and the unrolled step; one wave, waves
-without atoms, and splits that meet in several passes over the LDS.
+counts around a wave's 64-atom tile and the unrolled step; one wave, waves without atoms, and splits that
+meet in several passes over the LDS. Wide blocks and large sides at sampled points.
 
 Bars as for every form: 1e-5 plain, 1e-6 compensated, normalised by sum_i |q_i| / r_i."""
 
@@ -40,6 +40,18 @@ def check(capi, grid, count, form, config, spacing=0.5):
     assert worst <= BARS[form], (worst, rms)
 
 
+def check_sampled(capi, grid, count, form, config, spacing=0.5):
+    """As check, at sampled points, the grid's last row among them."""
+    atoms = workloads.uniform_atoms(1000 * grid + count, count, box=grid * spacing)
+    points = np.concatenate([workloads.sample_points(grid, 2048, grid),
+                             np.array([[x, grid - 1, grid - 1] for x in range(grid)], dtype=np.int32)])
+    print(f"grid {grid} atoms {count} form {form} config {config}", flush=True)
+    values, norms = oracle.points_f64(atoms, spacing, points)
+    out = run_guarded(capi, atoms, spacing, grid, form, config).reshape(grid, grid, grid)
+    worst, rms = oracle.normalised_error(out[points[:, 2], points[:, 1], points[:, 0]], values, norms)
+    assert worst <= BARS[form], (worst, rms)
+
+
 @pytest.mark.parametrize("form", [0, 1])
 @pytest.mark.parametrize("grid", [1, 2, 3, 6, 7, 16, 31, 33, 48, 65, 70])
 def test_default_shapes(capi, grid, form):
@@ -53,6 +65,22 @@ def test_default_shapes(capi, grid, form):
 @pytest.mark.parametrize("waves,count", [(1, 7), (1, 65), (3, 257), (4, 521), (16, 9), (16, 1025)])
 def test_splits(capi, shape, waves, count, form):
     check(capi, 45, count, form, f"WAVE_SPLIT={waves},{shape}")
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("shape", ["POINTS_X=3,ROWS_PER_THREAD=8", "POINTS_X=4,ROWS_PER_THREAD=4", "POINTS_X=4,ROWS_PER_THREAD=8"])
+@pytest.mark.parametrize("waves,count", [(1, 65), (16, 1025)])
+def test_wide_blocks(capi, shape, waves, count, form):
+    """The widest blocks a configuration may name (4 x 8 points spill registers), on rows they do not divide."""
+    check_sampled(capi, 91, count, form, f"WAVE_SPLIT={waves},{shape}")
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("grid,count", [(257, 100), (300, 1000), (513, 300)])
+def test_default_above_256(capi, grid, count, form):
+    """The default of sides above 256, up to 1,024, that 256 does not divide."""
+    assert capi.coulomb3d_launch_plan(count, grid, form=form)["block"][1] == 1
+    check_sampled(capi, grid, count, form, None)
 
 
 @pytest.mark.parametrize("form", [0, 1])

@@ -1,9 +1,9 @@
 """The entry point that allocates nothing (ktt_coulomb3d_compensated_noalloc) against the entry
 point it is a variant of (ktt_coulomb3d, compensated form, default configuration).
 
-Two calls in a row share the library's static scratch: the first at 256^3 x 65,536 atoms (the
-tail split's partials fill about 40 MiB of it), the second smaller (160^3 x 600 atoms, a
-different split). Each must agree with ktt_coulomb3d to the compensated form's bar (normalised
+Three calls in a row: 256^3 x 65,536 atoms and 256^3 x 600 share the library's static scratch (the tail
+split's partials fill about 40 MiB of it, then less by a different split), and 160^3 x 600 runs the
+wave engine, which takes none. Each must agree with ktt_coulomb3d to the compensated form's bar (normalised
 by sum_i |q_i| / r_i at every sampled point) and meet that bar against the FP64 oracle.
 """
 
@@ -37,8 +37,9 @@ def run_both(capi, atoms, spacing, grid):
     return existing, no_alloc
 
 
-def test_no_alloc_matches_existing_entry_point_on_two_calls(capi):
-    cases = [(workloads.volume3d().atoms, 0.5, 256, 41), (workloads.uniform_atoms(30, 600, box=80.0), 0.5, 160, 42)]
+def test_no_alloc_matches_existing_entry_point_on_calls_in_a_row(capi):
+    cases = [(workloads.volume3d().atoms, 0.5, 256, 41), (workloads.uniform_atoms(31, 600, box=128.0), 0.5, 256, 43),
+             (workloads.uniform_atoms(30, 600, box=80.0), 0.5, 160, 42)]
     for atoms, spacing, grid, seed in cases:
         print(f"no-alloc call: grid {grid}, {atoms.shape[0]} atoms", flush=True)
         existing, no_alloc = run_both(capi, atoms, spacing, grid)
