@@ -24,7 +24,8 @@ while the GPU idles between legs, has climbed back):
   precision    256^3 grid, 1,048,576 atoms in 64 Gaussian clusters of +-1 pairs 1 A apart,
                plain and compensated;
   batched      1,024 independent systems (atoms log-uniform in [200, 20000], sides in
-               {32, 48, 64, 96, 128}) in one launch, against one plain launch per system;
+               {32, 48, 64, 96, 128}) in one launch, against one plain launch per system at fixed
+               workgroup shapes and against ktt_coulomb3d per system by default;
   dynamic      192^3 grid, 131,072 atoms, 500 steps of N(0, 0.05^2 I) jitter on the device, ktt
                TuneIteration (MCMC, 48 steps) then the best configuration; the best configuration
                of a whole-space search (profiles/coulomb3d_dynamic_192x131072_exhaustive.json) is
@@ -53,6 +54,7 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--dynamic [--exhaust
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
 import sys
@@ -251,7 +253,8 @@ def headline_leg(capi, workloads, args, samples: dict):
 def iterative_leg(capi, workloads, work, samples: dict) -> dict:
     """CoulombSum3dIterative on the headline inputs: the reference's host dz^2 path (one upload
     and launch per slice) and the fused device path (one launch per slice). Naming the slice
-    kernel's shape keeps the launch per slice; without one both run as a single volume launch."""
+    kernel's shape keeps the launch per slice; without one both run as a single volume launch, the
+    default of both calls, timed last."""
     per_slice = "ATOM_BLOCKS=256"
     n_atoms = work.atoms.shape[0]
     atoms = capi.DeviceBuffer.from_array(work.atoms)
@@ -267,12 +270,20 @@ def iterative_leg(capi, workloads, work, samples: dict) -> dict:
     slices_ms, _ = timed_loop(capi, lambda: capi.coulomb3d_slices(atoms, n_atoms, work.spacing, work.grid, energy, config=per_slice,
                                                                   timed=False), 1, 0)
     samples["iterative_device"] = [sample(work.atoms, work.spacing, points, energy.download((work.grid,) * 3))]
+    capi.coulomb3d_slices(atoms, n_atoms, work.spacing, work.grid, energy, timed=False)  # compiles the wave engine's kernel
+    energy.zero()
+    default_ms, _ = timed_loop(capi, lambda: capi.coulomb3d_slices(atoms, n_atoms, work.spacing, work.grid, energy, timed=False), 1, 0)
+    energy.zero()
+    _, default_wall_ms = capi.coulomb3d_iterative(work.atoms, work.spacing, work.grid, energy)
+    samples["iterative_default"] = [sample(work.atoms, work.spacing, points, energy.download((work.grid,) * 3))]
     atoms.close()
     energy.close()
     return {
         "host_dz2": {"kernel_ms": kernel_ms, "wall_ms": wall_ms, "value": work.interactions / (kernel_ms * 1e-3),
                      "value_wall": work.interactions / (wall_ms * 1e-3)},
         "device_slices": {"ms": slices_ms, "value": work.interactions / (slices_ms * 1e-3)},
+        "default": {"device_atoms_ms": default_ms, "host_atoms_wall_ms": default_wall_ms,
+                    "value": work.interactions / (default_ms * 1e-3)},
     }
 
 
@@ -368,6 +379,13 @@ def precision_leg(capi, workloads, samples: dict) -> dict:
     return timing
 
 
+class DeviceView:
+    """Part of a device buffer, for the calls that take a capi.DeviceBuffer."""
+
+    def __init__(self, pointer: int):
+        self.ptr = ctypes.c_void_p(pointer)
+
+
 def batched_leg(capi, workloads, samples: dict, config=None, repeats: int = 3) -> dict:
     systems = workloads.batch()
     batch = capi.Batch(systems, config=config)
@@ -390,6 +408,18 @@ def batched_leg(capi, workloads, samples: dict, config=None, repeats: int = 3) -
     for _ in range(max(1, repeats - 1)):
         batch.zero()
         per_system.append(batch.run_per_system(form=capi.PLAIN))
+    # The baseline above names its workgroup shapes; this is ktt_coulomb3d per system as a caller gets it, by default.
+    packed_atoms = capi.DeviceBuffer.from_array(np.concatenate([s.atoms for s in systems], axis=0))
+    first_atoms = np.concatenate([[0], np.cumsum([s.atoms.shape[0] for s in systems])])
+    views = [(DeviceView(packed_atoms.ptr.value + 16 * int(first_atoms[k])), DeviceView(info["grids"].value + 4 * int(info["offsets"][k])))
+             for k in range(len(systems))]
+
+    def default_calls():
+        for system, (atoms, grid) in zip(systems, views):
+            capi.coulomb3d(atoms, system.atoms.shape[0], system.spacing, system.grid, grid, form=capi.COMPENSATED, timed=False)
+
+    per_system_default_ms, _ = timed_loop(capi, default_calls, 2, 1)
+    packed_atoms.close()
     batch.close()
     graph_ms = float(np.median(graph))
     per_system_ms = float(np.median(per_system))
@@ -404,6 +434,8 @@ def batched_leg(capi, workloads, samples: dict, config=None, repeats: int = 3) -
         "per_system_plain_ms": per_system_ms,
         "per_system_plain_value": info["interactions"] / (per_system_ms * 1e-3),
         "speedup_vs_per_system_plain": per_system_ms / graph_ms,
+        "per_system_default_compensated_ms": per_system_default_ms,
+        "speedup_vs_per_system_default": per_system_default_ms / graph_ms,
         "form": "compensated, one launch",
     }
 
