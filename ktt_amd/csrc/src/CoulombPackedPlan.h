@@ -174,13 +174,14 @@ inline int SliceAtomBlocks(const int atomCount)
  *  then costs more per atom and per workgroup than the workgroup shapes of CoulombSum2d.hip. Over 19 grids of
  *  64^2 to 2,048^2 points and 1 to 30,000 atoms (MI355X, workgroup shapes / wave engine) it is the faster one
  *   - while all its workgroups start at once (4 per CU) and the busiest CU's work through at most 64 atoms per
- *     wave one after the other: 256^2 x 64 5.97 / 4.14 us, 64 x 1,024 x 512 7.20 / 6.17, 192^2 x 768 6.80 / 6.13,
- *     512^2 x 128 7.04 / 6.77; beyond, 256^2 x 1,024 9.64 / 9.70, 192^2 x 1,024 7.49 / 7.96, 512^2 x 256 9.53 / 9.80;
+ *     wave one after the other, 96 if no CU has fewer: 256^2 x 64 5.97 / 4.14 us, 64 x 1,024 x 512 7.20 / 6.17,
+ *     192^2 x 768 6.80 / 6.13, 512^2 x 128 7.04 / 6.77, 256^2 x 768 8.37 / 8.04; beyond, 256^2 x 1,024 9.64 / 9.70,
+ *     192^2 x 1,024 7.49 / 7.96, 512^2 x 256 9.53 / 9.80;
  *   - on up to 4,096 points, where the atom blocks of the workgroup shapes end at 128: 64^2 x 16,384 12.77 / 9.91,
  *     to 75 million interactions (64^2 x 30,000 16.81 / 16.83);
- *   - with at most 16 atoms, whose brackets and adds are little beside the grid: 768^2 x 16 8.07 / 6.50, 1,024^2 x
- *     16 10.06 / 9.72; beyond, 1,024^2 x 32 10.03 / 10.83 and x 64 10.0 / 14.3, 2,048^2 x 16 31.0 / 32.4, 4,096^2 x 1
- *     105 / 116. */
+ *   - with at most 16 atoms, 8 above 2^20 points, whose brackets and adds are little beside the grid: 768^2 x 16
+ *     8.07 / 6.50, 1,024^2 x 16 10.06 / 9.72, 2,048^2 x 8 31.0 / 29.3; beyond, 1,024^2 x 32 10.03 / 10.83 and x 64
+ *     10.0 / 14.3, 2,048^2 x 16 31.0 / 32.4, 4,096^2 x 1 105 / 116. */
 inline bool SliceOnWaveEngine(const long gridX, const long gridY, const int atomCount)
 {
     const long points = gridX * gridY;
@@ -195,7 +196,8 @@ inline bool SliceOnWaveEngine(const long gridX, const long gridY, const int atom
         return false;
     }
     const long workgroups = static_cast<long>(plan.workgroups) * blocks;
-    if (workgroups <= 4 * 256 && (workgroups + 255) / 256 * plan.share <= 64)
+    const long perUnit = (workgroups + 255) / 256;
+    if (perUnit <= 4 && (perUnit * plan.share <= 64 || (perUnit * plan.share <= 96 && workgroups * 50 >= perUnit * 256 * 49)))
     {
         return true;
     }
@@ -203,7 +205,7 @@ inline bool SliceOnWaveEngine(const long gridX, const long gridY, const int atom
     {
         return true;
     }
-    return atomCount <= 16 && points <= 1L << 22 && points * atomCount <= 1L << 24;
+    return atomCount <= 16 && points <= 1L << (atomCount > 8 ? 20 : 22);
 }
 
 /** Whether a volume of few atoms runs faster on the workgroup shapes although its side takes the wave engine by default.
