@@ -213,14 +213,15 @@ int ktt_coulomb_batch_info(void* batch, float** grids, size_t* grid_points, long
 /* Clears all grids of the batch (zero-fill kernel). */
 int ktt_coulomb_batch_zero(void* batch, void* stream);
 
-/* Adds V of every system to its grid in one launch, compensated: the wave engine's workgroups in the
- * order of the systems' atoms, or, with buckets set, persistent workgroups that take (system, tile) items
+/* Adds V of every system to its grid in one launch, compensated: the wave engine's workgroups, systems
+ * with the most atoms first, or, with buckets set, persistent workgroups that take (system, tile) items
  * from a device-side queue; use_graph != 0 then replays a HIP graph (queue reset + persistent kernel)
  * captured on the first call. The wave engine is one launch with or without it. */
 int ktt_coulomb_batch_run(void* batch, int use_graph, void* stream, float* kernel_ms);
 
 /* Baseline: one ktt_coulomb3d launch per system (form KTT_COULOMB_PLAIN or _COMPENSATED), all
- * on one stream; kernel_ms is the event time around the whole sequence. */
+ * on one stream, at workgroup shapes fixed by the grid side (not the shapes ktt_coulomb3d picks by
+ * default, which are faster on small grids); kernel_ms is the event time around the whole sequence. */
 int ktt_coulomb_batch_run_per_system(void* batch, int form, void* stream, float* kernel_ms);
 
 /* Tunes the tile shape of every bucket with ktt::Tuner on ComputeApi::HIP (a composite kernel
@@ -248,7 +249,9 @@ int ktt_coulomb_batch_tune(void* batch, int searcher, int max_configurations_per
  * extension) receives the KTT JSON results; best_config (optional) the best configuration
  * as NAME=VALUE,...; best_ms (optional) its kernel time; valid_count (optional) the number
  * of configurations with status Ok; tested_count (optional) the number tested.
- * energy_grid (optional, host, G^3 floats) receives the output of the best configuration. */
+ * energy_grid (optional, host, G^3 floats) receives the output of the best configuration. The space
+ * is that of the workgroup kernel (CoulombSum3d.hip) and does not hold the wave engine: at the sides
+ * where ktt_coulomb3d runs that by default, a call without a configuration can be the faster one. */
 int ktt_coulomb3d_tune(const float* host_atoms, int n_atoms, float spacing, int grid_size, int searcher,
                        int max_configurations, double tolerance, const char* results_file,
                        char* best_config, size_t best_config_length, double* best_ms,
@@ -281,7 +284,8 @@ int ktt_script_generate(const char* expression, long long count, double* values)
  * (seed, s, atom index) on the device, clears the G^3 map and recomputes it. The first
  * min(tuning_budget, space) steps each run the searcher's next configuration
  * (tuning_budget <= 0: the whole space); every later step runs Tuner::GetBestConfiguration
- * (Source/Tuner.h:776-782). Outputs, each optional: step_kernel_ms[steps] (Coulomb kernel
+ * (Source/Tuner.h:776-782). The space is that of the workgroup kernel, as for ktt_coulomb3d_tune.
+ * Outputs, each optional: step_kernel_ms[steps] (Coulomb kernel
  * time, -1 for a configuration that failed), step_wall_ms[steps] (host time of the step,
  * compilation included), step_tuned[steps] (1 for a tuning step), best_config
  * (NAME=VALUE,...), tested_count, space_size, final_atoms (4 * n_atoms floats) and

@@ -863,14 +863,18 @@ static void CheckForm(const int gridSize, const int form)
 // Whether a ktt_coulomb3d call runs the wave engine (CoulombPacked.hip), and with what plan: when its
 // configuration says so (WAVE_SPLIT), or by default on grids that the workgroup shapes of
 // CoulombSum3d.hip do not fill. Those span 128 points of x (256 at multiples of 256) and need some
-// 160^3 points to fill the chip, so on 110 grids of 24^3 to 640^3 points the wave engine was faster at
-// all sides but the multiples of 256 (250^3 x 4,000: 5.36 against 5.86 ms plain, 5.56 against 6.42
-// compensated; 150^3 x 20,011: 5.9 against 11.2, 6.2 against 12.7; 33^3 x 500: 0.007 against 0.108,
-// 0.008 against 0.061). There the workgroup shapes fill every lane and share one set of row brackets
-// among 4 to 8 waves: 256^3 and 512^3 with 64 to 8,192 atoms ran between 3% faster and 5% slower than the wave
-// engine (256^3 x 8,192: 11.66 against 11.74 ms plain, 11.77 against 12.01 compensated; x 500
-// compensated 0.803 against 0.765, where the last round of workgroups is nearly empty), with no line between
-// the two. Above 1,024 the last span's idle lanes are under an eighth.
+// 160^3 points to fill the chip. On 32 sides of 24 to 1,023 with 100 to 4,000 atoms (MI355X, workgroup
+// shapes / wave engine) the wave engine is 1.02 to 7.6 times as fast in the compensated form, and 1.06 to 24
+// times in the plain form where rows leave a twentieth of their spans idle or more (150^3 x 4,000 1.85, 448^3 1.14,
+// 832^3 x 500 1.06). On sides that nearly fill their spans (384, 511, 640, 767, 896, 1,023) the plain form runs between
+// 4% slower and 21% faster: slower where the atoms also fill the 128-atom tiles (256 atoms 0.96 to 0.97, 1,000 atoms
+// 1.00), faster where they do not (100 atoms 1.20). The wave engine is the default there too: its 64-atom partial
+// sums are two to three times as exact as the plain workgroup shapes' running sums. At multiples
+// of 256 the workgroup shapes fill every lane and share one set of row brackets among 4 to 8 waves: 256^3 and
+// 512^3 with 64 to 8,192 atoms ran between 3% faster and 5% slower than the wave engine (256^3 x 8,192: 11.66
+// against 11.74 ms plain, 11.77 against 12.01 compensated; x 500 compensated 0.803 against 0.765, where the
+// last round of workgroups is nearly empty), with no line between the two. Above 1,024 the last span's idle lanes
+// are under an eighth. Few atoms: FewAtomsOnWorkgroupShapes.
 static bool PackedPlanFor(const int atomCount, const int gridSize, const int form, const char* config, PackedPlan& plan)
 {
     const CoulombConfig given = CoulombConfig::Parse(config, CoulombConfig());

@@ -108,10 +108,10 @@ struct PackedShape
     double atom;      // us a SIMD takes per wave and atom with enough waves to hide latency
     double compensated; // what the compensated form's offsets and sums multiply it by
     double alone;     // share of that rate that one wave per SIMD reaches
-    int wavesPerSimd; // at the kernel's registers, plain and compensated
+    int wavesPerSimd; // at the kernel's registers (78, 50, 46 and 96, 67, 51 VGPRs), plain and compensated
     int wavesPerSimdCompensated;
 };
-constexpr PackedShape kPackedShapes[] = {{2, 8, 0.071, 1.035, 0.49, 6, 5}, {1, 8, 0.0376, 1.0, 0.36, 7, 7},
+constexpr PackedShape kPackedShapes[] = {{2, 8, 0.071, 1.035, 0.49, 6, 5}, {1, 8, 0.0376, 1.0, 0.36, 8, 7},
     {1, 4, 0.0192, 1.124, 0.41, 8, 8}};
 
 // Workgroups a CU holds at once, by registers and LDS.
@@ -123,8 +123,10 @@ inline int PackedGroupsPerUnit(const PackedPlan& plan, const PackedShape& shape,
 
 // Estimated time of a plan in us beyond the launch itself. The constants are a fit to 27 grids of 24^3 to
 // 320^3 points with 64 to 20,000 atoms, both forms, each timed on MI355X at every shape and 4, 8 and 16
-// waves (1 too for 64 atoms): the shape it picks is within 1.0% of the fastest on average (at worst
-// 7%), while any one shape for all is several times slower somewhere.
+// waves (1 too for 64 atoms): the shape it picks is within 1.0% of the fastest of these on average (at worst
+// 7%), while any one shape for all is several times slower somewhere. It knows nothing of the store of rows
+// that a lane's run does not divide: with up to 64 atoms on full spans it is 5 to 9% off (127^3 x 64 plain 21.4
+// us, 19.7 in 2 x 8 blocks).
 inline double EstimatePacked(const PackedPlan& plan, const PackedShape& shape, const bool compensated)
 {
     constexpr double kComputeUnits = 256.0;
@@ -152,9 +154,9 @@ inline double EstimatePacked(const PackedPlan& plan, const PackedShape& shape, c
     return load * wave / rate;
 }
 
-/** Whether a volume of side^3 points runs the wave engine without a configuration: not at multiples of
- *  256, whose lanes and chip the workgroup shapes fill, and not above 1,024, where their idle lanes are
- *  under an eighth (the figures stand at PackedPlanFor in CoulombApi.cpp). */
+/** Whether a volume of side^3 points runs the wave engine without a configuration (but for a few atoms on some
+ *  sides, below): not at multiples of 256, whose lanes and chip the workgroup shapes fill, and not above 1,024, where
+ *  their idle lanes are under an eighth (the figures stand at PackedPlanFor in CoulombApi.cpp). */
 inline bool WaveEngineByDefault(const int side)
 {
     return side % 256 != 0 && side <= 1024;

@@ -757,8 +757,8 @@ void TestSliceRule()
     const Measured measured[] = {{64, 16, 1, true}, {64, 64, 8000, true}, {64, 64, 16384, true}, {64, 1024, 512, true},
         {128, 128, 2048, true}, {192, 192, 768, true}, {256, 256, 64, true}, {256, 256, 500, true}, {320, 320, 256, true},
         {384, 384, 128, true}, {512, 256, 256, true}, {512, 512, 64, true}, {512, 512, 128, true}, {64, 8192, 16, true},
-        {768, 768, 16, true}, {1024, 1024, 8, true}, {2048, 2048, 8, true}, {64, 1024, 768, true}, {512, 256, 257, true}, {256, 256, 4000, false}, {192, 192, 1024, false},
-        {320, 320, 512, false}, {384, 384, 256, false}, {512, 512, 256, false}, {64, 8192, 64, false}, {8192, 64, 64, false},
+        {768, 768, 16, true}, {1024, 1024, 8, true}, {2048, 2048, 8, true}, {64, 1024, 768, true}, {512, 256, 257, true},
+        {256, 256, 4000, false}, {192, 192, 1024, false}, {320, 320, 512, false}, {384, 384, 256, false}, {512, 512, 256, false}, {64, 8192, 64, false}, {8192, 64, 64, false},
         {768, 768, 64, false}, {1024, 512, 64, false}, {1024, 1024, 32, false}, {1024, 1024, 64, false}, {2048, 1024, 32, false},
         {2048, 2048, 16, false}, {4096, 4096, 1, false}, {64, 1024, 3000, false}, {256, 256, 1 << 30, false}};
     for (const Measured& m : measured)

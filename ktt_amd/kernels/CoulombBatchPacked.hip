@@ -3,7 +3,9 @@
 // keeps the tile-shape buckets that a configuration or the autotuner sets.
 //
 // Work items (system, block of lanes) are listed by the host, systems with the most atoms first, and
-// workgroups start in that order, so that the long items do not end last. The waves of a workgroup
+// workgroups start in that order, so that the items of large systems do not end last. (By atoms alone: an item of a
+// small grid holds fewer points per lane. Ordering by atoms times points per lane takes the same time on twelve
+// mixed batches, 27.96 against 27.97 ms on the one with 7s below.) The waves of a workgroup
 // split the system's atoms. Lanes are packed within each system, so a side of any size wastes at most its
 // last wave, and one block serves all sides of a class: 2 x 8 points per lane from 64 points up, 1 x 8 from
 // 32, 1 x 4 below. From side 21 up that keeps a wave to 3 or 4 row groups and its LDS to 8 KiB; smaller sides
