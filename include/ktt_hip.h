@@ -103,7 +103,7 @@ int ktt_hip_event_elapsed_ms(void* start, void* end, float* milliseconds);
  * and the point index is 64-bit (the reference kernel's int index overflows above G = 1,290).
  * Without a configuration, sides up to 1,024 that are not a multiple of 256 run the wave engine
  * (CoulombPacked.hip), whose lanes pack any side and whose waves split the atoms of small grids (up to
- * 64 atoms on sides that suit the workgroup shapes excepted);
+ * 64 atoms in the plain form, on sides that suit the workgroup shapes, excepted);
  * WAVE_SPLIT (1 to 16 waves sharing the atoms of 64 lanes), with POINTS_X (1 to 4, default 2) and
  * ROWS_PER_THREAD (4 or 8, the default), selects it explicitly. The kernel that a call without a
  * configuration compiles at its first use depends on the side, the form and the number of atoms. */
@@ -155,8 +155,9 @@ int ktt_coulomb2d_reference(const float* atoms, int n_atoms, float spacing, int 
  * configuration, as the reference launcher does it: for every slice the host computes dz^2 of all atoms,
  * uploads the atom records with .z replaced, and launches the slice kernel (CoulombSum3dIterative.cl:35)
  * with zIndex = z. Without one, or with WAVE_SPLIT as in ktt_coulomb3d, the atoms are uploaded once and one
- * launch covers all slices, forming dz^2 on the device. wall_ms receives the host time of the whole call's work, kernel_ms the (sum of the)
- * kernels' event times; the call returns when they have ended. */
+ * launch covers all slices, forming dz^2 on the device. wall_ms receives the host time of the whole call's
+ * work (without compiling and allocating), kernel_ms the (sum of the) kernels' event times; the call returns
+ * when they have ended. */
 int ktt_coulomb3d_iterative(const float* host_atoms, int n_atoms, float spacing, int grid_size, float* energy_grid,
                             const char* config, void* stream, float* kernel_ms, float* wall_ms);
 

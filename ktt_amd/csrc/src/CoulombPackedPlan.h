@@ -173,59 +173,44 @@ inline int SliceAtomBlocks(const int atomCount)
 
 /** Whether a slice runs the wave engine without a configuration. A small slice is over in a few microseconds,
  *  most of them one workgroup's start: tile, barriers, brackets, adds, which the wave engine does faster. It
- *  then costs more per atom and per workgroup than the workgroup shapes of CoulombSum2d.hip. Over 19 grids of
- *  64^2 to 2,048^2 points and 1 to 30,000 atoms (MI355X, workgroup shapes / wave engine) it is the faster one
- *   - while all its workgroups start at once (4 per CU) and the busiest CU's work through at most 64 atoms per
- *     wave one after the other, 96 if no CU has fewer: 256^2 x 64 5.97 / 4.14 us, 64 x 1,024 x 512 7.20 / 6.17,
- *     192^2 x 768 6.80 / 6.13, 512^2 x 128 7.04 / 6.77, 256^2 x 768 8.37 / 8.04; beyond, 256^2 x 1,024 9.64 / 9.70,
- *     192^2 x 1,024 7.49 / 7.96, 512^2 x 256 9.53 / 9.80;
- *   - on up to 4,096 points, where the atom blocks of the workgroup shapes end at 128: 64^2 x 16,384 12.77 / 9.91,
- *     to 75 million interactions (64^2 x 30,000 16.81 / 16.83);
- *   - with at most 16 atoms, 8 above 2^20 points, whose brackets and adds are little beside the grid: 768^2 x 16
- *     8.07 / 6.50, 1,024^2 x 16 10.06 / 9.72, 2,048^2 x 8 31.0 / 29.3; beyond, 1,024^2 x 32 10.03 / 10.83 and x 64
- *     10.0 / 14.3, 2,048^2 x 16 31.0 / 32.4, 4,096^2 x 1 105 / 116. */
+ *  then costs more per workgroup and per atom than the workgroup shapes of CoulombSum2d.hip. MI355X, workgroup
+ *  shapes / wave engine, over 19 grids of 64^2 to 2,048^2 points and 1 to 30,000 atoms:
+ *   - up to 512^2 points the wave engine up to 75 million interactions: 256^2 x 64 5.97 / 4.14 us, 64 x 1,024 x 512
+ *     7.20 / 6.17, 64^2 x 16,384 12.77 / 9.91, 512^2 x 128 7.04 / 6.77. Near the limit it is between 6% slower and
+ *     level (384^2 x 256 7.49 / 8.01, 192^2 x 1,024 7.49 / 7.96, 256^2 x 1,024 9.64 / 9.70), for an error that is a
+ *     quarter smaller (1.1e-7 against 1.5e-7 of the slice at 384^2 x 256: 32 atoms a partial sum, not 64);
+ *   - above, only with at most 16 atoms, 8 above 2^20 points: 768^2 x 16 8.07 / 6.50, 1,024^2 x 16 10.06 / 9.72,
+ *     2,048^2 x 8 31.0 / 29.3. The wave engine's workgroups no longer start at once there and each costs its start: 64
+ *     x 8,192 x 64 6.6 / 8.2, 1,024^2 x 32 10.0 / 10.8 and x 64 10.0 / 14.3, 2,048^2 x 16 31.0 / 32.4, 4,096^2 x 1
+ *     105 / 116. */
 inline bool SliceOnWaveEngine(const long gridX, const long gridY, const int atomCount)
 {
     const long points = gridX * gridY;
-    const int blocks = SliceAtomBlocks(atomCount);
-    if (blocks > 65535)
+    if (points <= 1L << 18)
     {
-        return false;
+        return points * atomCount <= 75000000L;
     }
-    const PackedPlan plan = PlanShape(kSlicePx, kSliceRows, kSliceWaves, blocks, atomCount, gridX, gridY, false);
-    if (plan.workgroups == 0)
-    {
-        return false;
-    }
-    const long workgroups = static_cast<long>(plan.workgroups) * blocks;
-    const long perUnit = (workgroups + 255) / 256;
-    if (perUnit <= 4 && (perUnit * plan.share <= 64 || (perUnit * plan.share <= 96 && workgroups * 50 >= perUnit * 256 * 49)))
-    {
-        return true;
-    }
-    if (points <= 4096 && points * atomCount <= 75000000L)
-    {
-        return true;
-    }
-    return atomCount <= 16 && points <= 1L << (atomCount > 8 ? 20 : 22);
+    return points <= 1L << 22 && atomCount <= (points <= 1L << 20 ? 16 : 8);
 }
 
-/** Whether a volume of few atoms runs faster on the workgroup shapes although its side takes the wave engine by default.
- *  Up to 64 atoms are one tile of either kernel, and clearing, reading and writing the grid count as much as the sum.
- *  The workgroup shapes win where they compute no padding to speak of: atoms that fill their 16-, 32- or 64-atom
- *  tile to the wave engine's step of 8, and rows that nearly fill the 128-point spans. (MI355X, workgroup shapes / wave
- *  engine, plain and compensated:)
+/** Whether a volume of few atoms in the plain form runs faster on the workgroup shapes although its side takes the wave
+ *  engine by default. Up to 64 atoms are one tile of either kernel, and clearing, reading and writing the grid count
+ *  as much as the sum. The workgroup shapes win where they compute no padding to speak of: atoms that fill their 16-,
+ *  32- or 64-atom tile to the wave engine's step of 8, and rows that nearly fill the 128-point spans (MI355X, workgroup
+ *  shapes / wave engine):
  *   - below a side of 128, where 2 x 8 blocks are two waves per SIMD and the chooser's narrower ones pay for their
- *     start: 117^3 x 16 0.86 and 0.91, 125^3 x 32 0.83 and 0.83, 127^3 x 64 0.90 and 0.87, but 113^3 x 64 1.07 and 1.07;
- *   - in the plain form at odd sides, whose rows the wave engine stores point by point: 9 to 16 atoms at 251^3 0.90,
- *     at 511^3 0.85, at 1,023^3 0.87 (32 atoms 0.96, 0.94, 0.98; even sides and the compensated form 1.0 to 1.5), and
- *     1 to 8 atoms above a side of 448: 511^3 0.93, 1,023^3 0.94 (383^3 1.10).
- *  The sums are as exact either way: one tile, added in order. */
+ *     start: 117^3 x 16 0.86, 125^3 x 32 0.83, 127^3 x 64 0.90, but 113^3 x 64 1.07;
+ *   - at odd sides, whose rows the wave engine stores point by point: 9 to 16 atoms at 251^3 0.90, at 511^3 0.85, at
+ *     1,023^3 0.87 (32 atoms 0.96, 0.94, 0.98; even sides 1.0 to 1.5), and 1 to 8 atoms above a side of 448: 511^3
+ *     0.93, 1,023^3 0.94 (383^3 1.10).
+ *  The plain sums are as exact either way (one tile, added in order: 1.1e-7 of the map at 117^3 x 16). The compensated
+ *  form stays on the wave engine, 0.77 to 1.1 below a side of 128 and level above: its x offsets carry one rounding, the
+ *  workgroup shapes' two (127^3 x 64 at a spacing of 0.49: 1.8e-7 against 4.3e-7, 117^3 x 16 1.2e-7 against 1.1e-6). */
 inline bool FewAtomsOnWorkgroupShapes(const int side, const int atomCount, const bool compensated)
 {
     const int spans = (side + 127) / 128;
     const int tile = atomCount <= 16 ? 16 : (atomCount <= 32 ? 32 : 64);
-    if (atomCount < 1 || atomCount > tile)
+    if (compensated || atomCount < 1 || atomCount > tile)
     {
         return false;
     }
@@ -234,7 +219,7 @@ inline bool FewAtomsOnWorkgroupShapes(const int side, const int atomCount, const
     {
         return full && side * 10 >= 128 * 9;
     }
-    return !compensated && side % 2 != 0 && side * 20 >= spans * 128 * 17 && atomCount <= 16 && (full || side > 448);
+    return side % 2 != 0 && side * 20 >= spans * 128 * 17 && atomCount <= 16 && (full || side > 448);
 }
 
 /** The shape with the smallest estimated time. */

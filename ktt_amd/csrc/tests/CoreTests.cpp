@@ -743,8 +743,8 @@ void TestPackedVariants()
     CHECK(covered.size() == static_cast<size_t>(ktt::kPackedVariantCount));
 }
 
-/** Which slices run the wave engine by default: the faster kernel of the measured ones, and a launch that exists
- *  for all it takes. */
+/** Which slices run the wave engine by default: the measured ones that it makes faster, or more exact at under 7%
+ *  of their time; and a launch exists for all it takes. */
 void TestSliceRule()
 {
     struct Measured
@@ -755,12 +755,12 @@ void TestSliceRule()
         bool wave;
     };
     const Measured measured[] = {{64, 16, 1, true}, {64, 64, 8000, true}, {64, 64, 16384, true}, {64, 1024, 512, true},
-        {128, 128, 2048, true}, {192, 192, 768, true}, {256, 256, 64, true}, {256, 256, 500, true}, {320, 320, 256, true},
-        {384, 384, 128, true}, {512, 256, 256, true}, {512, 512, 64, true}, {512, 512, 128, true}, {64, 8192, 16, true},
-        {768, 768, 16, true}, {1024, 1024, 8, true}, {2048, 2048, 8, true}, {64, 1024, 768, true}, {512, 256, 257, true},
-        {256, 256, 4000, false}, {192, 192, 1024, false}, {320, 320, 512, false}, {384, 384, 256, false}, {512, 512, 256, false}, {64, 8192, 64, false}, {8192, 64, 64, false},
-        {768, 768, 64, false}, {1024, 512, 64, false}, {1024, 1024, 32, false}, {1024, 1024, 64, false}, {2048, 1024, 32, false},
-        {2048, 2048, 16, false}, {4096, 4096, 1, false}, {64, 1024, 3000, false}, {256, 256, 1 << 30, false}};
+        {128, 128, 2048, true}, {192, 192, 1024, true}, {256, 256, 64, true}, {256, 256, 1000, true}, {320, 320, 256, true},
+        {384, 384, 256, true}, {512, 256, 256, true}, {512, 512, 64, true}, {512, 512, 128, true}, {64, 8192, 16, true},
+        {768, 768, 16, true}, {1024, 1024, 8, true}, {2048, 2048, 8, true}, {256, 256, 4000, false}, {320, 320, 1000, false},
+        {64, 8192, 64, false}, {8192, 64, 64, false}, {768, 768, 64, false}, {1024, 512, 64, false}, {1024, 1024, 32, false},
+        {1024, 1024, 64, false}, {2048, 1024, 32, false}, {2048, 2048, 16, false}, {4096, 4096, 1, false}, {64, 1024, 3000, false},
+        {256, 256, 1 << 30, false}};
     for (const Measured& m : measured)
     {
         CHECK(ktt::SliceOnWaveEngine(m.x, m.y, m.atoms) == m.wave);
@@ -781,17 +781,15 @@ void TestSliceRule()
     CHECK(exists);
 }
 
-/** Which volumes of few atoms leave the wave engine: those measured slower on it. */
+/** Which volumes of few atoms leave the wave engine: those measured slower and no more exact on it. */
 void TestFewAtomsRule()
 {
     const auto plain = [](const int side, const int atoms) { return ktt::FewAtomsOnWorkgroupShapes(side, atoms, false); };
     const auto compensated = [](const int side, const int atoms) { return ktt::FewAtomsOnWorkgroupShapes(side, atoms, true); };
-    for (const auto& [side, atoms] : {std::pair<int, int>{117, 16}, {120, 12}, {121, 32}, {125, 16}, {125, 32}, {127, 64}})
+    for (const auto& [side, atoms] : {std::pair<int, int>{117, 16}, {120, 12}, {121, 32}, {125, 16}, {125, 32}, {127, 64}, {251, 16},
+        {383, 12}, {511, 16}, {511, 1}, {1023, 16}, {1023, 8}})
     {
-        CHECK(plain(side, atoms) && compensated(side, atoms));
-    }
-    for (const auto& [side, atoms] : {std::pair<int, int>{251, 16}, {383, 12}, {511, 16}, {511, 1}, {1023, 16}, {1023, 8}})
-    {
+        // The compensated form is more exact on the wave engine.
         CHECK(plain(side, atoms) && !compensated(side, atoms));
     }
     for (const auto& [side, atoms] : {std::pair<int, int>{24, 16}, {101, 16}, {113, 64}, {125, 48}, {127, 65}, {127, 200}, {127, 0},

@@ -230,11 +230,10 @@ def test_batches(capi, sides, config):
 @pytest.mark.parametrize("form", [0, 1])
 @pytest.mark.parametrize("grid,count", [(117, 16), (127, 64), (251, 12), (255, 16)])
 def test_few_atoms(capi, grid, count, form):
-    """Sides of the wave engine whose few atoms run on the workgroup shapes (plain; compensated below 128):
-    the plan says so, and the map meets the bar at sampled points."""
+    """Sides of the wave engine whose few atoms run on the workgroup shapes in the plain form: the plan says so,
+    and the map meets the bar at sampled points."""
     plan = capi.coulomb3d_launch_plan(count, grid, form=form)
-    workgroup_shapes = grid < 128 or form == 0
-    assert (plan["block"][1] > 1) == workgroup_shapes, plan
+    assert (plan["block"][1] > 1) == (form == 0), plan
     assert plan["scratch_bytes"] == 0
     atoms = workloads.uniform_atoms(500 + grid, count, box=grid * 0.5)
     print(f"few atoms: grid {grid} atoms {count} form {form}", flush=True)
