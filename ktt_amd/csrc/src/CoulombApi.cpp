@@ -864,7 +864,7 @@ static void CheckForm(const int gridSize, const int form)
 // configuration says so (WAVE_SPLIT), or by default on grids that the workgroup shapes of
 // CoulombSum3d.hip do not fill. Those span 128 points of x (256 at multiples of 256) and need some
 // 160^3 points to fill the chip. On 32 sides of 24 to 1,023 with 100 to 4,000 atoms (MI355X, workgroup
-// shapes / wave engine) the wave engine is 1.02 to 7.6 times as fast in the compensated form, and 1.06 to 24
+// shapes / wave engine) the wave engine is level to 7.7 times as fast in the compensated form, and 1.06 to 24
 // times in the plain form where rows leave a twentieth of their spans idle or more (150^3 x 4,000 1.85, 448^3 1.14,
 // 832^3 x 500 1.06). On sides that nearly fill their spans (384, 511, 640, 767, 896, 1,023) the plain form runs between
 // 4% slower and 21% faster: slower where the atoms also fill the 128-atom tiles (256 atoms 0.96 to 0.97, 1,000 atoms
